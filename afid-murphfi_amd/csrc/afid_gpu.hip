@@ -22,6 +22,7 @@
 #include "afid_params.hpp"
 #include "afid_stencils.hpp"
 #include "afid_kernels.hpp"
+#include "afid_column.hpp"
 #include "afid_poisson.hpp"
 #include "afid_phase.hpp"
 #include "afid_means.hpp"
@@ -470,12 +471,12 @@ static int setup(afid_ctx *c) {
     if (c->pf && c->sal) return set_err(c, AFID_E_ARG, "phase field together with salinity is not supported");
     if (c->pf && !(g.pf_a != 0.0 && g.pf_s != 0.0)) return set_err(c, AFID_E_ARG, "phase field needs pf_A and pf_S nonzero");
     c->nxm = g.nxm; c->nx = g.nxm + 1; c->ny = g.nym; c->nz = g.nzm;
-    c->ldx = (c->nx + 7) / 8 * 8;
+        c->ldx = (c->nx + 15) / 16 * 16;
     c->ldt = (c->nx + 3 + 7) / 8 * 8;
     c->nymh = c->ny / 2 + 1;
     if (c->sal || c->pf) {
         c->nxmr = g.nxmr; c->nxr = g.nxmr + 1; c->nyr = g.nymr; c->nzr = g.nzmr;
-        c->ldxr = (c->nxr + 7) / 8 * 8;
+        c->ldxr = (c->nxr + 15) / 16 * 16;
         if (c->nxmr < 2 || c->nyr < 2 || c->nzr < 2) return set_err(c, AFID_E_ARG, "refined grid too small");
     }
     // ReadInputFile.F90:101-122
@@ -580,7 +581,11 @@ static int setup(afid_ctx *c) {
     H["ak1"] = ak1; H["ak2"] = ak2; H["amphk"] = amphk; H["acphk"] = acphk; H["apphk"] = apphk;
 
     int rc;
-    auto up = [&](const std::vector<double> &v, const double **d) { return rc ? rc : (rc = upload_vec(c, v, d)); };
+    // (zero-padded to whole rows: the column kernel reads them in 16-byte pairs)
+    auto up = [&](std::vector<double> v, const double **d) {
+        v.resize(std::max(v.size(), size_t(std::max(c->ldx, c->ldxr))), 0.0);
+        return rc ? rc : (rc = upload_vec(c, v, d));
+    };
     rc = 0;
     std::vector<double> udx3m_v = farr_range(udx3m, 1, nxm), udx3c_v = farr_range(udx3c, 1, nx), g3rc_v = farr_range(g3rc, 1, nx);
     std::vector<double> xm_v = farr_range(xm, 1, nxm);
@@ -712,7 +717,7 @@ static int setup(afid_ctx *c) {
     int chmax = 1;
     for (int k = 0; k < MAT_NKIND; ++k) { c->chunk[k] = std::max(1, (c->nrows[k] + 63) / 64); chmax = std::max(chmax, c->chunk[k]); }
     if (chmax > 16) return set_err(c, AFID_E_ARG, "wall-normal size above 1024 points is not supported");
-    c->npadmax = 64 * chmax;
+    c->npadmax = (64 * chmax + 127) / 128 * 128;      // whole groups of the column kernel (128 rows)
     if ((rc = dalloc(c, reinterpret_cast<void **>(&c->tri), sizeof(double) * size_t(3 * MAT_NKIND * kTriArrays) * c->npadmax))) return rc;
 
     // mixed form: the reference buoyancy of the FP32 vx explicit term (zero until the walls are set)
@@ -1565,7 +1570,7 @@ static void launch_column_base(afid_ctx *c, const KP &p) {
     else if (c->pf) launch_column_base_form<CH, double, true>(c, p);
     else launch_column_base_form<CH, double, false>(c, p);
 }
-// single-pass kernel; CH here is the chunk of the nxm-row systems
+// single-pass kernel through LDS; CH here is the chunk of the nxm-row systems
 template <int CH, typename HT, bool PF>
 static void launch_column_base1_form(afid_ctx *c, const KP &p) {
     BaseOut o{c->alt[0], c->alt[1], c->alt[2], c->alt[3]};
@@ -1601,11 +1606,53 @@ static int column_humid(afid_ctx *c) {
     }
     return check_launch(c, "k_column_humid");
 }
+// the register kernel (k_column_base_reg): LPC lanes per column, MG groups,
+// NW wavefronts per workgroup, KEEP old fields in LDS, row tables in LDS (LT)
+template <int LPC, int MG, int NW, int KEEP, bool LT>
+static void launch_column_reg(afid_ctx *c, const KP &p, long long nblk, long long nwg) {
+    const BaseOut o{c->alt[0], c->alt[1], c->alt[2], c->alt[3]};
+    const dim3 gr(unsigned(std::min((nblk + 7) / 8 * 8, nwg)));
+    if (c->mixed)
+        hipLaunchKernelGGL((k_column_base_reg<LPC, MG, NW, KEEP, LT, float>), gr, dim3(64 * NW), 0, c->stream, p, base_const<float>(p),
+                           factors(c, MAT_X), factors(c, MAT_YZ), factors(c, MAT_T), o);
+    else
+        hipLaunchKernelGGL((k_column_base_reg<LPC, MG, NW, KEEP, LT, double>), gr, dim3(64 * NW), 0, c->stream, p, base_const<double>(p),
+                           factors(c, MAT_X), factors(c, MAT_YZ), factors(c, MAT_T), o);
+}
+// The grid is what the card holds at once (two wavefronts per SIMD by
+// registers: 512 workgroups of 4, 256 of 8), each walking its blocks, so the
+// row tables are staged once.  LPC: two columns per wavefront where one
+// column would leave a quarter of its lanes idle or more (nxm <= 64, and 129
+// to 192).  8-wavefront workgroups, where the tables (61 / 82 KB of LDS) and
+// the old fields fill the LDS with one workgroup.  Without the staged tables
+// only where every workgroup has a single block of at most 64 rows: 18.6
+// against 21.1 us for a 64 x 64^2 launch; elsewhere they win (128 x 256^2:
+// 313 against 387 us, 48 x 96^2: 32.6 against 34.0).
+static int column_base_reg(afid_ctx *c, const KP &p) {
+    const long long b32 = col_blocks<32, 4>(c->ny, c->nz), b64 = col_blocks<64, 4>(c->ny, c->nz), b8 = col_blocks<64, 8>(c->ny, c->nz);
+    switch (c->chunk[MAT_YZ]) {
+    case 1:
+        if (b32 <= 512) launch_column_reg<32, 1, 4, 4, false>(c, p, b32, 512);
+        else launch_column_reg<32, 1, 4, 4, true>(c, p, b32, 512);
+        break;
+    case 2: launch_column_reg<64, 1, 4, 4, true>(c, p, b64, 512); break;
+    case 3: launch_column_reg<32, 3, 4, 4, true>(c, p, b32, 512); break;
+    case 4: launch_column_reg<64, 2, 4, 4, true>(c, p, b64, 512); break;
+    case 5: case 6: launch_column_reg<64, 3, 8, 4, true>(c, p, b8, 256); break;
+    default: launch_column_reg<64, 4, 8, 2, true>(c, p, b8, 256); break;
+    }
+    return check_launch(c, "k_column_base_reg");
+}
 static int column_base(afid_ctx *c) {
     KP p = make_kp(c);
-    // single pass up to 512 wall-normal cells (its registers hold two
-    // right-hand sides of CH rows), four passes above
-    if (!c->col_four_pass && c->chunk[MAT_YZ] <= 8) {
+    int rc;
+    // up to 512 wall-normal cells: the register kernel for fields it can
+    // address with 32-bit byte offsets, else (and with the phase field, whose
+    // solves are masked) the single pass through LDS; four passes above
+    const bool reg = !c->pf && (unsigned long long)p.plane * c->nz * sizeof(double) < (1ull << 32);
+    if (!c->col_four_pass && c->chunk[MAT_YZ] <= 8 && reg) {
+        if ((rc = column_base_reg(c, p))) return rc;
+    } else if (!c->col_four_pass && c->chunk[MAT_YZ] <= 8) {
         switch (c->chunk[MAT_YZ]) {
 #define AFID_CB1_CASE(CH) case CH: launch_column_base1<CH>(c, p); break;
             AFID_CB1_CASE(1) AFID_CB1_CASE(2) AFID_CB1_CASE(3) AFID_CB1_CASE(4) AFID_CB1_CASE(5) AFID_CB1_CASE(6)
@@ -1622,8 +1669,7 @@ static int column_base(afid_ctx *c) {
         default: return set_err(c, AFID_E_ARG, "nx too large");
         }
     }
-    int rc = check_launch(c, "k_column_base");
-    if (rc) return rc;
+    if ((rc = check_launch(c, "k_column_base"))) return rc;
     std::swap(c->f[AFID_VX], c->alt[0]);
     std::swap(c->f[AFID_VY], c->alt[1]);
     std::swap(c->f[AFID_VZ], c->alt[2]);
