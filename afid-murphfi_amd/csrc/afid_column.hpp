@@ -468,4 +468,213 @@ __global__ void __launch_bounds__(64 * NW) k_column_base_reg(KP p, BaseConst<HT>
 #undef AFID_FENCE
 }
 
+// ---------------------------------------------------------------------------
+// refined columns (salinity, phase field) the same way
+// ---------------------------------------------------------------------------
+// Inclusive scans of one affine map over the LPC lanes of a column.
+template <int CTRL, int ROWS, bool LAST>
+__device__ __forceinline__ void scan1_step(double &A, double &B) {
+    B = A * dpp_into<CTRL, ROWS>(0.0, B) + B;
+    if (!LAST) A = A * dpp_into<CTRL, ROWS>(1.0, A);
+}
+template <int LPC>
+__device__ __forceinline__ void scan1_up(double &A, double &B) {
+    scan1_step<0x111, 0xf, false>(A, B);
+    scan1_step<0x112, 0xf, false>(A, B);
+    scan1_step<0x114, 0xf, false>(A, B);
+    scan1_step<0x118, 0xf, false>(A, B);
+    scan1_step<0x142, 0xa, LPC == 32>(A, B);
+    if (LPC == 64) scan1_step<0x143, 0xc, true>(A, B);
+}
+template <int LPC>
+__device__ __forceinline__ void scan1_down(double &A, double &B, unsigned lane) {
+    scan1_step<0x101, 0xf, false>(A, B);
+    scan1_step<0x102, 0xf, false>(A, B);
+    scan1_step<0x104, 0xf, false>(A, B);
+    scan1_step<0x108, 0xf, false>(A, B);
+    const int s16 = int((lane & 32) | 16);
+    const bool t16 = !(lane & 16);
+    const double b = __shfl(B, s16, 64);
+    B = A * (t16 ? b : 0.0) + B;
+    if (LPC == 64) {
+        const double a = __shfl(A, s16, 64);
+        A = A * (t16 ? a : 1.0);
+        const double b2 = __shfl(B, 32, 64);
+        B = A * (lane < 32 ? b2 : 0.0) + B;
+    }
+}
+// 16-byte vector access at a byte offset from a uniform base, plain or without keeping the line
+template <typename T> struct Native16;
+template <> struct Native16<float> { typedef float V __attribute__((ext_vector_type(4))); };
+template <> struct Native16<double> { typedef double V __attribute__((ext_vector_type(2))); };
+template <typename T>
+__device__ __forceinline__ typename Native16<T>::V ld16(const T *base, unsigned byte) {
+    return *reinterpret_cast<const typename Native16<T>::V *>(reinterpret_cast<const char *>(base) + byte);
+}
+template <typename T>
+__device__ __forceinline__ typename Native16<T>::V ld16_nt(const T *base, unsigned byte) {
+    return __builtin_nontemporal_load(reinterpret_cast<const typename Native16<T>::V *>(reinterpret_cast<const char *>(base) + byte));
+}
+template <typename T>
+__device__ __forceinline__ void st16_nt(T *base, unsigned byte, typename Native16<T>::V v) {
+    __builtin_nontemporal_store(v, reinterpret_cast<typename Native16<T>::V *>(reinterpret_cast<char *>(base) + byte));
+}
+
+// PHI false: ExplicitSalinity + ImplicitSalinity + SolveImpEqnUpdate_Sal
+// (salinity.F90:268-454), the new S to out.  PHI true: ExplicitPhase +
+// ImplicitPhase + SolveImpEqnUpdate_Phi (phasefield.F90:345-466), the new phi
+// to out and the increment to rhsr (read by AddLatentHeat).  RT: storage and
+// explicit-term arithmetic of the refined arrays; the implicit RHS, the solve
+// and the update run in FP64.  Layout as k_column_base_reg with NR = 16 /
+// sizeof(RT) rows per lane: lane l holds the rows NR (LPC g + l) ...
+//
+// What bounds it: bytes.  A form that went through LDS to the solver's layout
+// waited at two barriers per column and kept 43 to 51 KB of LDS per 4
+// wavefronts; the figures of both are at the launch.
+template <int LPC, int MG, int NW, typename RT, bool PHI>
+__global__ void __launch_bounds__(64 * NW) k_column_refined(KP p, TriFactors f, RT *out) {
+    using V = typename Native16<RT>::V;
+    constexpr int NR = 16 / sizeof(RT);
+    constexpr unsigned ROWS = unsigned(NR) * LPC * MG;
+    // row tables: metric (salinity), x operator, folded factors
+    enum { T_U3, T_AP, T_AC, T_AM, T_LN, T_SN, T_E, T_N };
+    __shared__ __align__(16) double tab[T_N][ROWS];
+    {
+        const double *src[T_N] = {PHI ? nullptr : p.udx3mr, PHI ? p.ap3spkr : p.ap3sskr, PHI ? p.ac3spkr : p.ac3sskr,
+                                  PHI ? p.am3spkr : p.am3sskr, f.ln, f.sn, f.e};
+#pragma unroll
+        for (int q = PHI ? 1 : 0; q < T_N; ++q)
+            for (unsigned r = threadIdx.x; r < ROWS; r += 64u * NW) tab[q][r] = r < unsigned(p.nxmr) ? src[q][r] : 0.0;
+    }
+    __syncthreads();
+    const unsigned lane = threadIdx.x & 63, l = lane % LPC;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr int CPB = col_per_block<LPC, NW>(), SB = COL_STRIP / CPB;
+    const unsigned n = p.nxmr, rmax = p.ldxr - NR;
+    const bool lo_lane = l == 0, hi_lane = l == LPC - 1;
+    const RT udy = RT(0.5) * RT(p.dyr), udz = RT(0.5) * RT(p.dzr);
+    const RT udyq = PHI ? RT(p.pf_d * p.dyqr) : RT(p.dyqr) / RT(p.pecs), udzq = PHI ? RT(p.pf_d * p.dzqr) : RT(p.dzqr) / RT(p.pecs);
+    const double adif = PHI ? p.al * p.pf_d : p.al / p.pecs;
+    const long long total = col_blocks<LPC, NW>(p.nyr, p.nzr), perx = (total + 7) / 8;
+    const long long b0 = (blockIdx.x % 8) * perx, b1 = min(b0 + perx, total);
+#pragma unroll 1
+    for (long long blk = b0 + blockIdx.x / 8; blk < b1; blk += gridDim.x / 8) {
+        const long long per = (long long)SB * p.nzr;
+        const int strip = int(blk / per), rem = int(blk - strip * per);
+        const int i = rem / SB, jw = strip * COL_STRIP + (rem % SB) * CPB + wave * (64 / LPC);
+        if (jw >= p.nyr) continue;
+        const bool live = LPC == 64 || jw + int(lane / LPC) < p.nyr;
+        const int j = live ? jw + int(lane / LPC) : jw;
+        const long long pc = (long long)i * p.planer, pm = (long long)wrapm(i, p.nzr) * p.planer, pp = (long long)wrapp(i, p.nzr) * p.planer;
+        const unsigned row = unsigned(p.ldxr) * unsigned(sizeof(RT));
+        const unsigned o_c = unsigned(j) * row, o_jm = unsigned(wrapm(j, p.nyr)) * row, o_jp = unsigned(wrapp(j, p.nyr)) * row;
+        const RT *S = (PHI ? sel<RT>(p.phi, p.phif) : sel<RT>(p.sal, p.salf));
+        const RT *Sc = S + pc, *Sm = S + pm, *Sp = S + pp;
+        const RT *TR = PHI ? sel<RT>(p.tempr, p.temprf) + pc : nullptr;
+        const RT *X = PHI ? nullptr : sel<RT>(p.vxr, p.vxrf) + pc, *Y = PHI ? nullptr : sel<RT>(p.vyr, p.vyrf) + pc;
+        const RT *Z = PHI ? nullptr : sel<RT>(p.vzr, p.vzrf) + pc, *Zp = PHI ? nullptr : sel<RT>(p.vzr, p.vzrf) + pp;
+        RT *RU = (PHI ? sel<RT>(p.ruphi, p.ruphif) : sel<RT>(p.rusal, p.rusalf)) + pc;
+        RT *O = out + pc, *D = PHI ? sel<RT>(p.rhsr, p.rhsrf) + pc : nullptr;
+        const double sbp = PHI ? 0.0 : p.salbp[(long long)i * p.nyr + j], stp_ = PHI ? 0.0 : p.saltp[(long long)i * p.nyr + j];
+        // (opaque: the row tables are read where they are used)
+        unsigned lr = unsigned(NR) * l;
+        asm volatile("" : "+v"(lr));
+
+        double y[MG][NR];
+        V own[MG];
+        double cy = 0.0;
+#pragma unroll
+        for (int g = 0; g < MG; ++g) {
+            const unsigned r0 = unsigned(NR) * unsigned(g) * LPC + lr, rb = min(r0, rmax) * unsigned(sizeof(RT)), c = o_c + rb;
+            const V s = ld16(Sc, c), sjm = ld16(Sc, o_jm + rb), sjp = ld16(Sc, o_jp + rb), sim = ld16(Sm, c), sip = ld16(Sp, c);
+            const V ru = ld16_nt(RU, c);
+            V vx{}, vy{}, vyp{}, vz{}, vzp{}, tr{};
+            if (PHI) tr = ld16(TR, c);
+            else { vx = ld16_nt(X, c); vy = ld16(Y, c); vyp = ld16(Y, o_jp + rb); vz = ld16(Z, c); vzp = ld16(Zp, c); }
+            // the rows just outside the group, by its end lanes
+            RT es = RT(0), ex = RT(0);
+            if ((lo_lane && g > 0) || hi_lane) {
+                const unsigned er = hi_lane ? min(r0 + NR, rmax + NR - 1u) : r0 - 1u, eb = o_c + er * unsigned(sizeof(RT));
+                es = ld1(Sc, eb);
+                if (!PHI && hi_lane) ex = ld1(X, eb);
+            }
+            own[g] = s;
+            const RT sb = pick(lo_lane, es, lane_prev(RT(s[NR - 1]))), sa = pick(hi_lane, es, lane_next(RT(s[0])));
+            const RT xa = PHI ? RT(0) : pick(hi_lane, ex, lane_next(RT(vx[0])));
+            V h;
+            double A = 1.0, B = 0.0;
+#pragma unroll
+            for (int q = 0; q < NR; ++q) {
+                const unsigned k = r0 + q;
+                const bool in = k < n, kl = k == 0, kh = k == n - 1;
+                const RT sc = s[q], sk = q ? s[q ? q - 1 : 0] : sb, sn = q == NR - 1 ? sa : s[q == NR - 1 ? q : q + 1];
+                RT hq;
+                if (PHI) {
+                    const RT nl = RT(p.pf_b) * sc * (RT(1.0) - sc) * (RT(1.0) - RT(2.0) * sc + RT(p.pf_a) * (tr[q] - RT(p.pf_tm)));
+                    hq = (sjp[q] - RT(2.0) * sc + sjm[q]) * udyq + (sip[q] - RT(2.0) * sc + sim[q]) * udzq - nl;
+                } else {
+                    const RT vc = vx[q], vp = q == NR - 1 ? xa : vx[q == NR - 1 ? q : q + 1];
+                    const RT up = kh ? RT(2.0) * RT(stp_) : sn + sc, dn = kl ? RT(2.0) * RT(sbp) : sc + sk;
+                    const RT hsx = (vp * up - vc * dn) * RT(tab[T_U3][r0 + q]) * RT(0.5);
+                    const RT hsy = (vyp[q] * (sjp[q] + sc) - vy[q] * (sc + sjm[q])) * udy;
+                    const RT hsz = (vzp[q] * (sip[q] + sc) - vz[q] * (sc + sim[q])) * udz;
+                    hq = -(hsx + hsy + hsz) + (sjp[q] - RT(2.0) * sc + sjm[q]) * udyq + (sip[q] - RT(2.0) * sc + sim[q]) * udzq;
+                }
+                const double ap = tab[T_AP][r0 + q], ac = tab[T_AC][r0 + q], am = tab[T_AM][r0 + q];
+                const double wall = PHI ? 0.0 : 1.0;
+                const double dxx = (kh ? -wall * (am + ac) * stp_ * p.sfixn : double(sn) * ap) + double(sc) * ac
+                                 + (kl ? -wall * (ap + ac) * sbp * p.sfixs : double(sk) * am);
+                const double d = in ? (p.ga * double(hq) + p.ro * double(ru[q]) + adif * dxx) * p.dt : 0.0;
+                h[q] = in ? hq : ru[q];                 // rows past the last keep their history
+                // forward sweep y_r = sn_r d_r - ln_r y_{r-1}, first with y_{r0-1} = 0
+                const double ln = tab[T_LN][r0 + q];
+                y[g][q] = d * tab[T_SN][r0 + q];
+                B = y[g][q] - ln * B;
+                A = -ln * A;
+            }
+            if (live && r0 < n) st16_nt(RU, c, h);
+            if (g > 0) B = A * (lo_lane ? cy : 0.0) + B;
+            scan1_up<LPC>(A, B);
+            double yr = pick(lo_lane, cy, lane_prev(B));
+#pragma unroll
+            for (int q = 0; q < NR; ++q) { yr = y[g][q] - tab[T_LN][r0 + q] * yr; y[g][q] = yr; }
+            if (g + 1 < MG) cy = column_last<LPC>(yr, lane);
+        }
+        // backward sweep x_r = y_r - e_r x_{r+1} and the update, top group first
+        cy = 0.0;
+#pragma unroll
+        for (int g = MG - 1; g >= 0; --g) {
+            const unsigned r0 = unsigned(NR) * unsigned(g) * LPC + lr, c = o_c + min(r0, rmax) * unsigned(sizeof(RT));
+            double A = 1.0, B = 0.0, e[NR];
+#pragma unroll
+            for (int q = NR - 1; q >= 0; --q) { e[q] = tab[T_E][r0 + q]; B = y[g][q] - e[q] * B; A = -e[q] * A; }
+            if (g + 1 < MG) B = A * (hi_lane ? cy : 0.0) + B;
+            scan1_down<LPC>(A, B, lane);
+            double x = pick(hi_lane, cy, lane_next(B));
+            V o, dv;
+#pragma unroll
+            for (int q = NR - 1; q >= 0; --q) {
+                x = y[g][q] - e[q] * x;
+                o[q] = r0 + q < n ? RT(double(own[g][q]) + x) : own[g][q];
+                dv[q] = RT(x);
+            }
+            if (g > 0) cy = column_first<LPC>(x, lane);
+            if (live && r0 < n) {
+                st16_nt(O, c, o);
+                if (PHI) {
+                    if (r0 + NR <= n) st16_nt(D, c, dv);
+                    else
+#pragma unroll
+                        for (int q = 0; q < NR; ++q)
+                            if (r0 + q < n) *reinterpret_cast<RT *>(reinterpret_cast<char *>(D) + c + q * sizeof(RT)) = dv[q];
+                }
+            }
+        }
+        if (live && lo_lane && n % NR == 0) {           // the unused index nxr is carried over
+            const unsigned b = o_c + n * unsigned(sizeof(RT));
+            *reinterpret_cast<RT *>(reinterpret_cast<char *>(O) + b) = ld1(Sc, b);
+        }
+    }
+}
+
 }  // namespace afid

@@ -717,7 +717,7 @@ static int setup(afid_ctx *c) {
     int chmax = 1;
     for (int k = 0; k < MAT_NKIND; ++k) { c->chunk[k] = std::max(1, (c->nrows[k] + 63) / 64); chmax = std::max(chmax, c->chunk[k]); }
     if (chmax > 16) return set_err(c, AFID_E_ARG, "wall-normal size above 1024 points is not supported");
-    c->npadmax = (64 * chmax + 127) / 128 * 128;      // whole groups of the column kernel (128 rows)
+    c->npadmax = (64 * chmax + 127) / 128 * 128;      // whole groups of the column kernels (128 rows)
     if ((rc = dalloc(c, reinterpret_cast<void **>(&c->tri), sizeof(double) * size_t(3 * MAT_NKIND * kTriArrays) * c->npadmax))) return rc;
 
     // mixed form: the reference buoyancy of the FP32 vx explicit term (zero until the walls are set)
@@ -1676,50 +1676,52 @@ static int column_base(afid_ctx *c) {
     std::swap(c->f[AFID_TEMP], c->alt[3]);
     return AFID_OK;
 }
-template <int CH>
-static void launch_column_sal(afid_ctx *c, const KP &p, long long nblk) {
-    const dim3 gr(unsigned((nblk + 7) / 8 * 8));
-    if (c->mixed) hipLaunchKernelGGL((k_column_sal<CH, float>), gr, dim3(256), 0, c->stream, p, factors(c, MAT_S), c->sal_alt_f);
-    else hipLaunchKernelGGL((k_column_sal<CH, double>), gr, dim3(256), 0, c->stream, p, factors(c, MAT_S), c->sal_alt);
+// refined columns (k_column_refined), 8 wavefronts per workgroup, two
+// workgroups per CU walking their blocks (512).  MG = 1, 3: two columns per
+// wavefront where one would leave a quarter of its lanes idle or more.
+// 768 x 768^2 S, mixed: 3976 -> 2980 us a launch (3.2 -> 4.3 TB/s of 28 B per
+// cell); 768 x 384^2 S in FP64: 1655 -> 1370 us (3.8 -> 4.6 TB/s); 512 x 512^2
+// phi, mixed: 1110 -> 710 us (2.9 -> 4.5 TB/s of 24 B per cell); 256 x 512^2
+// phi in FP64: 808 -> 703 us.  Workgroups of 4 (3 or 4 per CU) 0 to 7%
+// slower; 4 wavefronts per SIMD by force spills (768 rows FP64: 1615 us).
+template <int LPC, int MG, typename RT, bool PHI>
+static void launch_column_refined(afid_ctx *c, const KP &p, RT *out) {
+    const long long nblk = (col_blocks<LPC, 8>(c->nyr, c->nzr) + 7) / 8 * 8;
+    hipLaunchKernelGGL((k_column_refined<LPC, MG, 8, RT, PHI>), dim3(unsigned(std::min<long long>(nblk, 512))), dim3(512), 0, c->stream, p,
+                       factors(c, PHI ? MAT_P : MAT_S), out);
+}
+template <bool PHI>
+static int column_refined(afid_ctx *c, double *outd, float *outf) {
+    KP p = make_kp(c);
+    const int n = c->nxmr;
+    if (c->mixed) {
+        if (n <= 128) launch_column_refined<32, 1, float, PHI>(c, p, outf);
+        else if (n <= 256) launch_column_refined<64, 1, float, PHI>(c, p, outf);
+        else if (n <= 384) launch_column_refined<32, 3, float, PHI>(c, p, outf);
+        else if (n <= 512) launch_column_refined<64, 2, float, PHI>(c, p, outf);
+        else if (n <= 768) launch_column_refined<64, 3, float, PHI>(c, p, outf);
+        else launch_column_refined<64, 4, float, PHI>(c, p, outf);
+    } else {
+        if (n <= 64) launch_column_refined<32, 1, double, PHI>(c, p, outd);
+        else if (n <= 128) launch_column_refined<64, 1, double, PHI>(c, p, outd);
+        else if (n <= 192) launch_column_refined<32, 3, double, PHI>(c, p, outd);
+        else if (n <= 256) launch_column_refined<64, 2, double, PHI>(c, p, outd);
+        else if (n <= 384) launch_column_refined<64, 3, double, PHI>(c, p, outd);
+        else if (n <= 512) launch_column_refined<64, 4, double, PHI>(c, p, outd);
+        else if (n <= 768) launch_column_refined<64, 6, double, PHI>(c, p, outd);
+        else launch_column_refined<64, 8, double, PHI>(c, p, outd);
+    }
+    return check_launch(c, "k_column_refined");
 }
 static int column_sal(afid_ctx *c) {
-    KP p = make_kp(c);
-    const long long nblk = strip_blocks(c->nyr, c->nzr);
-    const int ch = (c->nxmr + 63) / 64;
-    switch (ch) {
-#define AFID_CS_CASE(CH) case CH: launch_column_sal<CH>(c, p, nblk); break;
-        AFID_CS_CASE(1) AFID_CS_CASE(2) AFID_CS_CASE(3) AFID_CS_CASE(4) AFID_CS_CASE(5) AFID_CS_CASE(6)
-        AFID_CS_CASE(7) AFID_CS_CASE(8) AFID_CS_CASE(9) AFID_CS_CASE(10) AFID_CS_CASE(11) AFID_CS_CASE(12)
-        AFID_CS_CASE(13) AFID_CS_CASE(14) AFID_CS_CASE(15) AFID_CS_CASE(16)
-#undef AFID_CS_CASE
-    default: return set_err(c, AFID_E_ARG, "nxmr too large");
-    }
-    int rc = check_launch(c, "k_column_sal");
+    int rc = column_refined<false>(c, c->sal_alt, c->sal_alt_f);
     if (rc) return rc;
     if (c->mixed) std::swap(c->g[AFID_SAL], c->sal_alt_f);
     else std::swap(c->f[AFID_SAL], c->sal_alt);
     return AFID_OK;
 }
-
-template <int CH>
-static void launch_column_phi(afid_ctx *c, const KP &p, long long nblk) {
-    const dim3 gr(unsigned((nblk + 7) / 8 * 8));
-    if (c->mixed) hipLaunchKernelGGL((k_column_phi<CH, float>), gr, dim3(256), 0, c->stream, p, factors(c, MAT_P), c->phi_alt_f);
-    else hipLaunchKernelGGL((k_column_phi<CH, double>), gr, dim3(256), 0, c->stream, p, factors(c, MAT_P), c->phi_alt);
-}
 static int column_phi(afid_ctx *c) {
-    KP p = make_kp(c);
-    const long long nblk = strip_blocks(c->nyr, c->nzr);
-    const int ch = (c->nxmr + 63) / 64;
-    switch (ch) {
-#define AFID_CP_CASE(CH) case CH: launch_column_phi<CH>(c, p, nblk); break;
-        AFID_CP_CASE(1) AFID_CP_CASE(2) AFID_CP_CASE(3) AFID_CP_CASE(4) AFID_CP_CASE(5) AFID_CP_CASE(6)
-        AFID_CP_CASE(7) AFID_CP_CASE(8) AFID_CP_CASE(9) AFID_CP_CASE(10) AFID_CP_CASE(11) AFID_CP_CASE(12)
-        AFID_CP_CASE(13) AFID_CP_CASE(14) AFID_CP_CASE(15) AFID_CP_CASE(16)
-#undef AFID_CP_CASE
-    default: return set_err(c, AFID_E_ARG, "nxmr too large");
-    }
-    int rc = check_launch(c, "k_column_phi");
+    int rc = column_refined<true>(c, c->phi_alt, c->phi_alt_f);
     if (rc) return rc;
     if (c->mixed) std::swap(c->g[AFID_PHI], c->phi_alt_f);
     else std::swap(c->f[AFID_PHI], c->phi_alt);

@@ -192,32 +192,6 @@ __device__ __forceinline__ void wave_tri_solve(double (&v)[CH], const TriFactors
     for (int m = CH - 1; m >= 0; --m) { x = -e[m] * x + g[m] * v[m]; v[m] = x; }
 }
 
-// The same solve with the folded factors (TriFactors::ln, e): v in is the
-// right-hand side already scaled by sn, v out the solution.
-template <int CH>
-__device__ __forceinline__ void wave_tri_solve_folded(double (&v)[CH], const double *ln, const double *e) {
-    const int lane = threadIdx.x & 63;
-    const double *l = ln + lane * CH, *ee = e + lane * CH;
-    // forward: y'_r = v_r - ln_r y'_{r-1}
-    double A = 1.0, B = 0.0;
-#pragma unroll
-    for (int m = 0; m < CH; ++m) { const double lm = l[m]; B = -lm * B + v[m]; A = -lm * A; }
-    wave_affine_scan<true>(A, B);
-    double y = __shfl_up(B, 1, 64);
-    if (lane == 0) y = 0.0;
-#pragma unroll
-    for (int m = 0; m < CH; ++m) { y = -l[m] * y + v[m]; v[m] = y; }
-    // backward: x_r = y'_r - e_r x_{r+1}
-    A = 1.0; B = 0.0;
-#pragma unroll
-    for (int m = CH - 1; m >= 0; --m) { const double em = ee[m]; B = -em * B + v[m]; A = -em * A; }
-    wave_affine_scan<false>(A, B);
-    double x = __shfl_down(B, 1, 64);
-    if (lane == 63) x = 0.0;
-#pragma unroll
-    for (int m = CH - 1; m >= 0; --m) { x = -ee[m] * x + v[m]; v[m] = x; }
-}
-
 // 2x2 projective matrix (normalised so its largest entry is 1)
 struct Mob { double m00, m01, m10, m11; };
 __device__ __forceinline__ Mob mob_mul(const Mob &x, const Mob &y) {   // x * y
@@ -404,19 +378,6 @@ __device__ __forceinline__ void column_solve_lds(double *buf, const TriFactors &
     for (int m = 0; m < CH; ++m) buf[lane * CHP + m] = v[m];
 }
 
-// column_solve_lds with the folded factors (two tables, e.g. staged in LDS)
-template <int CH, int CHP = lds_chunk<CH>()>
-__device__ __forceinline__ void column_solve_lds_folded(double *buf, const double *ln, const double *e) {
-    const int lane = threadIdx.x & 63;
-    double v[CH];
-#pragma unroll
-    for (int m = 0; m < CH; ++m) v[m] = buf[lane * CHP + m];
-    wave_tri_solve_folded<CH>(v, ln, e);
-#pragma unroll
-    for (int m = 0; m < CH; ++m) buf[lane * CHP + m] = v[m];
-}
-
-// two-element vector of the storage type (64-bit or 128-bit lane accesses)
 // Masked solve of one column held in LDS (SolveImpEqnUpdate_X_pf /
 // _YZ_pf, phasefield.F90:821-930): rows flagged in msk are the identity with
 // the right-hand side already in buf; the others are the rows of f.
@@ -439,113 +400,10 @@ __device__ __forceinline__ void column_solve_masked_lds(double *buf, const doubl
     for (int m = 0; m < CH; ++m) buf[lane * lds_chunk<CH>() + m] = v[m];
 }
 
+// two-element vector of the storage type (64-bit or 128-bit lane accesses)
 template <typename RT> struct Pair;
 template <> struct Pair<float> { using T = float2; };
 template <> struct Pair<double> { using T = double2; };
-// 16-byte vector of the storage type: 4 floats or 2 doubles per lane access
-template <typename RT> struct Vec16;
-template <> struct Vec16<float> { using T = float4; static constexpr int n = 4; };
-template <> struct Vec16<double> { using T = double2; static constexpr int n = 2; };
-template <typename RT>
-__device__ __forceinline__ RT vget(const typename Vec16<RT>::T &v, int m) { return reinterpret_cast<const RT *>(&v)[m]; }
-
-// ExplicitSalinity + ImplicitSalinity + SolveImpEqnUpdate_Sal (salinity.F90:268-454).
-// RT is the storage (and explicit-stencil arithmetic) type of the refined
-// fields; the implicit RHS, the solve and the update run in FP64.
-// Stencil phase: each lane takes SUB adjacent rows (r0 = SUB*lane + 64*SUB*m
-// .. r0+SUB-1, 16 bytes) with one vector access per array, so a wavefront
-// access moves 1 KiB; the x-neighbours outside the group come from two
-// scalar loads that hit the same cache lines.  The RHS goes through LDS to
-// the solver's layout (CH rows per lane).
-template <int CH, typename RT>
-__global__ void __launch_bounds__(256) k_column_sal(KP p, TriFactors f, RT *sal_out) {
-    using V = typename Vec16<RT>::T;
-    constexpr int SUB = Vec16<RT>::n;
-    constexpr int MG = (64 * CH + 64 * SUB - 1) / (64 * SUB);   // group iterations covering the solver's 64*CH rows
-    __shared__ double lds[4][lds_col_size<CH>()];
-    // the solver's folded factors, read by every column of the workgroup
-    // (two tables: 39 KB of LDS in all at CH = 12, four workgroups per CU)
-    __shared__ double fac[2][64 * CH];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const unsigned lane = threadIdx.x & 63;
-    for (int q = threadIdx.x; q < 64 * CH; q += 256) { fac[0][q] = f.ln[q]; fac[1][q] = f.e[q]; }
-    int j, i;
-    const bool live = strip_column(xcd_block(0), wave, p.nyr, p.nzr, j, i);
-    double *buf = lds[wave];
-    const NbS<RT> n = make_nbs<RT>(p, j, i);
-    const long long c0 = (long long)i * p.planer + (long long)j * p.ldxr;
-    RT *rus = sel<RT>(p.rusal, p.rusalf) + c0;
-    const unsigned nxmr = p.nxmr;
-    V own[MG];
-#pragma unroll
-    for (int m = 0; m < MG; ++m) {
-        const unsigned r0 = SUB * lane + 64 * SUB * m;
-        double rhs[SUB];
-#pragma unroll
-        for (int q = 0; q < SUB; ++q) { rhs[q] = 0.0; reinterpret_cast<RT *>(&own[m])[q] = RT(0); }
-        if (live && r0 + SUB <= nxmr) {
-            // r0 a multiple of SUB and every row 8-aligned: the group is one
-            // aligned 16-byte access; r0 + SUB <= nxmr < ldxr stays in the row
-            auto ld = [&](const RT *a) { return *reinterpret_cast<const V *>(a + r0); };
-            const V sc = ld(n.s), sjm = ld(n.s_jm), sjp = ld(n.s_jp), sim = ld(n.s_im), sip = ld(n.s_ip);
-            const V vx = ld(n.vxr), vy = ld(n.vyr), vyp = ld(n.vyr_jp), vz = ld(n.vzr), vzp = ld(n.vzr_ip), ru = ld(rus);
-            const RT sm = r0 > 0 ? n.s[r0 - 1] : RT(0);
-            const RT sn = r0 + SUB < nxmr ? n.s[r0 + SUB] : RT(0);
-            const RT vn = n.vxr[r0 + SUB];
-            V h;
-#pragma unroll
-            for (int q = 0; q < SUB; ++q) {
-                const unsigned k = r0 + q;
-                const RT a = q == 0 ? sm : vget<RT>(sc, q - 1), b = vget<RT>(sc, q);
-                const RT c = q == SUB - 1 ? sn : vget<RT>(sc, q + 1);
-                const RT x1 = q == SUB - 1 ? vn : vget<RT>(vx, q + 1);
-                const RT hq = ex_sal_val<RT>(p, k, a, b, c, vget<RT>(sjm, q), vget<RT>(sjp, q), vget<RT>(sim, q),
-                                             vget<RT>(sip, q), vget<RT>(vx, q), x1, vget<RT>(vy, q), vget<RT>(vyp, q),
-                                             vget<RT>(vz, q), vget<RT>(vzp, q), n.sbp, n.stp);
-                reinterpret_cast<RT *>(&h)[q] = hq;
-                rhs[q] = rhs_sal_val(p, k, double(hq), double(vget<RT>(ru, q)), double(a), double(b), double(c), n.sbp, n.stp);
-            }
-            own[m] = sc;
-            *reinterpret_cast<V *>(rus + r0) = h;
-        } else if (live) {
-            // the group holding row nxmr - 1 when nxmr is not a multiple of SUB
-#pragma unroll
-            for (int q = 0; q < SUB; ++q) {
-                const unsigned k = r0 + q;
-                if (k < nxmr) {
-                    const RT hq = ex_sal<RT, RT>(p, n, k);
-                    rhs[q] = rhs_sal<RT>(p, n, double(hq), double(rus[k]), k);
-                    reinterpret_cast<RT *>(&own[m])[q] = n.s[k];
-                    rus[k] = hq;
-                }
-            }
-        }
-#pragma unroll
-        for (int q = 0; q < SUB; ++q)
-            if (r0 + q < 64u * CH) buf[lds_row<CH>(r0 + q)] = rhs[q] * f.sn[r0 + q];
-    }
-    __syncthreads();
-    column_solve_lds_folded<CH>(buf, fac[0], fac[1]);
-    __syncthreads();
-    if (!live) return;
-    RT *out = sal_out + c0;
-#pragma unroll
-    for (int m = 0; m < MG; ++m) {
-        const unsigned r0 = SUB * lane + 64 * SUB * m;
-        if (r0 >= nxmr) continue;
-        V o;
-#pragma unroll
-        for (int q = 0; q < SUB; ++q)
-            reinterpret_cast<RT *>(&o)[q] = RT(double(vget<RT>(own[m], q)) + (r0 + q < 64u * CH ? buf[lds_row<CH>(r0 + q)] : 0.0));
-        if (r0 + SUB <= nxmr) *reinterpret_cast<V *>(out + r0) = o;
-        else
-#pragma unroll
-            for (int q = 0; q < SUB; ++q)
-                if (r0 + q < nxmr) out[r0 + q] = vget<RT>(o, q);
-    }
-    if (lane == 0) out[nxmr] = n.s[nxmr];       // the unused index nxr is carried over
-}
-
 // Explicit terms of vx, vy, vz, T (+ AddSalBuoyancy) and ImplicitAndUpdate
 // VX/VY/VZ/Temp with their solves (TimeMarcher.F90:45-95) for one column.
 struct BaseOut { double *vx, *vy, *vz, *temp; };

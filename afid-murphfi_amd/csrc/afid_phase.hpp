@@ -57,83 +57,6 @@ __global__ void __launch_bounds__(256) k_volume_penalty(KP p) {
     p.dq[c] -= (pc[c] + pc[bidx(p, k, j, im)]) * p.vz[c] * p.heta;
 }
 
-// ExplicitPhase + ImplicitPhase + SolveImpEqnUpdate_Phi (phasefield.F90:
-// 345-466) for one refined column per wavefront, rows in pairs as in
-// k_column_sal.  Writes the new phi to phi_out, the explicit term to ruphi
-// and the increment phi(l+1) - phi(l) to rhsr (read by AddLatentHeat).
-// RT: storage and explicit-term arithmetic of the refined arrays; the
-// implicit RHS, the solve and the update run in FP64.
-template <int CH, typename RT>
-__global__ void __launch_bounds__(256) k_column_phi(KP p, TriFactors f, RT *phi_out) {
-    using V = typename Pair<RT>::T;
-    constexpr int M2 = (64 * CH + 127) / 128;
-    __shared__ double lds[4][lds_col_size<CH>()];
-    // the solver's folded factors, read by every column of the workgroup
-    __shared__ double fac[2][64 * CH];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const unsigned lane = threadIdx.x & 63;
-    for (int q = threadIdx.x; q < 64 * CH; q += 256) { fac[0][q] = f.ln[q]; fac[1][q] = f.e[q]; }
-    int j, i;
-    const bool live = strip_column(xcd_block(0), wave, p.nyr, p.nzr, j, i);
-    double *buf = lds[wave];
-    const int jm = wrapm(j, p.nyr), jp = wrapp(j, p.nyr), im = wrapm(i, p.nzr), ip = wrapp(i, p.nzr);
-    auto col = [&](int jj, int ii) { return (long long)ii * p.planer + (long long)jj * p.ldxr; };
-    const long long c0 = col(j, i);
-    const RT *phi = sel<RT>(p.phi, p.phif);
-    const RT *ph = phi + c0, *pym = phi + col(jm, i), *pyp = phi + col(jp, i);
-    const RT *pzm = phi + col(j, im), *pzp = phi + col(j, ip), *tr = sel<RT>(p.tempr, p.temprf) + c0;
-    RT *ru = sel<RT>(p.ruphi, p.ruphif) + c0;
-    const unsigned nxmr = p.nxmr;
-    V own[M2];
-#pragma unroll
-    for (int m = 0; m < M2; ++m) {
-        const unsigned r0 = 2 * lane + 128 * m, r1 = r0 + 1;
-        double rhs0 = 0.0, rhs1 = 0.0;
-        own[m] = V{RT(0), RT(0)};
-        if (live && r0 < nxmr) {
-            // r0 even, rows 8-aligned: aligned pairs; r0 + 1 <= nxmr < ldxr
-            const V pc = *reinterpret_cast<const V *>(ph + r0);
-            const V a = *reinterpret_cast<const V *>(pym + r0), b = *reinterpret_cast<const V *>(pyp + r0);
-            const V cz = *reinterpret_cast<const V *>(pzm + r0), d = *reinterpret_cast<const V *>(pzp + r0);
-            const V t = *reinterpret_cast<const V *>(tr + r0), u = *reinterpret_cast<const V *>(ru + r0);
-            const RT pm = r0 > 0 ? ph[r0 - 1] : RT(0);
-            const RT pp2 = r1 + 1 < nxmr ? ph[r1 + 1] : RT(0);
-            const RT h0 = ex_phase_val<RT>(p, pc.x, a.x, b.x, cz.x, d.x, t.x);
-            rhs0 = rhs_phase_val(p, r0, double(h0), double(u.x), double(pm), double(pc.x), double(pc.y));
-            own[m] = pc;
-            if (r1 < nxmr) {
-                const RT h1 = ex_phase_val<RT>(p, pc.y, a.y, b.y, cz.y, d.y, t.y);
-                rhs1 = rhs_phase_val(p, r1, double(h1), double(u.y), double(pc.x), double(pc.y), double(pp2));
-                *reinterpret_cast<V *>(ru + r0) = V{h0, h1};
-            } else {
-                ru[r0] = h0;
-            }
-        }
-        if (r0 < 64u * CH) buf[lds_row<CH>(r0)] = rhs0 * f.sn[r0];
-        if (r1 < 64u * CH) buf[lds_row<CH>(r1)] = rhs1 * f.sn[r1];
-    }
-    __syncthreads();
-    column_solve_lds_folded<CH>(buf, fac[0], fac[1]);
-    __syncthreads();
-    if (!live) return;
-    RT *out = phi_out + c0, *dphi = sel<RT>(p.rhsr, p.rhsrf) + c0;
-#pragma unroll
-    for (int m = 0; m < M2; ++m) {
-        const unsigned r0 = 2 * lane + 128 * m, r1 = r0 + 1;
-        if (r0 >= nxmr) continue;
-        const double d0 = buf[lds_row<CH>(r0)];
-        if (r1 < nxmr) {
-            const double d1 = buf[lds_row<CH>(r1)];
-            *reinterpret_cast<V *>(out + r0) = V{RT(double(own[m].x) + d0), RT(double(own[m].y) + d1)};
-            *reinterpret_cast<V *>(dphi + r0) = V{RT(d0), RT(d1)};
-        } else {
-            out[r0] = RT(double(own[m].x) + d0);
-            dphi[r0] = RT(d0);
-        }
-    }
-    if (lane == 0) out[nxmr] = ph[nxmr];        // the unused index nxr is carried over
-}
-
 // SolveImpEqnUpdate_X_pf / _YZ_pf (phasefield.F90:821-930) for the
 // per-routine path: one column per wavefront, rhs as assembled by
 // ImplicitAndUpdateV*, q updated in place (rows 2..nxm of vx, 1..nxm of
