@@ -25,6 +25,7 @@
 #include "afid_column.hpp"
 #include "afid_poisson.hpp"
 #include "afid_phase.hpp"
+#include "afid_transfer.hpp"
 #include "afid_means.hpp"
 #include "afid_restart.hpp"
 #include "afid_ibm.hpp"
@@ -84,7 +85,6 @@ struct afid_ctx {
     double *alt[4] = {nullptr};        // second buffers of vx, vy, vz, temp (fused column step)
     double *sal_alt = nullptr;
     float *sal_alt_f = nullptr;
-    double *tpdv = nullptr;
     void *spec = nullptr;              // cpx<double> (FP64 form) or cpx<float> (mixed form)
     // phase field
     bool pf = false;
@@ -118,7 +118,6 @@ struct afid_ctx {
     double *d_phi_part = nullptr, *d_phi_out = nullptr;
     int mean_groups = 0, sal_groups = 0, phi_groups = 0;
     bool col_four_pass = false;         // base columns through the four-pass kernel (AFID_COLUMN_FOUR_PASS=1)
-    bool vyz_tile = false;              // vyr / vzr through the LDS tile kernel (AFID_VYZ_TILE=1)
     // mixed form, gAxis = 1: the FP32 vx explicit term and its history hold
     // the buoyancy minus a per-row FP64 reference bref (that of the
     // conductive profile between the mean wall temperatures), which the FP64
@@ -161,9 +160,16 @@ struct afid_ctx {
     PoissonFactors<double> pois{};
     PoissonFactors<float> pff{};
     int pchunk = 1;
-    // LDS plan of the transfer kernels
-    int vxr_xc = 0, vxr_cj = 0, vxr_ci = 0, vy_cs = 0, vy_co = 0, vz_cs = 0, vz_co = 0;
-    size_t lds_vxr = 0, lds_vy = 0, lds_vz = 0;
+    // coarse -> refined transfers: rows of refined x per coarse column, and
+    // those of the velocity of the first plane (k_xfer_x); whether pairs
+    // of refined z lines read at most 5 coarse ones (k_xfer_yz)
+    void *xfer = nullptr, *xfer0 = nullptr;
+    bool pair_z = false;
+    // refined steps of y / z two by two (ratio 2, see XferJob::two)
+    bool two_y = false, two_z = false;
+    // vyr, vzr, tempr uploaded by the host since their unused index nxr was
+    // last known to be zero (InterpVelMgrd.F90:29-31, phasefield.F90:502)
+    bool tail_dirty[3] = {false, false, false};
     // reductions
     unsigned long long *redmax = nullptr;
     double *redsum = nullptr, *redout = nullptr;
@@ -247,7 +253,7 @@ static KP make_kp(const afid_ctx *c) {
     p.rux = c->f[AFID_RUX]; p.ruy = c->f[AFID_RUY]; p.ruz = c->f[AFID_RUZ]; p.rut = c->f[AFID_RUTEMP];
     p.qcap = c->f[AFID_QCAP]; p.dph = c->f[AFID_DPH]; p.dq = c->f[AFID_DQ]; p.hro = c->f[AFID_HRO];
     p.rhsx = c->rhs4[0]; p.rhsy = c->rhs4[1]; p.rhsz = c->rhs4[2]; p.rhst = c->rhs4[3];
-    p.salc = c->f[AFID_SALC]; p.tpdv = c->tpdv;
+    p.salc = c->f[AFID_SALC];
     p.tempbp = c->f[AFID_TEMPBP]; p.temptp = c->f[AFID_TEMPTP];
     p.sal = c->f[AFID_SAL]; p.rusal = c->f[AFID_RUSAL]; p.hsal = c->f[AFID_HSAL]; p.rhsr = c->f[AFID_RHSR];
     p.vxr = c->f[AFID_VXR]; p.vyr = c->f[AFID_VYR]; p.vzr = c->f[AFID_VZR];
@@ -928,23 +934,37 @@ static int setup(afid_ctx *c) {
         }
         return m;
     };
-    c->vxr_xc = span(sx.src, nxmr, 64);
-    if (c->vxr_xc > 128) return set_err(c, AFID_E_ARG, "refined x coarser than the base x is not supported");
-    c->vxr_cj = span(sy.src, nyr, VXR_TJ);
-    c->vxr_ci = span(sz.src, nzr, VXR_TI);
-    if (c->vxr_cj * c->vxr_ci > 256) return set_err(c, AFID_E_ARG, "refinement ratio too small for the vxr tiles");
-    const size_t es = c->mixed ? sizeof(float) : sizeof(double);      // element size of the transfer LDS
-    c->lds_vxr = es * size_t(c->vxr_xc * c->vxr_cj * c->vxr_ci + c->vxr_xc * c->vxr_cj * VXR_TI +
-                             c->vxr_xc * VXR_TJ * VXR_TI);
-    c->vy_cs = span(sy.src, nyr - 1, VYZ_CHUNK); c->vy_co = span(sz.src, nzr, VYZ_LINES);
-    c->vz_cs = span(sz.src, nzr - 1, VYZ_CHUNK); c->vz_co = span(sy.src, nyr, VYZ_LINES);
-    if (std::max(std::max(c->vy_cs, c->vz_cs), std::max(c->vy_co, c->vz_co)) > 32)
-        return set_err(c, AFID_E_ARG, "refinement ratio too small for the vyr/vzr tiles");
-    auto lds_yz = [&](int cs, int co) {
-        return es * size_t(std::max(c->vxr_xc * cs * co, cs * VYZ_LINES * 64) + c->vxr_xc * cs * VYZ_LINES);
+    auto pairs = [](const std::vector<int> &src, int n) {
+        for (int a = 0; a + 1 < n; a += 2)
+            if (src[size_t(a + 1)] - src[size_t(a)] > 1) return false;
+        return true;
     };
-    c->lds_vy = lds_yz(c->vy_cs, c->vy_co);
-    c->lds_vz = lds_yz(c->vz_cs, c->vz_co);
+    auto twos = [](const std::vector<int> &src, int n) {
+        for (int a = 1; a < n; ++a)
+            if (src[size_t(a)] != src[1] + (a - 1) / 2) return false;
+        return src[0] == src[1] - 1;
+    };
+    c->two_y = twos(sy.src, nyr);
+    c->two_z = twos(sz.src, nzr);
+    c->pair_z = pairs(sz.src, nzr);
+    {
+        const size_t e = c->mixed ? sizeof(float) : sizeof(double);
+        if ((rc = dalloc(c, &c->xfer, e * size_t(c->nz) * c->ny * c->ldxr))) return rc;
+        if ((rc = dalloc(c, &c->xfer0, e * size_t(std::max(c->ny, c->nz)) * c->ldxr))) return rc;
+    }
+    // Refinement ratios that set-up admits: the coarse spans of 64 x, 16 y and
+    // 4 z refined points of the transfers, as a block of 64 KiB holds them.
+    const size_t es = c->mixed ? sizeof(float) : sizeof(double);
+    const int x64 = span(sx.src, nxmr, 64);
+    if (x64 > 128) return set_err(c, AFID_E_ARG, "refined x coarser than the base x is not supported");
+    const int y16 = span(sy.src, nyr, 16), z4 = span(sz.src, nzr, 4);
+    if (y16 * z4 > 256) return set_err(c, AFID_E_ARG, "refinement ratio too small for the vxr tiles");
+    const int ys = span(sy.src, nyr - 1, 16), yo = span(sz.src, nzr, 4);
+    const int zs = span(sz.src, nzr - 1, 16), zo = span(sy.src, nyr, 4);
+    if (std::max(std::max(ys, zs), std::max(yo, zo)) > 32)
+        return set_err(c, AFID_E_ARG, "refinement ratio too small for the vyr/vzr tiles");
+    const auto block_yz = [&](int cs, int co) { return es * size_t(std::max(x64 * cs * co, cs * 4 * 64) + x64 * cs * 4); };
+    const size_t most = std::max(es * size_t(x64 * y16 * z4 + x64 * y16 * 4 + x64 * 16 * 4), std::max(block_yz(ys, yo), block_yz(zs, zo)));
     // refined -> coarse tiles: 64 coarse x by SALC_TJ coarse y, two refined
     // planes of the tile in LDS (storage type of the refined field)
     for (int q = 0; q < 2; ++q) {
@@ -957,7 +977,7 @@ static int setup(afid_ctx *c) {
         t.lds = es * size_t(2 * t.yr * t.xr);
         if (t.lds > 65536) return set_err(c, AFID_E_ARG, "refinement ratio too small for the refined -> coarse tiles");
     }
-    if (c->lds_vxr > 65536 || c->lds_vy > 65536 || c->lds_vz > 65536)
+    if (most > 65536)
         return set_err(c, AFID_E_ARG, "refinement ratio too small for the transfer tiles (LDS plan above 64 KiB)");
     return AFID_OK;
 }
@@ -985,7 +1005,6 @@ static int ctx_create(const afid_config *cfg, hipStream_t shared, afid_ctx **out
     }
     c->device = dev;
     if (const char *e = std::getenv("AFID_COLUMN_FOUR_PASS")) c->col_four_pass = std::atoi(e) != 0;
-    if (const char *e = std::getenv("AFID_VYZ_TILE")) c->vyz_tile = std::atoi(e) != 0;
     if (const char *e = std::getenv("AFID_FFT_Z16")) c->fft_z16 = std::atoi(e) != 0;
     if (shared) {
         c->stream = shared;
@@ -1062,6 +1081,8 @@ int afid_upload(afid_ctx *c, int f, const double *host, const int64_t lb[3], con
             HIPCHK(c, hipMemcpy(c->f[f] + size_t(i - 1) * ny * ld, slab.data(), sizeof(double) * slab.size(), hipMemcpyHostToDevice));
         }
     }
+    for (int q = 0; q < 3; ++q)
+        if (f == (q == 0 ? AFID_VYR : q == 1 ? AFID_VZR : AFID_TEMPR)) c->tail_dirty[q] = true;
     if (f == AFID_TEMPBP || f == AFID_TEMPTP) {
         double sum = 0.0;
         for (int i = 1; i <= nz; ++i)
@@ -1433,11 +1454,118 @@ static int poisson_mixed(afid_ctx *c) {
     return AFID_OK;
 }
 
-// vyr / vzr, one wavefront per refined line (k_vyz_wave)
-template <int AX, bool TWO>
-static void launch_vyz_wave(afid_ctx *c, const KP &p, dim3 grid, int nxc) {
-    if (c->mixed) hipLaunchKernelGGL((k_vyz_wave<AX, float, TWO>), grid, dim3(256), 0, c->stream, p, nxc);
-    else hipLaunchKernelGGL((k_vyz_wave<AX, double, TWO>), grid, dim3(256), 0, c->stream, p, nxc);
+static constexpr int kTailFields[3] = {AFID_VYR, AFID_VZR, AFID_TEMPR};
+// the reference clears vyr, vzr, tempr before it fills them: index nxr, which
+// no kernel writes, after an upload that may have set it
+static int clean_tails(afid_ctx *c) {
+    for (int q = 0; q < 3; ++q) {
+        if (!c->tail_dirty[q]) continue;
+        const long long rows = (long long)c->nyr * c->nzr;
+        const dim3 gr(unsigned((rows + 255) / 256));
+        if (float *g = c->g[kTailFields[q]]) hipLaunchKernelGGL(k_zero_tail<float>, gr, dim3(256), 0, c->stream, g, c->nxmr, c->ldxr, rows);
+        else hipLaunchKernelGGL(k_zero_tail<double>, gr, dim3(256), 0, c->stream, c->f[kTailFields[q]], c->nxmr, c->ldxr, rows);
+        int rc = check_launch(c, "k_zero_tail");
+        if (rc) return rc;
+        c->tail_dirty[q] = false;
+    }
+    return AFID_OK;
+}
+// one coarse -> refined transfer: the x part of every coarse column, then the
+// y / z part of every refined line
+template <typename RT, int FLD>
+static int xfer_x(afid_ctx *c, const KP &p) {
+    const long long ncol = (long long)c->ny * c->nz;
+    const int ch = (std::max(c->nxm, c->nxmr) + 63) / 64;
+    RT *D = static_cast<RT *>(c->xfer), *F = static_cast<RT *>(c->xfer0);
+    // 512 workgroups: two on each CU, each loading the weights once; fewer
+    // wavefronts where the rows of 8 do not fit beside the weights in 64 KiB
+    auto launch = [&](auto k, int chr) {
+        int waves = XFX_WAVES;
+        auto lds = [&] { return sizeof(RT) * (size_t(4) * 64 * chr + waves * size_t(c->nxm + 4)); };
+        while (waves > 1 && lds() > 65536) waves /= 2;
+        const dim3 gr(unsigned(std::min<long long>((ncol + 8 * waves - 1) / (8 * waves) * 8, 512 * XFX_WAVES / waves)));
+        hipLaunchKernelGGL(k, gr, dim3(64u * unsigned(waves)), lds(), c->stream, p, D, F);
+    };
+#define AFID_XF(CH) launch(k_xfer_x<CH, RT, FLD>, CH)
+    if (ch <= 1) AFID_XF(1);
+    else if (ch <= 2) AFID_XF(2);
+    else if (ch <= 3) AFID_XF(3);
+    else if (ch <= 4) AFID_XF(4);
+    else if (ch <= 6) AFID_XF(6);
+    else if (ch <= 8) AFID_XF(8);
+    else if (ch <= 12) AFID_XF(12);
+    else AFID_XF(16);
+#undef AFID_XF
+    return check_launch(c, "k_xfer_x");
+}
+// Lines per wavefront: pairs for vxr and T (5 coarse rows instead of 8 for two
+// refined ones: 438 us a step against 527 with single lines, vxr of 128 x 192^2
+// -> 256 x 384^2 FP64), single lines for the sums of vyr / vzr, where a pair's
+// registers leave one wavefront per SIMD (395 us against 418 there, 71 against
+// 97 at 64^3 -> 128^3).
+// nseg: ranges until the card has wavefronts enough.  vxr and T take 2048 (a
+// range costs them 3 more coarse steps: 768 x 384^2 FP64 437 -> 367 us a
+// launch), the sums, which run a range twice, 1024 (128 x 192^2: 31 -> 23 us).
+template <typename RT, int NR, int NL, bool SUM>
+static void launch_xfer_yz(afid_ctx *c, XferJob &jb) {
+    const long long nch = (jb.nx + 64 * NR - 1) / (64 * NR), ngr = (jb.nO + NL - 1) / NL, waves = nch * ngr;
+    jb.nseg = 1;
+    while (jb.nseg < 8 && waves * jb.nseg < (SUM ? 1024 : 2048)) jb.nseg *= 2;
+    const size_t lds = SUM && jb.nseg > 1 ? sizeof(RT) * NR * 64 * NL * size_t(jb.nseg) : 0;
+    if (jb.nseg > 1)
+        hipLaunchKernelGGL((k_xfer_yz<RT, NR, NL, SUM, true>), dim3(tile_grid(waves)), dim3(64u * unsigned(jb.nseg)), lds, c->stream, jb);
+    else
+        hipLaunchKernelGGL((k_xfer_yz<RT, NR, NL, SUM, false>), dim3(tile_grid((waves + 3) / 4)), dim3(256), 0, c->stream, jb);
+}
+// refined x per lane: 16 bytes; in FP32 8 on rows of up to 512 that 16 would
+// not fill (192 points: one wavefront of 64 lanes or 1.5 of 32 useful ones)
+template <typename RT, bool SUM>
+static int xfer_yz(afid_ctx *c, XferJob &jb, bool pair) {
+    const bool wide = sizeof(RT) == 4 && (c->nxmr % 256 == 0 || c->nxmr > 512);
+    constexpr int W = sizeof(RT) == 4 ? 4 : 2;
+    if constexpr (SUM) {
+        if (wide) launch_xfer_yz<RT, W, 1, SUM>(c, jb);
+        else launch_xfer_yz<RT, 2, 1, SUM>(c, jb);
+    } else {
+        if (pair && wide) launch_xfer_yz<RT, W, 2, SUM>(c, jb);
+        else if (pair) launch_xfer_yz<RT, 2, 2, SUM>(c, jb);
+        else if (wide) launch_xfer_yz<RT, W, 1, SUM>(c, jb);
+        else launch_xfer_yz<RT, 2, 1, SUM>(c, jb);
+    }
+    return check_launch(c, "k_xfer_yz");
+}
+// walks y (vzr: z) with the other axis' lines as the units
+template <typename RT, int FLD>
+static int xfer(afid_ctx *c, RT *out, const char *timer) {
+    KP p = make_kp(c);
+    int rc = clean_tails(c);
+    if (rc) return rc;
+    tstart(c, timer);
+    if ((rc = xfer_x<RT, FLD>(c, p))) return rc;
+    constexpr bool SUM = FLD == XF_VY || FLD == XF_VZ;
+    const long long plane = (long long)c->ny * c->ldxr;
+    const RT *yw = sizeof(RT) == 8 ? reinterpret_cast<const RT *>(c->d_ys_w) : reinterpret_cast<const RT *>(c->f_ys_w);
+    const RT *zw = sizeof(RT) == 8 ? reinterpret_cast<const RT *>(c->d_zs_w) : reinterpret_cast<const RT *>(c->f_zs_w);
+    XferJob jb{};
+    jb.D = c->xfer; jb.out = out; jb.nx = c->nxmr; jb.ld = c->ldxr;
+    // vzr starts from zero on a single plane (InterpVelMgrd.F90:184)
+    jb.F = FLD == XF_VY || (FLD == XF_VZ && c->nz > 1) ? c->xfer0 : nullptr;
+    if (FLD == XF_VZ) {
+        jb.s_src = c->d_zs_src; jb.o_src = c->d_ys_src; jb.s_w = zw; jb.o_w = yw;
+        jb.nS = c->nzr; jb.nO = c->nyr; jb.cS = c->nz; jb.cO = c->ny;
+        jb.ds = plane; jb.dq = c->ldxr; jb.rs = p.planer; jb.ro = c->ldxr; jb.dl = 1.0 / c->dzr;
+    } else {
+        jb.s_src = c->d_ys_src; jb.o_src = c->d_zs_src; jb.s_w = yw; jb.o_w = zw;
+        jb.nS = c->nyr; jb.nO = c->nzr; jb.cS = c->ny; jb.cO = c->nz;
+        jb.ds = c->ldxr; jb.dq = plane; jb.rs = c->ldxr; jb.ro = p.planer; jb.dl = 1.0 / c->dyr;
+    }
+    // vxr has a face more; the other fields leave the unused index nxr alone
+    // (zero: clean_tails)
+    if (FLD == XF_VX) jb.nx = c->nxr;
+    jb.two = (FLD == XF_VZ ? c->two_z : c->two_y) ? 1 : 0;
+    rc = xfer_yz<RT, SUM>(c, jb, c->pair_z);
+    tstop(c);
+    return rc;
 }
 
 extern "C" {
@@ -1447,46 +1575,23 @@ int afid_solve_pressure_correction(afid_ctx *c) { NEED_SUBSTEP(c) NEED_FP64(c) r
 int afid_correct_velocity(afid_ctx *c) { NEED_SUBSTEP(c) NEED_FP64(c) return project(c, 1, 0); }
 int afid_correct_pressure(afid_ctx *c) { NEED_SUBSTEP(c) NEED_FP64(c) return project(c, 0, 1); }
 
+// us per step (3 launches; vxr / vyr / vzr), tiles in LDS and refined lines
+// with lane shuffles before, k_xfer_x + k_xfer_yz now:
+//   64^3 -> 128^3 FP64                 75 / 157 / 160       61 / 71 / 71
+//   128 x 192^2 -> 256 x 384^2 FP64    657 / 689 / 695      441 / 400 / 388
+//   384 x 192^2 -> 768 x 384^2 FP64    2032 / 1690 / 1741   1355 / 1361 / 1249
+//   384 x 384^2 -> 768^3 FP32          3950 / 4344 / 4345   3182 / 3018 / 3001
+// and T at 128 x 256^2 -> 256 x 512^2 FP64 1227 -> 611.
 static int interp_vel(afid_ctx *c) {
-    KP p = make_kp(c);
     int rc;
-    const dim3 gx(tile_grid((long long)((c->nyr + VXR_TJ - 1) / VXR_TJ) * ((c->nzr + VXR_TI - 1) / VXR_TI)));
-    const dim3 gy(unsigned((c->nxmr + 63) / 64), unsigned((c->nzr + VYZ_LINES - 1) / VYZ_LINES));
-    const dim3 gz(unsigned((c->nxmr + 63) / 64), unsigned((c->nyr + VYZ_LINES - 1) / VYZ_LINES));
-    tstart(c, "mgrd_vxr");
-    if (c->mixed) hipLaunchKernelGGL(k_vxr_tile<float>, gx, dim3(256), c->lds_vxr, c->stream, p, c->vxr_xc, c->vxr_cj, c->vxr_ci);
-    else hipLaunchKernelGGL(k_vxr_tile<double>, gx, dim3(256), c->lds_vxr, c->stream, p, c->vxr_xc, c->vxr_cj, c->vxr_ci);
-    tstop(c);
-    if ((rc = check_launch(c, "k_vxr_tile"))) return rc;
-    if (c->vyz_tile) {
-        tstart(c, "mgrd_vyr");
-        if (c->mixed) hipLaunchKernelGGL((k_vyz_tile<1, float>), gy, dim3(64 * VYZ_LINES), c->lds_vy, c->stream, p, c->vxr_xc, c->vy_cs, c->vy_co);
-        else hipLaunchKernelGGL((k_vyz_tile<1, double>), gy, dim3(64 * VYZ_LINES), c->lds_vy, c->stream, p, c->vxr_xc, c->vy_cs, c->vy_co);
-        tstop(c);
-        if ((rc = check_launch(c, "k_vyz_tile<1>"))) return rc;
-        tstart(c, "mgrd_vzr");
-        if (c->mixed) hipLaunchKernelGGL((k_vyz_tile<2, float>), gz, dim3(64 * VYZ_LINES), c->lds_vz, c->stream, p, c->vxr_xc, c->vz_cs, c->vz_co);
-        else hipLaunchKernelGGL((k_vyz_tile<2, double>), gz, dim3(64 * VYZ_LINES), c->lds_vz, c->stream, p, c->vxr_xc, c->vz_cs, c->vz_co);
-        tstop(c);
-        return check_launch(c, "k_vyz_tile<2>");
+    if (c->mixed) {
+        if ((rc = xfer<float, XF_VX>(c, c->g[AFID_VXR], "mgrd_vxr"))) return rc;
+        if ((rc = xfer<float, XF_VY>(c, c->g[AFID_VYR], "mgrd_vyr"))) return rc;
+        return xfer<float, XF_VZ>(c, c->g[AFID_VZR], "mgrd_vzr");
     }
-    // one wavefront per refined line: (x chunks) x (groups of 4 lines)
-    // workgroups, padded to a multiple of 8 for the XCD map
-    // (a chunk of 64 refined x spanning more than 64 coarse points, refinement
-    // ratio below 1.05 in x, takes the second register per lane)
-    const int nxc = (c->nxmr + 63) / 64;
-    const dim3 wy(unsigned(((long long)nxc * ((c->nzr + 3) / 4) + 7) / 8 * 8));
-    const dim3 wz(unsigned(((long long)nxc * ((c->nyr + 3) / 4) + 7) / 8 * 8));
-    tstart(c, "mgrd_vyr");
-    if (c->vxr_xc > 64) launch_vyz_wave<1, true>(c, p, wy, nxc);
-    else launch_vyz_wave<1, false>(c, p, wy, nxc);
-    tstop(c);
-    if ((rc = check_launch(c, "k_vyz_wave<1>"))) return rc;
-    tstart(c, "mgrd_vzr");
-    if (c->vxr_xc > 64) launch_vyz_wave<2, true>(c, p, wz, nxc);
-    else launch_vyz_wave<2, false>(c, p, wz, nxc);
-    tstop(c);
-    return check_launch(c, "k_vyz_wave<2>");
+    if ((rc = xfer<double, XF_VX>(c, c->f[AFID_VXR], "mgrd_vxr"))) return rc;
+    if ((rc = xfer<double, XF_VY>(c, c->f[AFID_VYR], "mgrd_vyr"))) return rc;
+    return xfer<double, XF_VZ>(c, c->f[AFID_VZR], "mgrd_vzr");
 }
 int afid_interp_vel_mgrd(afid_ctx *c) { NEED_SAL(c) return interp_vel(c); }
 
@@ -1544,13 +1649,8 @@ int afid_interp_phi_multigrid(afid_ctx *c) {
 }
 int afid_interp_temp_multigrid(afid_ctx *c) {
     NEED_PF(c)
-    KP p = make_kp(c);
-    tstart(c, "pf_interp_temp");
-    const dim3 gr(unsigned((c->nyr + VXR_TJ - 1) / VXR_TJ), unsigned((c->nzr + VXR_TI - 1) / VXR_TI));
-    if (c->mixed) hipLaunchKernelGGL(k_interp_temp_tile<float>, gr, dim3(256), c->lds_vxr, c->stream, p, c->vxr_xc, c->vxr_cj, c->vxr_ci);
-    else hipLaunchKernelGGL(k_interp_temp_tile<double>, gr, dim3(256), c->lds_vxr, c->stream, p, c->vxr_xc, c->vxr_cj, c->vxr_ci);
-    tstop(c);
-    return check_launch(c, "k_interp_temp_tile");
+    if (c->mixed) return xfer<float, XF_T>(c, c->g[AFID_TEMPR], "pf_interp_temp");
+    return xfer<double, XF_T>(c, c->f[AFID_TEMPR], "pf_interp_temp");
 }
 
 }  // extern "C"
@@ -1824,6 +1924,8 @@ int afid_time_marcher_graph(afid_ctx *c, double dt, int nsteps) {
         for (int f = 0; f < AFID_NFIELDS; ++f) c->graph_ptrs[f] = c->f[f];
     }
     int done = 0;
+    // (an upload between replays: the captured steps leave index nxr alone)
+    if (nsteps > 0 && (rc = clean_tails(c))) return rc;
     if (c->graph)
         for (; done + 2 <= nsteps; done += 2) HIPCHK(c, hipGraphLaunch(c->graph, c->stream));
     for (; done < nsteps; ++done)

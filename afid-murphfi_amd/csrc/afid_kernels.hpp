@@ -309,21 +309,6 @@ __device__ __forceinline__ long long xcd_block(long long) {
 // tiles, which read the same halo cache lines, run on one L2 at about the
 // same time.  False for the padding workgroups.
 __host__ __device__ __forceinline__ unsigned tile_grid(long long ntiles) { return unsigned((ntiles + 7) / 8 * 8); }
-// The vxr tiles (ny_tiles x nz_tiles) in groups of TILE_GY y tiles walked
-// z-fastest: y-neighbour tiles are 1 apart and z-neighbour tiles, which
-// share 3 of the 5 coarse planes of their block, TILE_GY apart, so both are
-// in flight on one XCD together.
-constexpr int TILE_GY = 4;
-__device__ __forceinline__ bool tile_yz_grouped(int nyt, int nzt, int &ty, int &tz) {
-    const long long t = xcd_block(0);
-    if (t >= (long long)nyt * nzt) return false;
-    const long long per = (long long)TILE_GY * nzt;
-    const int g = int(t / per), r = int(t - g * per);
-    const int w = min(TILE_GY, nyt - g * TILE_GY);      // the last group may be narrower
-    ty = g * TILE_GY + r % w;
-    tz = r / w;
-    return true;
-}
 __device__ __forceinline__ bool tile_3d(int nxt, int nyt, int nzt, int &tx, int &ty, int &tz) {
     const long long t = xcd_block(0);
     if (t >= (long long)nxt * nyt * nzt) return false;
@@ -843,35 +828,6 @@ __global__ void __launch_bounds__(256) k_max_partials(const double *partial, lon
 // ---------------------------------------------------------------------------
 // multiresolution transfers
 // ---------------------------------------------------------------------------
-// tiled transfers of InterpVelMgrd: the coarse gradient is computed on the
-// fly from the velocity (InterpVelMgrd.F90:37-51, :75-86, :161-172, with the
-// wall ghosts), a coarse block is staged in LDS once per tile, contracted
-// axis by axis (separable Hermite stencil), and the transferred gradient is
-// integrated along its axis with the running sum carried across chunks.
-// ---------------------------------------------------------------------------
-// coarse gradient of component comp at reference x index xc (-1..nx+1) and
-// 0-based periodic (j, i); the difference of the FP64 velocities is taken in
-// FP64 and handed on in the transfer type RT
-template <typename RT>
-__device__ __forceinline__ RT mgrd_grad(const KP &p, int comp, int xc, int j, int i) {
-    int kc = xc, sgn = 1;
-    if (xc == 0) { kc = 1; sgn = 1 - 2 * p.inslws; }
-    else if (xc == p.nx) { kc = p.nxm; sgn = 1 - 2 * p.inslwn; }
-    else if (xc < 0 || xc > p.nx) return RT(0);
-    const int k = kc - 1;
-    double d;
-    if (comp == 0) {
-        const double *c = p.vx + (long long)i * p.plane + (long long)j * p.ldx;
-        d = (c[k + 1] - c[k]) * p.udx3m[k];
-    } else if (comp == 1) {
-        const double *c = p.vy + (long long)i * p.plane;
-        d = (c[(long long)wrapp(j, p.ny) * p.ldx + k] - c[(long long)j * p.ldx + k]) * p.dy;
-    } else {
-        const double *c = p.vz + (long long)j * p.ldx;
-        d = (c[(long long)wrapp(i, p.nz) * p.plane + k] - c[(long long)i * p.plane + k]) * p.dz;
-    }
-    return RT(sgn * d);
-}
 __device__ __forceinline__ int wrapn(int j, int n) { j %= n; return j < 0 ? j + n : j; }
 // periodic wrap of an index a few periods away at most, without a division
 __device__ __forceinline__ int wrapf(int j, int n) {
@@ -879,10 +835,6 @@ __device__ __forceinline__ int wrapf(int j, int n) {
     while (j >= n) j -= n;
     return j;
 }
-
-// (c * B + b) * A + a for staging-block indices (all below 2^24): 24-bit
-// multiplies, which issue at full rate
-__device__ __forceinline__ int ix3(int c, int B, int b, int A, int a) { return __mul24(__mul24(c, B) + b, A) + a; }
 
 // Components (a, b, c) of a linear index q = a + A (b + B c) that advances by a
 // fixed step: the divisions happen once, each step costs a few adds.
@@ -898,13 +850,6 @@ struct Walk3 {
         if (b >= B) { b -= B; ++c; }
     }
 };
-
-// Tile sizes of the transfer kernels (host computes the LDS each needs).
-constexpr int VXR_TJ = 16, VXR_TI = 4;      // refined columns per vxr tile
-constexpr int VYZ_LINES = 4;                // refined lines (waves) per vyr/vzr tile
-constexpr int VYZ_CHUNK = 16;               // refined points per scan chunk
-constexpr int VXR_BU = 4, VYZ_BU = 4;       // coarse-block items loaded per batch and thread
-constexpr int VYZ_NB = 4;                   // coarse planes per load batch of k_vyz_wave (8: slower)
 
 // Inclusive prefix sum over the 64 lanes of a wavefront with DPP lane
 // moves: Kogge-Stone within each row of 16 lanes (row_shr 1, 2, 4, 8),
@@ -938,463 +883,6 @@ __device__ __forceinline__ T wave_incl_scan(T v) {
     v += dpp_move<0x142, 0xa, false>(v);     // row_bcast:15
     v += dpp_move<0x143, 0xc, false>(v);     // row_bcast:31
     return v;
-}
-
-// vxr: tile of VXR_TJ x VXR_TI refined columns, x processed in chunks of 64
-// refined points (one per lane); xcmax/cjmax/cimax bound the coarse block.
-// RT: storage and arithmetic type of the transfer (double or float).  The
-// tile's coarse column offsets and its y / z stencils are staged in LDS once.
-template <typename RT>
-__device__ __forceinline__ void vxr_tile(const KP &p, int xcmax, int cjmax, int cimax) {
-    extern __shared__ __align__(16) unsigned char smraw[];
-    __shared__ long long coff[16 * 16];                 // coarse column offsets [ci][cj] (cimax, cjmax <= 16)
-    // per coarse x of the chunk: the row of its difference and the metric
-    // with the wall-ghost sign (0 outside -1..nx+1)
-    __shared__ int krow[128];
-    __shared__ double kfac[128];
-    __shared__ RT yw[VXR_TJ][4], zw[VXR_TI][4];
-    __shared__ int yo[VXR_TJ], zo[VXR_TI];
-    RT *sm = reinterpret_cast<RT *>(smraw);
-    RT *vxr = sel<RT>(p.vxr, p.vxrf);
-    const RT *xs_w = sel<RT>(p.xs_w, p.xs_wf), *ys_w = sel<RT>(p.ys_w, p.ys_wf), *zs_w = sel<RT>(p.zs_w, p.zs_wf);
-    const RT *lxa = sel<RT>(p.lxa, p.lxaf);
-    int tj0, ti0;
-    if (!tile_yz_grouped((p.nyr + VXR_TJ - 1) / VXR_TJ, (p.nzr + VXR_TI - 1) / VXR_TI, tj0, ti0)) return;
-    const int J0 = tj0 * VXR_TJ, I0 = ti0 * VXR_TI;
-    const int nj = min(VXR_TJ, p.nyr - J0), ni = min(VXR_TI, p.nzr - I0);
-    const int cj0 = p.ys_src[J0] - 1, CJ = p.ys_src[J0 + nj - 1] - 1 + 4 - cj0;
-    const int ci0 = p.zs_src[I0] - 1, CI = p.zs_src[I0 + ni - 1] - 1 + 4 - ci0;
-    RT *B = sm;                                       // [ci][cj][xc]
-    RT *Z = B + xcmax * cjmax * cimax;                // [ti][cj][xc]
-    RT *Q = Z + xcmax * cjmax * VXR_TI;               // [ti][tj][xc]
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    for (int q = t; q < CI * CJ; q += 256) {
-        const int c = q / CJ, b = q - c * CJ;
-        coff[c * CJ + b] = (long long)wrapf(ci0 + c, p.nz) * p.plane + (long long)wrapf(cj0 + b, p.ny) * p.ldx;
-    }
-    if (t < nj) {
-        yo[t] = p.ys_src[J0 + t] - 1 - cj0;
-        for (int a = 0; a < 4; ++a) yw[t][a] = ys_w[4 * (J0 + t) + a];
-    }
-    if (t < ni) {
-        zo[t] = p.zs_src[I0 + t] - 1 - ci0;
-        for (int a = 0; a < 4; ++a) zw[t][a] = zs_w[4 * (I0 + t) + a];
-    }
-    for (int q = t; q < nj * ni; q += 256) {
-        const int ti = q / nj, tj = q - ti * nj;
-        vxr[ridx(p, 0, J0 + tj, I0 + ti)] = RT(0);      // vxr(1) = 0
-    }
-    // running sums of the columns (ti, wave + 4u) this wavefront writes,
-    // carried from one x chunk to the next
-    RT run[VXR_TI][VXR_TJ / 4];
-#pragma unroll
-    for (int ti = 0; ti < VXR_TI; ++ti)
-#pragma unroll
-        for (int u = 0; u < VXR_TJ / 4; ++u) run[ti][u] = RT(0);
-    const int sS = 1 - 2 * p.inslws, sN = 1 - 2 * p.inslwn;
-    for (int R0 = 0; R0 < p.nxmr; R0 += 64) {
-        const int R1 = min(R0 + 64, p.nxmr);
-        const int x0 = p.xs_src[R0], XC = p.xs_src[R1 - 1] + 4 - x0;
-        __syncthreads();
-        for (int xo = t; xo < XC; xo += 256) {
-            const int xc = x0 + xo;
-            const bool ok = xc >= 0 && xc <= p.nx;
-            const int k = !ok ? 0 : (xc == 0 ? 0 : (xc == p.nx ? p.nxm - 1 : xc - 1));
-            krow[xo] = k;
-            kfac[xo] = !ok ? 0.0 : (xc == 0 ? sS * p.udx3m[k] : (xc == p.nx ? sN * p.udx3m[k] : p.udx3m[k]));
-        }
-        __syncthreads();
-        {
-            // coarse gradient dvx/dx at reference x index xc with the wall
-            // ghosts (InterpVelMgrd.F90:37-51); zero outside -1..nx+1
-            // (kfac = sign * udx3m: the sign is +-1, so the product is
-            // exactly the signed difference quotient).  The loads of VXR_BU
-            // items are issued before any is used: an item outside the block
-            // reads a valid address.
-            const int nB = XC * CJ * CI;
-            Walk3 w(t, 256, XC, CJ);
-            for (int q0 = t; q0 < nB; q0 += 256 * VXR_BU) {
-                double a0[VXR_BU], a1[VXR_BU], f[VXR_BU];
-                int dst[VXR_BU];
-#pragma unroll
-                for (int r = 0; r < VXR_BU; ++r) {
-                    const bool live = q0 + 256 * r < nB;
-                    const int xo = live ? w.a : 0;
-                    const int k = krow[xo];
-                    f[r] = kfac[xo];
-                    const double *col = p.vx + coff[min(w.c, CI - 1) * CJ + min(w.b, CJ - 1)];
-                    a0[r] = col[k]; a1[r] = col[k + 1];
-                    dst[r] = live ? ix3(w.c, cjmax, w.b, xcmax, w.a) : -1;
-                    w.next();
-                }
-#pragma unroll
-                for (int r = 0; r < VXR_BU; ++r)
-                    if (dst[r] >= 0) B[dst[r]] = RT(f[r] * (a1[r] - a0[r]));
-            }
-        }
-        __syncthreads();
-        Walk3 wz(t, 256, XC, CJ);
-        for (int q = t; q < XC * CJ * ni; q += 256, wz.next()) {
-            const int xc = wz.a, cj = wz.b, ti = wz.c;
-            const RT *b = B + ix3(zo[ti], cjmax, cj, xcmax, xc);
-            const int st = __mul24(cjmax, xcmax);
-            Z[ix3(ti, cjmax, cj, xcmax, xc)] = b[0] * zw[ti][0] + b[st] * zw[ti][1] + b[2 * st] * zw[ti][2] + b[3 * st] * zw[ti][3];
-        }
-        __syncthreads();
-        Walk3 wy(t, 256, XC, nj);
-        for (int q = t; q < XC * nj * ni; q += 256, wy.next()) {
-            const int xc = wy.a, tj = wy.b, ti = wy.c;
-            const RT *z = Z + ix3(ti, cjmax, yo[tj], xcmax, xc);
-            Q[ix3(ti, VXR_TJ, tj, xcmax, xc)] = z[0] * yw[tj][0] + z[xcmax] * yw[tj][1] + z[2 * xcmax] * yw[tj][2] + z[3 * xcmax] * yw[tj][3];
-        }
-        __syncthreads();
-        const int kr = R0 + lane;
-        const bool in = kr < R1;
-        int xa = 0;
-        RT wx0 = 0, wx1 = 0, wx2 = 0, wx3 = 0, lx = 0;
-        if (in) {
-            xa = p.xs_src[kr] - x0;
-            wx0 = xs_w[4 * kr]; wx1 = xs_w[4 * kr + 1]; wx2 = xs_w[4 * kr + 2]; wx3 = xs_w[4 * kr + 3];
-            lx = lxa[kr];
-        }
-#pragma unroll
-        for (int ti = 0; ti < VXR_TI; ++ti) {
-            if (ti >= ni) break;
-            RT *orow = vxr + (long long)(I0 + ti) * p.planer + (long long)J0 * p.ldxr + kr + 1;
-#pragma unroll
-            for (int u = 0; u < VXR_TJ / 4; ++u) {
-                const int tj = wave + 4 * u;
-                if (tj >= nj) break;
-                const RT *qq = Q + ix3(ti, VXR_TJ, tj, xcmax, xa);
-                RT v = in ? (qq[0] * wx0 + qq[1] * wx1 + qq[2] * wx2 + qq[3] * wx3) * lx : RT(0);
-                v = wave_incl_scan(v);
-                const RT base = run[ti][u];
-                if (in) orow[(long long)tj * p.ldxr] = base + v;
-                run[ti][u] = base + wave_lane63(v);
-            }
-        }
-    }
-}
-
-template <typename RT>
-__global__ void __launch_bounds__(256) k_vxr_tile(KP p, int xcmax, int cjmax, int cimax) { vxr_tile<RT>(p, xcmax, cjmax, cimax); }
-// FP32: 96 registers leave room for the 5 workgroups per CU its LDS allows
-template <>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) k_vxr_tile<float>(KP p, int xcmax, int cjmax, int cimax) {
-    vxr_tile<float>(p, xcmax, cjmax, cimax);
-}
-
-// vyr (AX = 1) / vzr (AX = 2): lanes = 64 refined x, waves = VYZ_LINES lines
-// of the other periodic axis; the scan axis is walked in chunks of VYZ_CHUNK.
-// Per chunk: B = coarse gradient block [xc][cs][co], O = contraction over the
-// other axis [xc][cs][line], X = contraction over x [cs][line][lane], then a
-// running sum along the scan axis in registers.
-template <int AX, typename RT>
-__global__ void __launch_bounds__(256) k_vyz_tile(KP p, int xcmax, int csmax, int comax) {
-    extern __shared__ __align__(16) unsigned char smraw[];
-    RT *sm = reinterpret_cast<RT *>(smraw);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, t = threadIdx.x;
-    const int nS = AX == 1 ? p.nyr : p.nzr, nO = AX == 1 ? p.nzr : p.nyr;          // refined extents
-    const int cS = AX == 1 ? p.ny : p.nz, cO = AX == 1 ? p.nz : p.ny;              // coarse extents
-    const int *sS = AX == 1 ? p.ys_src : p.zs_src, *sO = AX == 1 ? p.zs_src : p.ys_src;
-    const RT *ysw = sel<RT>(p.ys_w, p.ys_wf), *zsw = sel<RT>(p.zs_w, p.zs_wf), *xs_w = sel<RT>(p.xs_w, p.xs_wf);
-    const RT *wS = AX == 1 ? ysw : zsw, *wO = AX == 1 ? zsw : ysw;
-    const int R0 = blockIdx.x * 64, R1 = min(R0 + 64, p.nxmr);
-    const int O0 = blockIdx.y * VYZ_LINES, nl = min(VYZ_LINES, nO - O0);
-    const int kr = R0 + lane, line = O0 + wave;
-    const bool live = wave < nl;
-    RT *outp = AX == 1 ? sel<RT>(p.vyr, p.vyrf) : sel<RT>(p.vzr, p.vzrf);
-    const long long sstride = AX == 1 ? (long long)p.ldxr : p.planer;
-    const long long obase = AX == 1 ? (long long)line * p.planer : (long long)line * p.ldxr;
-    // the unused x index nxr of vyr / vzr stays zero (InterpVelMgrd.F90:29-31)
-    if (blockIdx.x == gridDim.x - 1 && lane == 0 && live)
-        for (int s = 0; s < nS; ++s) outp[obase + s * sstride + p.nxmr] = RT(0);
-    const int x0 = p.xs_src[R0], XC = p.xs_src[R1 - 1] + 4 - x0;
-    const int co0 = sO[O0] - 1, CO = sO[O0 + nl - 1] - 1 + 4 - co0;
-    RT wx[4] = {0, 0, 0, 0}, wo[4] = {0, 0, 0, 0};
-    int xa = 0, oa = 0;
-    if (kr < R1) { xa = p.xs_src[kr] - x0; for (int a = 0; a < 4; ++a) wx[a] = xs_w[4 * kr + a]; }
-    if (live) { oa = sO[line] - 1 - co0; for (int a = 0; a < 4; ++a) wo[a] = wO[4 * line + a]; }
-    // first guess on the plane s = 0 (InterpVelMgrd.F90:93-123 / :179-209):
-    // velocity plane with wall ghosts, contracted over the other axis, then x
-    RT v = RT(0);
-    if (live && kr < R1 && (AX == 1 || p.nz > 1)) {
-        const int sSg = 1 - 2 * p.inslws, sNg = 1 - 2 * p.inslwn;
-        for (int a = 0; a < 4; ++a) {
-            const int kc = x0 + xa + a;
-            RT q1 = RT(0);
-            for (int c = 0; c < 4; ++c) {
-                const int o = wrapn(co0 + oa + c, cO);
-                const double *col = AX == 1 ? p.vy + (long long)o * p.plane : p.vz + (long long)o * p.ldx;
-                RT f;
-                if (kc >= 1 && kc <= p.nxm) f = RT(col[kc - 1]);
-                else if (kc == 0) f = RT(sSg * col[0]);
-                else if (kc == p.nx) f = RT(sNg * col[p.nxm - 1]);
-                else f = RT(0);
-                q1 = c == 0 ? f * wo[0] : q1 + f * wo[c];
-            }
-            v = a == 0 ? q1 * wx[0] : v + q1 * wx[a];
-        }
-    }
-    if (live && kr < R1) outp[obase + kr] = v;
-    const RT dl = AX == 1 ? RT(1.0 / p.dyr) : RT(1.0 / p.dzr);
-    RT *B = sm;                                               // [co][cs][xc]
-    RT *X = B;                                                // [cs][line][lane], reuses B
-    RT *O = B + max(xcmax * csmax * comax, csmax * VYZ_LINES * 64);   // [line][cs][xc]
-    // coarse offsets of the tile: the other axis (fixed) and, per chunk, the
-    // scan axis and its periodic successor; the lines' stencils
-    __shared__ long long ooff[32], soff[32], snext[32];
-    __shared__ RT lw[VYZ_LINES][4];
-    __shared__ int lo[VYZ_LINES];
-    const long long ostride = AX == 1 ? p.plane : (long long)p.ldx, sstr = AX == 1 ? (long long)p.ldx : p.plane;
-    for (int q = t; q < CO; q += 256) ooff[q] = (long long)wrapf(co0 + q, cO) * ostride;
-    if (t < nl) {
-        lo[t] = sO[O0 + t] - 1 - co0;
-        for (int a = 0; a < 4; ++a) lw[t][a] = wO[4 * (O0 + t) + a];
-    }
-    const double *vel = AX == 1 ? p.vy : p.vz;
-    const double dgrid = AX == 1 ? p.dy : p.dz;
-    const int sSg = 1 - 2 * p.inslws, sNg = 1 - 2 * p.inslwn;
-    for (int S0 = 0; S0 < nS - 1; S0 += VYZ_CHUNK) {
-        const int S1 = min(S0 + VYZ_CHUNK, nS - 1);
-        const int cs0 = sS[S0] - 1, CS = sS[S1 - 1] - 1 + 4 - cs0;
-        __syncthreads();
-        for (int q = t; q < CS; q += 256) {
-            const int js = wrapf(cs0 + q, cS);
-            soff[q] = (long long)js * sstr;
-            snext[q] = (long long)wrapp(js, cS) * sstr;
-        }
-        __syncthreads();
-        {
-            // coarse gradient d(vy)/dy or d(vz)/dz at reference x index xc
-            // with the wall ghosts (InterpVelMgrd.F90:75-86, :161-172)
-            // (loads of VYZ_BU items issued before any is used; an item
-            // outside the block or the grid reads a valid address)
-            const int nB = XC * CS * CO;
-            Walk3 w(t, 256, XC, CS);
-            for (int q0 = t; q0 < nB; q0 += 256 * VYZ_BU) {
-                double a0[VYZ_BU], a1[VYZ_BU];
-                int dst[VYZ_BU], xs[VYZ_BU];
-#pragma unroll
-                for (int r = 0; r < VYZ_BU; ++r) {
-                    const int xc = x0 + w.a;
-                    const bool live = q0 + 256 * r < nB, ok = live && xc >= 0 && xc <= p.nx;
-                    const int k = !ok ? 0 : (xc == 0 ? 0 : (xc == p.nx ? p.nxm - 1 : xc - 1));
-                    const int c = min(w.c, CO - 1), b = min(w.b, CS - 1);
-                    const double *cb = vel + (ok ? ooff[c] : 0) + k;
-                    a1[r] = cb[ok ? snext[b] : 0];
-                    a0[r] = cb[ok ? soff[b] : 0];
-                    dst[r] = live ? ix3(w.c, csmax, w.b, xcmax, w.a) : -1;
-                    xs[r] = ok ? xc : -1;
-                    w.next();
-                }
-#pragma unroll
-                for (int r = 0; r < VYZ_BU; ++r)
-                    if (dst[r] >= 0) {
-                        const int xc = xs[r];
-                        const double d = (a1[r] - a0[r]) * dgrid;
-                        B[dst[r]] = xc < 0 ? RT(0) : RT(xc == 0 ? sSg * d : (xc == p.nx ? sNg * d : d));
-                    }
-            }
-        }
-        __syncthreads();
-        // contraction over the other axis: one (cs, xc) per item, all lines
-        {
-            const int st = __mul24(csmax, xcmax);
-            Walk3 wo(t, 256, XC, CS);
-            for (int q = t; q < XC * CS; q += 256, wo.next()) {
-                const int base = __mul24(wo.b, xcmax) + wo.a;
-#pragma unroll
-                for (int l = 0; l < VYZ_LINES; ++l)
-                    if (l < nl) {
-                        const RT *b = B + __mul24(lo[l], st) + base;
-                        O[__mul24(l, st) + base] = b[0] * lw[l][0] + b[st] * lw[l][1] + b[2 * st] * lw[l][2] + b[3 * st] * lw[l][3];
-                    }
-            }
-        }
-        __syncthreads();
-        if (live && kr < R1)
-            for (int cs = 0; cs < CS; ++cs) {
-                const RT *o = O + ix3(wave, csmax, cs, xcmax, xa);
-                X[(cs * VYZ_LINES + wave) * 64 + lane] = o[0] * wx[0] + o[1] * wx[1] + o[2] * wx[2] + o[3] * wx[3];
-            }
-        __syncthreads();
-        if (live && kr < R1)
-            for (int s = S0; s < S1; ++s) {
-                const int b0 = sS[s] - 1 - cs0;
-                const RT *w = wS + 4 * s, *xx = X + (b0 * VYZ_LINES + wave) * 64 + lane;
-                const int st = VYZ_LINES * 64;
-                const RT tv = xx[0] * w[0] + xx[st] * w[1] + xx[2 * st] * w[2] + xx[3 * st] * w[3];
-                v = v + tv * dl;
-                outp[obase + (s + 1) * sstride + kr] = v;
-            }
-    }
-}
-
-// vyr (AX = 1) / vzr (AX = 2) with one wavefront per refined line of the
-// other periodic axis and no LDS: lanes = 64 refined x, the scan axis walked
-// point by point (InterpVelMgrd.F90:68-237).  Per coarse scan index cs the
-// wavefront forms, for each coarse x of its chunk (one per lane; a second
-// register when the chunk spans more than 64 coarse points), P(xc) = sum_c
-// wo_c G(xc, cs, o_c), the coarse gradient G with the wall ghosts contracted
-// over the other axis; then X(kr) = sum_a wx_a P(xa + a) by lane shuffles.
-// The last four X stay in registers for the scan-axis stencil of each
-// refined point, and the velocity row of plane cs + 1 is carried to the
-// next step, so a step loads one row per o_c.  The arithmetic is that of
-// k_vyz_tile term by term.  Workgroups of 4 wavefronts take 4 consecutive
-// lines of one x chunk; consecutive workgroups on an XCD take consecutive
-// line groups (shared coarse rows in its L2).
-// (FP32: at least 6 wavefronts per SIMD, 71 VGPRs, which make 7; FP64 keeps
-// its 94 VGPRs, since the 80 that 6 wavefronts allow spill and cost 30% on a
-// 768 x 1536^2 refined grid; 8 wavefronts spill in FP32 too)
-template <int AX, typename RT, bool TWO>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(RT) == 4 ? 6 : 1, 8))) k_vyz_wave(KP p, int nxchunk) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int nS = AX == 1 ? p.nyr : p.nzr, nO = AX == 1 ? p.nzr : p.nyr;          // refined extents
-    const int cS = AX == 1 ? p.ny : p.nz, cO = AX == 1 ? p.nz : p.ny;              // coarse extents
-    const int *sS = AX == 1 ? p.ys_src : p.zs_src, *sO = AX == 1 ? p.zs_src : p.ys_src;
-    const RT *ysw = sel<RT>(p.ys_w, p.ys_wf), *zsw = sel<RT>(p.zs_w, p.zs_wf), *xs_w = sel<RT>(p.xs_w, p.xs_wf);
-    const RT *wS = AX == 1 ? ysw : zsw, *wO = AX == 1 ? zsw : ysw;
-    const int ngroups = (nO + 3) / 4;
-    const long long blk = xcd_block(0);
-    if (blk >= (long long)nxchunk * ngroups) return;
-    const int xchunk = int(blk / ngroups), line = int(blk % ngroups) * 4 + wave;
-    if (line >= nO) return;
-    const int R0 = xchunk * 64, R1 = min(R0 + 64, p.nxmr);
-    const int kr = R0 + lane;
-    const bool in = kr < R1;
-    RT *outp = AX == 1 ? sel<RT>(p.vyr, p.vyrf) : sel<RT>(p.vzr, p.vzrf);
-    const long long sstride = AX == 1 ? (long long)p.ldxr : p.planer;
-    const long long obase = AX == 1 ? (long long)line * p.planer : (long long)line * p.ldxr;
-    // the unused x index nxr of vyr / vzr stays zero (InterpVelMgrd.F90:29-31)
-    if (xchunk == nxchunk - 1 && lane == 0)
-        for (int s = 0; s < nS; ++s) outp[obase + s * sstride + p.nxmr] = RT(0);
-    const int x0 = p.xs_src[R0];
-    RT wx[4] = {0, 0, 0, 0};
-    int xa = 0;
-    if (in) { xa = p.xs_src[kr] - x0; for (int a = 0; a < 4; ++a) wx[a] = xs_w[4 * kr + a]; }
-    // the line's stencil over the other axis (wavefront-uniform)
-    const long long ostride = AX == 1 ? p.plane : (long long)p.ldx, sstr = AX == 1 ? (long long)p.ldx : p.plane;
-    const int o0 = sO[line] - 1;
-    RT wo[4];
-    long long ooff[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) { wo[c] = wO[4 * line + c]; ooff[c] = (long long)wrapn(o0 + c, cO) * ostride; }
-    const int sSg = 1 - 2 * p.inslws, sNg = 1 - 2 * p.inslwn;
-    const double *vel = AX == 1 ? p.vy : p.vz;
-    // first guess on the plane s = 0 (InterpVelMgrd.F90:93-123 / :179-209):
-    // velocity plane with wall ghosts, contracted over the other axis, then x
-    RT v = RT(0);
-    if (in && (AX == 1 || p.nz > 1)) {
-        for (int a = 0; a < 4; ++a) {
-            const int kc = x0 + xa + a;
-            RT q1 = RT(0);
-            for (int c = 0; c < 4; ++c) {
-                const double *col = vel + ooff[c];
-                RT f;
-                if (kc >= 1 && kc <= p.nxm) f = RT(col[kc - 1]);
-                else if (kc == 0) f = RT(sSg * col[0]);
-                else if (kc == p.nx) f = RT(sNg * col[p.nxm - 1]);
-                else f = RT(0);
-                q1 = c == 0 ? f * wo[0] : q1 + f * wo[c];
-            }
-            v = a == 0 ? q1 * wx[0] : v + q1 * wx[a];
-        }
-    }
-    if (in) outp[obase + kr] = v;
-    if (nS < 2) return;
-    // this lane's coarse x rows (xc = x0 + lane, and + 64): row, ghost sign
-    // (0 outside -1..nx+1 reads row 0)
-    auto xrow = [&](int xc, int &k, double &sg) {
-        const bool ok = xc >= 0 && xc <= p.nx;
-        k = !ok ? 0 : (xc == 0 ? 0 : (xc == p.nx ? p.nxm - 1 : xc - 1));
-        sg = !ok ? 0.0 : (xc == 0 ? double(sSg) : (xc == p.nx ? double(sNg) : 1.0));
-    };
-    // lanes past the chunk's XC coarse points are never gathered: they take
-    // the last point's row, so their loads stay on cache lines in use
-    const int XC = p.xs_src[R1 - 1] + 4 - x0;
-    int k0, k1;
-    double g0, g1;
-    xrow(x0 + min(lane, XC - 1), k0, g0);
-    xrow(x0 + min(64 + lane, XC - 1), k1, g1);
-    const double dgrid = AX == 1 ? p.dy : p.dz;
-    const RT dl = AX == 1 ? RT(1.0 / p.dyr) : RT(1.0 / p.dzr);
-    int cs = sS[0] - 1;                       // unwrapped coarse scan index of the next X
-    double va[4], vb[4];                      // velocity rows of plane cs (second register: vb)
-    {
-        const long long pl = (long long)wrapf(cs, cS) * sstr;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) { va[c] = vel[ooff[c] + pl + k0]; vb[c] = TWO ? vel[ooff[c] + pl + k1] : 0.0; }
-    }
-    // X at the VYZ_NB coarse indices cs .. cs + VYZ_NB - 1 into W[3 ..]; the
-    // rows of all VYZ_NB planes are loaded before any is used, so a wavefront
-    // keeps 4 VYZ_NB loads in flight instead of waiting on each plane
-    RT W[VYZ_NB + 3];
-    auto batch = [&]() {
-        double na[VYZ_NB][4], nb[VYZ_NB][4];
-#pragma unroll
-        for (int q = 0; q < VYZ_NB; ++q) {
-            const long long pn = (long long)wrapf(cs + 1 + q, cS) * sstr;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                na[q][c] = vel[ooff[c] + pn + k0];
-                nb[q][c] = TWO ? vel[ooff[c] + pn + k1] : 0.0;
-            }
-        }
-#pragma unroll
-        for (int q = 0; q < VYZ_NB; ++q) {
-            RT b[4], b2[4];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const double p0 = q == 0 ? va[c] : na[q - 1][c];
-                b[c] = RT(g0 * ((na[q][c] - p0) * dgrid));
-                if (TWO) {
-                    const double p1 = q == 0 ? vb[c] : nb[q - 1][c];
-                    b2[c] = RT(g1 * ((nb[q][c] - p1) * dgrid));
-                } else {
-                    b2[c] = RT(0);
-                }
-            }
-            const RT P = b[0] * wo[0] + b[1] * wo[1] + b[2] * wo[2] + b[3] * wo[3];
-            const RT P2 = b2[0] * wo[0] + b2[1] * wo[1] + b2[2] * wo[2] + b2[3] * wo[3];
-            RT o[4];
-#pragma unroll
-            for (int a = 0; a < 4; ++a) {
-                const int idx = xa + a;
-                o[a] = __shfl(P, idx & 63, 64);
-                if (TWO) {
-                    const RT o2 = __shfl(P2, idx & 63, 64);
-                    if (idx >= 64) o[a] = o2;
-                }
-            }
-            W[3 + q] = o[0] * wx[0] + o[1] * wx[1] + o[2] * wx[2] + o[3] * wx[3];
-        }
-#pragma unroll
-        for (int c = 0; c < 4; ++c) { va[c] = na[VYZ_NB - 1][c]; vb[c] = nb[VYZ_NB - 1][c]; }
-        cs += VYZ_NB;
-    };
-    // W[0 .. nv-1] hold X at coarse indices lo .. lo + nv - 1; the window of
-    // the refined point s is W[0 .. 3] once lo has reached its first source
-    batch();
-#pragma unroll
-    for (int q = 0; q < 3; ++q) W[q] = W[3 + q];
-#pragma unroll
-    for (int q = 3; q < VYZ_NB; ++q) W[q] = W[3 + q];
-    int lo = sS[0] - 1, nv = VYZ_NB;
-#pragma unroll 1
-    for (int s = 0; s < nS - 1; ++s) {
-        const int b0 = sS[s] - 1;
-        while (lo < b0) {
-#pragma unroll
-            for (int q = 0; q < VYZ_NB + 2; ++q) W[q] = W[q + 1];
-            ++lo;
-            if (--nv == 3) { batch(); nv += VYZ_NB; }
-        }
-        const RT *w = wS + 4 * s;
-        const RT tv = W[0] * w[0] + W[1] * w[1] + W[2] * w[2] + W[3] * w[3];
-        v = v + tv * dl;
-        if (in) outp[obase + (s + 1) * sstride + kr] = v;
-    }
 }
 
 // Refined -> coarse cell centres through the fast coarse-grid loop of

@@ -51,7 +51,7 @@ struct KP {
     double *rux, *ruy, *ruz, *rut;
     double *qcap, *dph, *dq, *hro;
     double *rhsx, *rhsy, *rhsz, *rhst;
-    double *salc, *tpdv;
+    double *salc;
     const double *tempbp, *temptp;      // [nz][ny]
     // refined fields
     double *sal, *rusal, *hsal, *rhsr, *vxr, *vyr, *vzr;

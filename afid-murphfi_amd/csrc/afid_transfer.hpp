@@ -1,0 +1,323 @@
+// afid_transfer.hpp -- coarse -> refined transfers: InterpVelMgrd
+// (InterpVelMgrd.F90:11-237) and InterpTempMultigrid (phasefield.F90:498-520).
+//
+// Every transfer is a product of one-dimensional 4-point Hermite stencils, so
+// the axes can be taken one after the other.
+//   k_xfer_x   per coarse column: the coarse gradient (or T) with its wall
+//              ghosts, the x stencil, and for vx the sum along x; one row of
+//              refined x per coarse column goes to a scratch array.
+//   k_xfer_yz  per refined line of one periodic axis, or pair of adjacent
+//              ones: walks the other axis, contracts the rows of the 4 (pair:
+//              5) coarse lines it reads, keeps the last four in registers for
+//              the stencil along the walk, and for vyr / vzr carries the sum
+//              along it.
+// The x stencil, the only one that crosses lanes, so runs on the coarse columns
+// alone (a quarter of the refined ones at ratio 2), and the second kernel is
+// whole aligned 16-byte rows of refined x: loads, multiply-adds, stores.
+//
+// What bounds it: bytes, with the scratch 13 B per refined cell at ratio 2 in
+// FP64 (7 in FP32) of which 9 (5) are needed.  Forms that did all three axes
+// per tile in LDS or per refined line with lane shuffles were bound by integer
+// and lane instructions and by 8-byte loads of mostly clamped lanes; figures of
+// both at interp_vel().
+#pragma once
+#include <hip/hip_runtime.h>
+#include "afid_params.hpp"
+#include "afid_stencils.hpp"
+#include "afid_kernels.hpp"
+#include "afid_column.hpp"
+#include <type_traits>
+
+namespace afid {
+
+enum XferField { XF_VX = 0, XF_VY = 1, XF_VZ = 2, XF_T = 3 };
+
+// read-only table behind a uniform index: scalar loads
+template <typename T>
+using ConstTab = const __attribute__((address_space(4))) T *;
+template <typename T>
+__device__ __forceinline__ ConstTab<T> const_tab(const T *q) { return (ConstTab<T>)(unsigned long long)q; }
+
+template <typename RT, int NR> struct XVec { typedef RT V __attribute__((ext_vector_type(NR))); };
+
+// x part of the transfer of field FLD: D[i][j][kr] (row stride ldxr) for every
+// coarse column; for vy / vz also F, the x-transferred velocity of the first
+// plane along the field's own axis ([i] for vy, [j] for vz), the start of the
+// sums (InterpVelMgrd.F90:93-123, :179-209).  One wavefront per column, walking
+// columns with the next one's values already on their way; the coarse values
+// of a column (reference x index -1 .. nx+1, wall ghosts InterpVelMgrd.F90:37-51,
+// phasefield.F90:502-512) go through LDS to the lanes' refined points (CHR per
+// lane), whose weights the workgroup keeps in LDS.
+// (CHR * 64 covers the base rows too.)
+constexpr int XFX_WAVES = 8;                // at most
+template <int CHR, typename RT, int FLD>
+__global__ void __launch_bounds__(64 * XFX_WAVES) k_xfer_x(KP p, RT *D, RT *F) {
+    using V4 = typename XVec<RT, 4>::V;
+    extern __shared__ __align__(16) unsigned char smraw[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    const int nxm = p.nxm, nxmr = p.nxmr, len = nxm + 4;
+    V4 *wt = reinterpret_cast<V4 *>(smraw);                     // [refined x] the 4 weights
+    RT *buf = reinterpret_cast<RT *>(wt + 64 * CHR) + wave * len;       // reference x index xc at buf[xc + 1]
+    const RT *xs_w = sel<RT>(p.xs_w, p.xs_wf), *lxa = sel<RT>(p.lxa, p.lxaf);
+    for (int k = threadIdx.x; k < 64 * CHR; k += blockDim.x)
+        for (int a = 0; a < 4; ++a) reinterpret_cast<RT *>(wt)[4 * k + a] = k < nxmr ? xs_w[4 * k + a] : RT(0);
+    RT lx[CHR];
+    int xa[CHR];
+#pragma unroll
+    for (int m = 0; m < CHR; ++m) {
+        const int k = lane + 64 * m;
+        xa[m] = k < nxmr ? p.xs_src[k] + 1 : 0;
+        lx[m] = FLD == XF_VX && k < nxmr ? lxa[k] : RT(0);
+    }
+    if (lane == 0) { buf[0] = RT(0); buf[len - 1] = RT(0); }
+    __syncthreads();
+    const double sS = 1 - 2 * p.inslws, sN = 1 - 2 * p.inslwn;
+    const long long ncol = (long long)p.ny * p.nz, nw = (long long)gridDim.x * waves;
+    const double *f = FLD == XF_VX ? p.vx : FLD == XF_VY ? p.vy : FLD == XF_VZ ? p.vz : p.temp;
+    double va[CHR], vb[CHR];                                    // rows k of the column and of its successor (vx: rows k + 1)
+    auto fetch = [&](long long col) {
+        const int i = int(col / p.ny), j = int(col - (long long)i * p.ny);
+        const double *a = f + (long long)i * p.plane + (long long)j * p.ldx;
+        const double *b = FLD == XF_VY ? f + (long long)i * p.plane + (long long)wrapp(j, p.ny) * p.ldx
+                        : FLD == XF_VZ ? f + (long long)wrapp(i, p.nz) * p.plane + (long long)j * p.ldx : a + 1;
+#pragma unroll
+        for (int m = 0; m < CHR; ++m) {
+            if (64 * m >= nxm) break;
+            const int k = min(lane + 64 * m, nxm - 1);
+            va[m] = a[k];
+            if (FLD != XF_T) vb[m] = b[k];
+        }
+    };
+    auto sync = [] {                                            // LDS of one wavefront
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    long long col = (long long)xcd_block(0) * waves + wave;
+    if (col < ncol) fetch(col);
+    for (; col < ncol; col += nw) {
+        const int i = int(col / p.ny), j = int(col - (long long)i * p.ny);
+        const bool first = (FLD == XF_VY && j == 0) || (FLD == XF_VZ && i == 0);
+        double tbp = 0.0, ttp = 0.0;
+        if (FLD == XF_T) { tbp = p.tempbp[col]; ttp = p.temptp[col]; }
+        for (int pass = first ? 1 : 0; pass >= 0; --pass) {
+            // pass 0: the gradient (T itself); pass 1: the velocity of the first plane
+#pragma unroll
+            for (int m = 0; m < CHR; ++m) {
+                const int k = lane + 64 * m;
+                if (64 * m >= nxm) break;
+                double v = va[m];
+                if (FLD == XF_VX) v = (vb[m] - v) * p.udx3m[min(k, nxm - 1)];
+                else if (FLD != XF_T && !pass) v = (vb[m] - v) * (FLD == XF_VY ? p.dy : p.dz);
+                if (k < nxm) {
+                    buf[k + 2] = RT(v);
+                    if (k == 0) buf[1] = FLD == XF_T ? RT((1.0 - 2.0 * p.tfixs) * v + 2.0 * p.tfixs * tbp) : RT(sS * v);
+                    if (k == nxm - 1) buf[nxm + 2] = FLD == XF_T ? RT((1.0 - 2.0 * p.tfixn) * v + 2.0 * p.tfixn * ttp) : RT(sN * v);
+                }
+            }
+            if (!pass && col + nw < ncol) fetch(col + nw);
+            sync();
+            RT *o = pass ? F + (long long)(FLD == XF_VY ? i : j) * p.ldxr : D + col * p.ldxr;
+            RT run = RT(0);
+#pragma unroll
+            for (int m = 0; m < CHR; ++m) {
+                const RT *t = buf + xa[m];
+                const V4 w = wt[lane + 64 * m];
+                RT v = t[0] * w[0] + t[1] * w[1] + t[2] * w[2] + t[3] * w[3];
+                if (FLD == XF_VX) {       // vxr at the face above refined cell k
+                    v = run + wave_incl_scan(v * lx[m]);
+                    run = wave_lane63(v);
+                }
+                // (zeros just past the last point: whole vectors of the second kernel)
+                const int k = lane + 64 * m;
+                if (FLD == XF_VX) { if (k < nxmr) o[k + 1] = v; }
+                else if (k < min(nxmr + 3, p.ldxr)) o[k] = v;
+            }
+            if (FLD == XF_VX && lane == 0) o[0] = RT(0);        // vxr(1) = 0
+            sync();
+        }
+    }
+}
+
+// the y / z part of one transfer
+struct XferJob {
+    const void *D, *F;              // rows of k_xfer_x (F: null for vxr and T)
+    void *out;                      // refined field
+    const int *s_src, *o_src;       // Hermite sources along the walked (s) and the other (o) axis
+    const void *s_w, *o_w;          // weights (RT)
+    int nS, nO, cS, cO;             // refined and coarse extents
+    long long ds, dq;               // D strides of a coarse step along s and o
+    long long rs, ro;               // out strides of a refined step along s and o
+    int nx, ld;                     // refined x points, row stride
+    int two;                        // the refined steps come two by two: sources s_src[s] = s_src[1] + (s - 1) / 2
+    double dl;                      // refined spacing along s
+    int nseg;                       // wavefronts that share one walk
+};
+// value of lane k (uniform) in every lane
+__device__ __forceinline__ float lane_value(float v, int k) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), k));
+}
+__device__ __forceinline__ double lane_value(double v, int k) {
+    const long long b = __builtin_bit_cast(long long, v);
+    const int lo = __builtin_amdgcn_readlane(int(b), k), hi = __builtin_amdgcn_readlane(int(b >> 32), k);
+    return __builtin_bit_cast(double, (long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+
+// NL adjacent refined lines per wavefront (their sources span NL + 3 coarse
+// lines), NR refined x per lane.  SUM: the walk carries the sum (vyr, vzr).
+// With nseg > 1 a workgroup's wavefronts share one walk: each takes a range
+// of refined steps; for a sum they first add up their ranges.
+template <typename RT, int NR, int NL, bool SUM, bool SEG>
+__global__ void __launch_bounds__(SEG ? 512 : 256) k_xfer_yz(XferJob jb) {
+    using V = typename XVec<RT, NR>::V;
+    constexpr int NU = NL + 3, PD = 4;                           // coarse lines; coarse steps loaded ahead
+    extern __shared__ __align__(16) unsigned char smraw[];
+    V *tot = reinterpret_cast<V *>(smraw);                       // [seg][line][lane]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nch = (jb.nx + 64 * NR - 1) / (64 * NR), ngr = (jb.nO + NL - 1) / NL;
+    // x chunks fastest: neighbouring wavefronts write one row
+    const int item = SEG ? int(xcd_block(0)) : int(xcd_block(0)) * 4 + wave;
+    const int grp = item / nch, chunk = item - grp * nch, seg = SEG ? wave : 0;
+    if (grp >= ngr) return;                      // whole workgroups where they share a walk
+    const ConstTab<int> sS = const_tab(jb.s_src), sO = const_tab(jb.o_src);
+    const ConstTab<RT> wO = const_tab(static_cast<const RT *>(jb.o_w));
+    const int l0 = grp * NL;
+    const int o0 = sO[l0] - 1;
+    RT w[NL][NU];
+    long long ro[NU];
+#pragma unroll
+    for (int c = 0; c < NU; ++c) ro[c] = (long long)wrapf(o0 + c, jb.cO) * jb.dq;
+#pragma unroll
+    for (int l = 0; l < NL; ++l) {
+        const int ll = min(l0 + l, jb.nO - 1), d = sO[ll] - 1 - o0;
+#pragma unroll
+        for (int c = 0; c < NU; ++c) w[l][c] = c >= d && c < d + 4 ? wO[4 * ll + (c >= d && c < d + 4 ? c - d : 0)] : RT(0);
+    }
+    // lanes past the row repeat its last vector (the same values to the same place)
+    const int x = min((chunk * 64 + lane) * NR, (jb.nx - 1) / NR * NR);
+    const RT *D = static_cast<const RT *>(jb.D);
+    // rows of the lines (an odd last line twice, with the same values)
+    RT *out[NL];
+#pragma unroll
+    for (int l = 0; l < NL; ++l) out[l] = static_cast<RT *>(jb.out) + min(l0 + l, jb.nO - 1) * jb.ro + x;
+    const RT dl = RT(jb.dl);
+    auto put = [&](int s, const V (&v)[NL]) {
+#pragma unroll
+        for (int l = 0; l < NL; ++l) __builtin_nontemporal_store(v[l], reinterpret_cast<V *>(out[l] + s * jb.rs));
+    };
+    const int nt = SUM ? jb.nS - 1 : jb.nS;
+    const int sa = SEG ? int((long long)nt * seg / jb.nseg) : 0, sb = SEG ? int((long long)nt * (seg + 1) / jb.nseg) : nt;
+    V v[NL];
+    // walk of the refined steps sa .. sb - 1
+    auto walk = [&](auto store) {
+        if (sa >= sb) return;
+        int cs = sS[sa] - 1;
+        const int end = sS[sb - 1] + 2;
+        int cw = wrapf(cs, jb.cS);                               // cs on the periodic axis
+        V R[PD][NU], W[4][NL];
+        auto load = [&](V (&r)[NU]) {
+            const RT *q = D + cw * jb.ds;
+#pragma unroll
+            for (int c = 0; c < NU; ++c) r[c] = *reinterpret_cast<const V *>(q + ro[c] + x);
+            if (++cw == jb.cS) cw = 0;
+        };
+#pragma unroll
+        for (int q = 0; q < PD; ++q) load(R[q]);
+        // the stencils of 64 refined steps at a time, one per lane
+        int s = sa, base = sa, tn = 0;
+        RT t0 = RT(0), t1 = RT(0), t2 = RT(0), t3 = RT(0);
+        auto fill = [&]() {
+            base = s;
+            const int k = min(s + lane, sb - 1);
+            tn = s + lane < sb ? jb.s_src[k] + 2 : -1 << 30;
+            const RT *w4 = static_cast<const RT *>(jb.s_w) + 4 * k;
+            t0 = w4[0]; t1 = w4[1]; t2 = w4[2]; t3 = w4[3];
+        };
+        fill();
+        int need = __builtin_amdgcn_readlane(tn, 0);
+        auto contract = [&](int q) {
+#pragma unroll
+            for (int l = 0; l < NL; ++l) {
+                V P = R[q % PD][0] * w[l][0];
+#pragma unroll
+                for (int c = 1; c < NU; ++c) P += R[q % PD][c] * w[l][c];
+                W[q][l] = P;
+            }
+        };
+        auto emit = [&](int q) {
+            const int k = s - base;
+            const RT w0 = lane_value(t0, k), w1 = lane_value(t1, k), w2 = lane_value(t2, k), w3 = lane_value(t3, k);
+            ++s;
+#pragma unroll
+            for (int l = 0; l < NL; ++l) {
+                const V tv = W[(q + 1) & 3][l] * w0 + W[(q + 2) & 3][l] * w1 + W[(q + 3) & 3][l] * w2 + W[q][l] * w3;
+                v[l] = SUM ? v[l] + tv * dl : tv;
+            }
+            if (store) put(SUM ? s : s - 1, v);
+        };
+        for (; cs <= end; cs += 4) {
+            if (jb.two && s + 8 <= sb && need == cs && s > 0 && (s & 1)) {
+                // ratio 2: every coarse step completes the refined steps s
+                // (odd) and s + 1.  Straight-line code, so that a wait for a
+                // row counts the stores issued after it instead of draining them.
+                if (s - base > 56) fill();
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    contract(q);
+                    load(R[q % PD]);
+                    emit(q);
+                    emit(q);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (s - base > 63) fill();
+                need = s < sb ? __builtin_amdgcn_readlane(tn, s - base) : -1 << 30;
+                continue;
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if (cs + q > end) break;
+                contract(q);
+                load(R[q % PD]);
+                while (need == cs + q) {
+                    emit(q);
+                    if (s - base > 63 && s < sb) fill();
+                    need = s < sb ? __builtin_amdgcn_readlane(tn, s - base) : -1 << 30;
+                }
+            }
+        }
+    };
+    if (SUM) {
+        if (SEG) {
+#pragma unroll
+            for (int l = 0; l < NL; ++l) v[l] = V(RT(0));
+            walk(std::false_type{});
+#pragma unroll
+            for (int l = 0; l < NL; ++l) tot[(seg * NL + l) * 64 + lane] = v[l];
+            __syncthreads();
+        }
+        const RT *F = static_cast<const RT *>(jb.F);
+#pragma unroll
+        for (int l = 0; l < NL; ++l) v[l] = V(RT(0));
+        if (F)
+#pragma unroll
+            for (int c = 0; c < NU; ++c) {
+                const V f = *reinterpret_cast<const V *>(F + (long long)wrapf(o0 + c, jb.cO) * jb.ld + x);
+#pragma unroll
+                for (int l = 0; l < NL; ++l) v[l] += f * w[l][c];
+            }
+        if (seg == 0) put(0, v);
+        for (int q = 0; SEG && q < seg; ++q)
+#pragma unroll
+            for (int l = 0; l < NL; ++l) v[l] += tot[(q * NL + l) * 64 + lane];
+    }
+    walk(std::true_type{});
+}
+
+// index nxr of a refined field to zero
+template <typename RT>
+__global__ void __launch_bounds__(256) k_zero_tail(RT *f, int n, int ld, long long rows) {
+    const long long r = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (r < rows) f[r * ld + n] = RT(0);
+}
+
+}  // namespace afid
