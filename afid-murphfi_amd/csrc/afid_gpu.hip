@@ -47,15 +47,15 @@ struct TimerRec {
 
 }  // namespace
 
-// Refined -> coarse tables of one transfer (k_interp_coarse_tile), per axis
+// Refined -> coarse tables of one transfer (k_to_coarse), per axis
 // and coarse index: the first refined source and 4 weights (FP64, and FP32
 // for the mixed form), with the tile's LDS plan.
 struct CoarseTab {
     const int *x_src = nullptr, *y_src = nullptr, *z_src = nullptr;
     const double *x_w = nullptr, *y_w = nullptr, *z_w = nullptr;
     const float *x_wf = nullptr, *y_wf = nullptr, *z_wf = nullptr;
-    int xr = 0, yr = 0;          // largest refined x / y span of a tile
-    size_t lds = 0;
+    int nseg = 1;                // ranges of z
+    bool two = false;            // coarse y lines in pairs two refined lines apart (ratio 2)
     bool general = false;        // interpolate_xyz_to_coarse (refined grid does not bracket)
 };
 
@@ -459,6 +459,32 @@ static int pick_lines(int N, int maxlds, int cap, int maxv = FFT_MAXV) {
     while (2 * L * line_stride<R>(N) * int(sizeof(cpx<R>)) <= maxlds && 2 * L * N <= maxv * FFT_THREADS && 2 * L <= cap)
         L *= 2;
     return L;
+}
+
+// LDS of k_to_coarse: two refined rows of each line
+template <typename RT, int NR, int NL>
+static size_t coarse_lds(int nxmr) { return sizeof(RT) * 2 * NL * size_t((nxmr + 3 * NR - 1) / NR * NR); }
+// Ranges of z of k_to_coarse: each reads 2 to 4 refined planes of its
+// neighbour's, and a last round of workgroups that is nearly empty costs as
+// much as a full one, so the number is the one with the least rounds x planes
+// of a workgroup (+ 4: its start).  us per step with ranges for 1024 / 2048 /
+// 4096 / 6144 wavefronts instead: 384 x 192^2 FP64 806 / 850 / 728 / 863,
+// 256^3 FP32 500 / 423 / 508 / 490; this rule takes the best of both.
+template <typename RT, int NR, int NL>
+static int coarse_ranges(afid_ctx *c) {
+    int per_cu = 0, cus = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_to_coarse<RT, NR, NL>, 64 * ((c->nxmr + 64 * NR - 1) / (64 * NR)),
+                                                     coarse_lds<RT, NR, NL>(c->nxmr)) != hipSuccess || per_cu < 1) per_cu = 1;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || cus < 1) cus = 256;
+    const long long ngr = (c->ny + NL - 1) / NL, slots = (long long)per_cu * cus;
+    int best = 1;
+    double least = 0;
+    for (int n = 1; n <= c->nz; ++n) {
+        const double planes = double(c->nzr) / c->nz * ((c->nz + n - 1) / n - 1) + 4;
+        const double cost = double((ngr * n + slots - 1) / slots) * (planes + 4);
+        if (n == 1 || cost < least) { best = n; least = cost; }
+    }
+    return best;
 }
 
 static int setup(afid_ctx *c) {
@@ -965,17 +991,18 @@ static int setup(afid_ctx *c) {
         return set_err(c, AFID_E_ARG, "refinement ratio too small for the vyr/vzr tiles");
     const auto block_yz = [&](int cs, int co) { return es * size_t(std::max(x64 * cs * co, cs * 4 * 64) + x64 * cs * 4); };
     const size_t most = std::max(es * size_t(x64 * y16 * z4 + x64 * y16 * 4 + x64 * 16 * 4), std::max(block_yz(ys, yo), block_yz(zs, zo)));
-    // refined -> coarse tiles: 64 coarse x by SALC_TJ coarse y, two refined
-    // planes of the tile in LDS (storage type of the refined field)
+    // refined -> coarse: the span of 64 x and 8 y coarse points, two planes in 64 KiB
     for (int q = 0; q < 2; ++q) {
         const HostTab &h = q == 0 ? hs : hp;
         CoarseTab &t = q == 0 ? c->tab_sal : c->tab_phi;
         if ((q == 0 && !c->sal) || (q == 1 && !c->pf)) continue;
-        t.xr = span(h.xs, nxm, 64);
-        t.yr = span(h.ys, c->ny, SALC_TJ);
-        if (t.yr > 64) return set_err(c, AFID_E_ARG, "refinement ratio too large for the refined -> coarse tiles");
-        t.lds = es * size_t(2 * t.yr * t.xr);
-        if (t.lds > 65536) return set_err(c, AFID_E_ARG, "refinement ratio too small for the refined -> coarse tiles");
+        const int x64c = span(h.xs, nxm, 64), y8 = span(h.ys, c->ny, 8);
+        if (y8 > 64) return set_err(c, AFID_E_ARG, "refinement ratio too large for the refined -> coarse tiles");
+        if (es * size_t(2 * y8 * x64c) > 65536) return set_err(c, AFID_E_ARG, "refinement ratio too small for the refined -> coarse tiles");
+        t.two = c->ny % 2 == 0;
+        for (int j = 0; j + 1 < c->ny; j += 2) t.two = t.two && h.ys[size_t(j + 1)] == h.ys[size_t(j)] + 2;
+        t.nseg = c->mixed ? (t.two ? coarse_ranges<float, 4, 2>(c) : coarse_ranges<float, 4, 1>(c))
+                          : (t.two ? coarse_ranges<double, 2, 2>(c) : coarse_ranges<double, 2, 1>(c));
     }
     if (most > 65536)
         return set_err(c, AFID_E_ARG, "refinement ratio too small for the transfer tiles (LDS plan above 64 KiB)");
@@ -1568,6 +1595,30 @@ static int xfer(afid_ctx *c, RT *out, const char *timer) {
     return rc;
 }
 
+// refined -> coarse cell centres
+template <typename RT, int NR, int NL>
+static void launch_to_coarse(afid_ctx *c, const KP &p, CoarseJob &jb) {
+    const int ngr = (c->ny + NL - 1) / NL;
+    const size_t lds = coarse_lds<RT, NR, NL>(c->nxmr);
+    const unsigned waves = unsigned((c->nxmr + 64 * NR - 1) / (64 * NR));
+    hipLaunchKernelGGL((k_to_coarse<RT, NR, NL>), dim3(tile_grid((long long)ngr * jb.nseg)), dim3(64u * waves), lds, c->stream, p, jb);
+}
+// (FP32 weights of the table for the mixed form's FP32 refined fields)
+static int to_coarse(afid_ctx *c, CoarseJob jb, const CoarseTab &t, const char *timer) {
+    KP p = make_kp(c);
+    jb.x_src = t.x_src; jb.y_src = t.y_src; jb.z_src = t.z_src;
+    if (c->mixed) { jb.x_w = t.x_wf; jb.y_w = t.y_wf; jb.z_w = t.z_wf; }
+    else { jb.x_w = t.x_w; jb.y_w = t.y_w; jb.z_w = t.z_w; }
+    tstart(c, timer);
+    jb.nseg = t.nseg;
+    if (c->mixed && t.two) launch_to_coarse<float, 4, 2>(c, p, jb);
+    else if (c->mixed) launch_to_coarse<float, 4, 1>(c, p, jb);
+    else if (t.two) launch_to_coarse<double, 2, 2>(c, p, jb);
+    else launch_to_coarse<double, 2, 1>(c, p, jb);
+    tstop(c);
+    return check_launch(c, "k_to_coarse");
+}
+
 extern "C" {
 
 int afid_solve_pressure_correction(afid_ctx *c) { NEED_SUBSTEP(c) NEED_FP64(c) return poisson(c, 1); }
@@ -1594,21 +1645,6 @@ static int interp_vel(afid_ctx *c) {
     return xfer<double, XF_VZ>(c, c->f[AFID_VZR], "mgrd_vzr");
 }
 int afid_interp_vel_mgrd(afid_ctx *c) { NEED_SAL(c) return interp_vel(c); }
-
-// refined -> coarse cell centres (k_interp_coarse_tile)
-// (FP32 weights of the table for the mixed form's FP32 refined fields)
-static int to_coarse(afid_ctx *c, CoarseJob jb, const CoarseTab &t, const char *timer) {
-    KP p = make_kp(c);
-    jb.x_src = t.x_src; jb.y_src = t.y_src; jb.z_src = t.z_src;
-    if (c->mixed) { jb.x_w = t.x_wf; jb.y_w = t.y_wf; jb.z_w = t.z_wf; }
-    else { jb.x_w = t.x_w; jb.y_w = t.y_w; jb.z_w = t.z_w; }
-    const dim3 gr(tile_grid((long long)((c->nxm + 63) / 64) * ((c->ny + SALC_TJ - 1) / SALC_TJ) * ((c->nz + SALC_TZ - 1) / SALC_TZ)));
-    tstart(c, timer);
-    if (c->mixed) hipLaunchKernelGGL(k_interp_coarse_tile<float>, gr, dim3(256), t.lds, c->stream, p, jb, t.xr, t.yr);
-    else hipLaunchKernelGGL(k_interp_coarse_tile<double>, gr, dim3(256), t.lds, c->stream, p, jb, t.xr, t.yr);
-    tstop(c);
-    return check_launch(c, "k_interp_coarse_tile");
-}
 
 int afid_interp_sal_multigrid(afid_ctx *c) {
     NEED_SAL(c)

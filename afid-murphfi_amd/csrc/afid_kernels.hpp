@@ -303,21 +303,10 @@ __device__ __forceinline__ long long xcd_block(long long) {
     const long long per = gridDim.x / 8;
     return (b % 8) * per + b / 8;
 }
-// Tile grids: a 1-D grid over the tiles (tile = tx + nx_tiles * (ty +
-// ny_tiles * tz)), padded to a multiple of 8 workgroups.  Through
-// xcd_block each XCD takes a contiguous range of tiles, so neighbouring
-// tiles, which read the same halo cache lines, run on one L2 at about the
-// same time.  False for the padding workgroups.
+// A 1-D grid over n items, padded to a multiple of 8 workgroups.  Through
+// xcd_block each XCD takes a contiguous range of them, so neighbours, which
+// read the same halo cache lines, run on one L2 at about the same time.
 __host__ __device__ __forceinline__ unsigned tile_grid(long long ntiles) { return unsigned((ntiles + 7) / 8 * 8); }
-__device__ __forceinline__ bool tile_3d(int nxt, int nyt, int nzt, int &tx, int &ty, int &tz) {
-    const long long t = xcd_block(0);
-    if (t >= (long long)nxt * nyt * nzt) return false;
-    tx = int(t % nxt);
-    const long long r = t / nxt;
-    ty = int(r % nyt);
-    tz = int(r / nyt);
-    return true;
-}
 // Column walk: a workgroup owns 4 consecutive y columns, one per
 // wavefront; workgroups form strips of STRIP_BLOCKS*4 columns in y, walked
 // along z, so the y and z neighbour columns a wavefront reads belong to its
@@ -828,28 +817,12 @@ __global__ void __launch_bounds__(256) k_max_partials(const double *partial, lon
 // ---------------------------------------------------------------------------
 // multiresolution transfers
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ int wrapn(int j, int n) { j %= n; return j < 0 ? j + n : j; }
 // periodic wrap of an index a few periods away at most, without a division
 __device__ __forceinline__ int wrapf(int j, int n) {
     while (j < 0) j += n;
     while (j >= n) j -= n;
     return j;
 }
-
-// Components (a, b, c) of a linear index q = a + A (b + B c) that advances by a
-// fixed step: the divisions happen once, each step costs a few adds.
-struct Walk3 {
-    int a, b, c, da, db, dc, A, B;
-    __device__ __forceinline__ Walk3(int q, int step, int A_, int B_) : A(A_), B(B_) {
-        a = q % A; b = (q / A) % B; c = q / (A * B);
-        da = step % A; db = (step / A) % B; dc = step / (A * B);
-    }
-    __device__ __forceinline__ void next() {
-        a += da; b += db; c += dc;
-        if (a >= A) { a -= A; ++b; }
-        if (b >= B) { b -= B; ++c; }
-    }
-};
 
 // Inclusive prefix sum over the 64 lanes of a wavefront with DPP lane
 // moves: Kogge-Stone within each row of 16 lanes (row_shr 1, 2, 4, 8),
@@ -883,159 +856,6 @@ __device__ __forceinline__ T wave_incl_scan(T v) {
     v += dpp_move<0x142, 0xa, false>(v);     // row_bcast:15
     v += dpp_move<0x143, 0xc, false>(v);     // row_bcast:31
     return v;
-}
-
-// Refined -> coarse cell centres through the fast coarse-grid loop of
-// interpolate_xyz_to_coarse_fast (HermiteInterpolations.F90:291-310):
-// InterpSalMultigrid (salinity.F90:458-491), InterpPhiMultigrid and the
-// transfer of AddLatentHeat (phasefield.F90:470-494, :651-725).
-// Tile: 64 coarse x (lanes) x SALC_TJ coarse y (two rows per wave), marching
-// through SALC_TZ coarse z planes.  Each refined z plane the tile needs is
-// staged once in LDS (with the wall ghosts of salinity.F90:466-482, double
-// buffered), contracted over x and y, and the last four contracted planes are
-// kept in registers for the z contraction.
-constexpr int SALC_TJ = 8, SALC_TZ = 16;
-constexpr int SALC_BU = 4;      // plane items loaded per batch and thread
-constexpr int SALC_IN = -(1 << 30);   // marks an interior point of a staged plane
-// What a refined-to-coarse tile interpolates and where the result goes.
-enum CoarseMode {
-    CM_SAL = 0,     // S with the wall ghosts of salinity.F90:466-482 -> salc (salc(nx) = 0)
-    CM_PHI = 1,     // phi with zero-gradient ghosts (phasefield.F90:479-487) -> phic (phic(nx) = 0)
-    CM_LAT = 2      // d phi with zero-gradient ghosts (:674-683) -> out (+)= scale * value
-};
-// Per axis and coarse index: the first of the 4 refined sources (1-based
-// reference index: x may name the wall ghosts 0 and nxr or the zero entries
-// beyond them, y/z may name periodic images) and its 4 weights (RT).  The
-// bracketing (fast) path of interpolate_xyz_to_coarse_fast and the general
-// path of interpolate_xyz_to_coarse differ only in these tables.
-struct CoarseJob {
-    int mode;
-    const void *src;            // refined field (RT)
-    void *out;                  // coarse field (RT for CM_SAL, double otherwise)
-    const int *x_src, *y_src, *z_src;
-    const void *x_w, *y_w, *z_w;
-    double scale;
-    int accumulate;
-};
-template <typename RT>
-__device__ __forceinline__ RT coarse_src(const KP &p, const CoarseJob &jb, const RT *f, int kr, int jj, int ii) {
-    const long long o2 = (long long)ii * p.planer + (long long)jj * p.ldxr;
-    if (kr >= 1 && kr <= p.nxmr) return f[o2 + kr - 1];
-    if (kr == 0) {
-        const RT s1 = f[o2];
-        if (jb.mode != CM_SAL) return s1;
-        return p.sfixs == 1 ? RT(2.0 * p.salbp[(long long)ii * p.nyr + jj]) - s1 : s1;
-    }
-    if (kr == p.nxr) {
-        const RT sn = f[o2 + p.nxmr - 1];
-        if (jb.mode != CM_SAL) return sn;
-        return p.sfixn == 1 ? RT(2.0 * p.saltp[(long long)ii * p.nyr + jj]) - sn : sn;
-    }
-    return RT(0);
-}
-template <typename RT>
-__global__ void __launch_bounds__(256) k_interp_coarse_tile(KP p, CoarseJob jb, int xrmax, int yrmax) {
-    extern __shared__ __align__(16) unsigned char smraw[];
-    RT *sm = reinterpret_cast<RT *>(smraw);
-    const RT *src = static_cast<const RT *>(jb.src);
-    const int *x_src = jb.x_src;
-    const RT *xb_w = static_cast<const RT *>(jb.x_w);
-    const RT *yb_w = static_cast<const RT *>(jb.y_w), *zb_w = static_cast<const RT *>(jb.z_w);
-    const int *yb_src = jb.y_src, *zb_src = jb.z_src;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, t = threadIdx.x;
-    const int nxt = (p.nxm + 63) / 64;
-    int tx, ty, tz;
-    if (!tile_3d(nxt, (p.ny + SALC_TJ - 1) / SALC_TJ, (p.nz + SALC_TZ - 1) / SALC_TZ, tx, ty, tz)) return;
-    const int K0 = tx * 64, K1 = min(K0 + 64, p.nxm);
-    const int J0 = ty * SALC_TJ, nj = min(SALC_TJ, p.ny - J0);
-    const int I0 = tz * SALC_TZ, I1 = min(I0 + SALC_TZ, p.nz);
-    const int x0 = x_src[K0], XR = x_src[K1 - 1] + 4 - x0;                  // reference refined x index
-    const int y0 = yb_src[J0] - 1, YR = yb_src[J0 + nj - 1] - 1 + 4 - y0;   // 0-based refined y
-    const int zfirst = zb_src[I0] - 1, zlast = zb_src[I1 - 1] - 1 + 3;      // 0-based refined z (unwrapped)
-    const int k = K0 + lane;
-    const bool kok = k < K1;
-    RT wx[4] = {0, 0, 0, 0};
-    int xa = 0;
-    if (kok) { xa = x_src[k] - x0; for (int a = 0; a < 4; ++a) wx[a] = xb_w[4 * k + a]; }
-    // two coarse rows per wave: tj = wave and wave + 4
-    int ya[2] = {0, 0};
-    RT wy[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
-    bool rok[2];
-    for (int h = 0; h < 2; ++h) {
-        const int tj = wave + 4 * h;
-        rok[h] = tj < nj;
-        if (rok[h]) { ya[h] = yb_src[J0 + tj] - 1 - y0; for (int b = 0; b < 4; ++b) wy[h][b] = yb_w[4 * (J0 + tj) + b]; }
-    }
-    RT ring[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}};   // contracted refined planes zr-3..zr
-    const int plane = XR * YR;
-    // refined y rows of the tile (periodic): their indices and row offsets
-    __shared__ int rowj[64];
-    for (int q = t; q < YR; q += 256) rowj[q] = wrapf(y0 + q, p.nyr);
-    __syncthreads();
-    int ic = I0;
-    for (int zr = zfirst; zr <= zlast; ++zr) {
-        RT *B = sm + ((zr - zfirst) & 1) * xrmax * yrmax;     // [yr][xr], double buffered
-        const int ii = wrapn(zr, p.nzr);
-        const RT *fz = src + (long long)ii * p.planer;
-        // SALC_BU loads per thread in flight: interior points read first
-        // (an item outside the plane reads a valid address), wall ghosts and
-        // points beyond them are filled in afterwards
-        Walk3 w(t, 256, XR, YR);
-        for (int q0 = t; q0 < plane; q0 += 256 * SALC_BU) {
-            RT v[SALC_BU];
-            int dst[SALC_BU], kx[SALC_BU], jy[SALC_BU];
-#pragma unroll
-            for (int r = 0; r < SALC_BU; ++r) {
-                const int kr = x0 + w.a, jj = rowj[min(w.b, YR - 1)];
-                const bool live = q0 + 256 * r < plane, in = live && kr >= 1 && kr <= p.nxmr;
-                v[r] = fz[(long long)jj * p.ldxr + (in ? kr - 1 : 0)];
-                dst[r] = live ? __mul24(w.b, xrmax) + w.a : -1;
-                kx[r] = in ? SALC_IN : kr;
-                jy[r] = jj;
-                w.next();
-            }
-#pragma unroll
-            for (int r = 0; r < SALC_BU; ++r)
-                if (dst[r] >= 0) B[dst[r]] = kx[r] == SALC_IN ? v[r] : coarse_src<RT>(p, jb, src, kx[r], jy[r], ii);
-        }
-        __syncthreads();
-        for (int h = 0; h < 2; ++h) {
-            RT v = RT(0);
-            if (kok && rok[h]) {
-                for (int b = 0; b < 4; ++b) {
-                    const RT *row = B + __mul24(ya[h] + b, xrmax) + xa;
-                    const RT q1 = row[0] * wx[0] + row[1] * wx[1] + row[2] * wx[2] + row[3] * wx[3];
-                    v = b == 0 ? q1 * wy[h][0] : v + q1 * wy[h][b];
-                }
-            }
-            ring[h][0] = ring[h][1]; ring[h][1] = ring[h][2]; ring[h][2] = ring[h][3]; ring[h][3] = v;
-        }
-        // every coarse plane whose 4-plane stencil ends at zr is complete
-        while (ic < I1 && zb_src[ic] - 1 + 3 == zr) {
-            const RT *wz = zb_w + 4 * ic;
-            for (int h = 0; h < 2; ++h)
-                if (kok && rok[h]) {
-                    const RT v = ring[h][0] * wz[0] + ring[h][1] * wz[1] + ring[h][2] * wz[2] + ring[h][3] * wz[3];
-                    const long long o = bidx(p, k, J0 + wave + 4 * h, ic);
-                    if (jb.mode == CM_SAL) static_cast<RT *>(jb.out)[o] = v;
-                    else {
-                        double *out = static_cast<double *>(jb.out);
-                        const double val = jb.mode == CM_LAT ? jb.scale * double(v) : double(v);
-                        out[o] = jb.accumulate ? out[o] + val : val;
-                    }
-                }
-            ++ic;
-        }
-    }
-    // salc(nx), phic(nx) stay zero (salinity.F90:463, phasefield.F90:476): written by the last x tile
-    if (jb.mode != CM_LAT && tx == nxt - 1 && lane == 0)
-        for (int h = 0; h < 2; ++h)
-            if (rok[h])
-                for (int iz = I0; iz < I1; ++iz) {
-                    const long long o = bidx(p, p.nxm, J0 + wave + 4 * h, iz);
-                    if (jb.mode == CM_SAL) static_cast<RT *>(jb.out)[o] = RT(0);
-                    else static_cast<double *>(jb.out)[o] = 0.0;
-                }
 }
 
 // ---------------------------------------------------------------------------

@@ -2,7 +2,7 @@
 // and implicit phi terms on the refined grid, the fused phi column, the
 // masked velocity solves, the coarse -> refined temperature transfer and the
 // seeded sphere.  The refined -> coarse transfers (phic, latent heat) share
-// k_interp_coarse_tile with InterpSalMultigrid.
+// k_to_coarse with InterpSalMultigrid.
 #pragma once
 #include <hip/hip_runtime.h>
 #include "afid_params.hpp"

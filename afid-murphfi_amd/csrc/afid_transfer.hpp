@@ -1,5 +1,6 @@
-// afid_transfer.hpp -- coarse -> refined transfers: InterpVelMgrd
-// (InterpVelMgrd.F90:11-237) and InterpTempMultigrid (phasefield.F90:498-520).
+// afid_transfer.hpp -- transfers between the grids.  Coarse -> refined:
+// InterpVelMgrd (InterpVelMgrd.F90:11-237) and InterpTempMultigrid
+// (phasefield.F90:498-520); refined -> coarse: k_to_coarse.
 //
 // Every transfer is a product of one-dimensional 4-point Hermite stencils, so
 // the axes can be taken one after the other.
@@ -311,6 +312,205 @@ __global__ void __launch_bounds__(SEG ? 512 : 256) k_xfer_yz(XferJob jb) {
             for (int l = 0; l < NL; ++l) v[l] += tot[(q * NL + l) * 64 + lane];
     }
     walk(std::true_type{});
+}
+
+// Refined -> coarse cell centres through the fast coarse-grid loop of
+// interpolate_xyz_to_coarse_fast (HermiteInterpolations.F90:291-310):
+// InterpSalMultigrid (salinity.F90:458-491), InterpPhiMultigrid and the
+// transfer of AddLatentHeat (phasefield.F90:470-494, :651-725).
+// What is interpolated and where the result goes.
+enum CoarseMode {
+    CM_SAL = 0,     // S with the wall ghosts of salinity.F90:466-482 -> salc (salc(nx) = 0)
+    CM_PHI = 1,     // phi with zero-gradient ghosts (phasefield.F90:479-487) -> phic (phic(nx) = 0)
+    CM_LAT = 2      // d phi with zero-gradient ghosts (:674-683) -> out (+)= scale * value
+};
+// Per axis and coarse index: the first of the 4 refined sources (1-based
+// reference index: x may name the wall ghosts 0 and nxr or the zero entries
+// beyond them, y/z may name periodic images) and its 4 weights (RT).  The
+// bracketing (fast) path of interpolate_xyz_to_coarse_fast and the general
+// path of interpolate_xyz_to_coarse differ only in these tables.
+struct CoarseJob {
+    int mode;
+    const void *src;            // refined field (RT)
+    void *out;                  // coarse field (RT for CM_SAL, double otherwise)
+    const int *x_src, *y_src, *z_src;
+    const void *x_w, *y_w, *z_w;
+    double scale;
+    int accumulate;
+    int nseg;                   // ranges of coarse z planes
+};
+// A workgroup takes NL adjacent coarse lines of y and a range of z, its
+// wavefronts the refined x (NR per lane).  It walks the refined z planes with
+// the rows of the next 2 on their way, contracts the 4 rows of each line
+// (NL = 2: lines two refined rows apart share them), keeps the last four
+// planes in registers, and where a coarse plane's stencil is complete puts the
+// contracted refined row in LDS, from which each thread takes its coarse x.
+// Ghosts at the walls are folded into the x weights: the mirrored value into
+// the tap it mirrors, the wall's 2 S into gS / gN, whose y / z contraction 16
+// lanes form.
+// What bounds it: the read of the refined field once (us a launch, at 5.2 TB/s,
+// now, and as 64 x 8 x 16 tiles staged in LDS with a barrier per refined plane
+// before, which left 72 workgroups at 64^3):
+//   64^3 from 128^3 FP64                 4     13     190
+//   384 x 192^2 from 768 x 384^2 FP64  196    242     495
+//   384 x 384^2 from 768^3 FP32        370    497    1189
+//   256 x 256^2 from 512^3 FP32 (phi)  129    148     482
+// Single lines instead of pairs: 1147 against 850 us a step at 384 x 192^2 (8
+// rows instead of 6 for two lines), 44 against 50 at 64^3 before the choice of
+// ranges (35 now).
+template <typename RT, int NR, int NL>
+__global__ void __launch_bounds__(512) k_to_coarse(KP p, CoarseJob jb) {
+    using V = typename XVec<RT, NR>::V;
+    constexpr int NU = 4 + 2 * (NL - 1), PD = 2;                // rows; planes loaded ahead (4: the same)
+    extern __shared__ __align__(16) unsigned char smraw[];
+    RT *sm = reinterpret_cast<RT *>(smraw);                     // [2][line][reference refined x + NR - 1]
+    const int LD = (p.nxmr + 3 * NR - 1) / NR * NR;
+    const int t = threadIdx.x, T = blockDim.x, lane = t & 63;
+    const int ngr = (p.ny + NL - 1) / NL, item = int(xcd_block(0));
+    if (item >= ngr * jb.nseg) return;                          // whole workgroups
+    const int seg = item / ngr, J0 = (item - seg * ngr) * NL;
+    const int I0 = int((long long)p.nz * seg / jb.nseg), I1 = int((long long)p.nz * (seg + 1) / jb.nseg);
+    if (I0 >= I1) return;
+    const RT *src = static_cast<const RT *>(jb.src);
+    const ConstTab<int> sy = const_tab(jb.y_src), sz = const_tab(jb.z_src);
+    const ConstTab<RT> ywc = const_tab(static_cast<const RT *>(jb.y_w));
+    const int y0 = sy[J0] - 1, xw = t * NR, x = min(xw, (p.nxmr - 1) / NR * NR);
+    RT wy[NL][4];
+    long long ro[NU];
+#pragma unroll
+    for (int l = 0; l < NL; ++l)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) wy[l][b] = ywc[4 * (J0 + l) + b];
+#pragma unroll
+    for (int c = 0; c < NU; ++c) ro[c] = (long long)wrapf(y0 + c, p.nyr) * p.ldxr + x;
+    // taps of coarse k: weights of reference x base .. base + 3, all interior
+    struct Taps { int base; RT w[4], gS, gN; };
+    auto taps = [&](int k) {
+        Taps q{1, {RT(0), RT(0), RT(0), RT(0)}, RT(0), RT(0)};
+        if (k >= p.nxm) return q;
+        const RT *w4 = static_cast<const RT *>(jb.x_w) + 4 * k;
+        const int s = jb.x_src[k];
+        q.base = max(1, min(s, p.nxmr - 3));
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            int kr = s + a;
+            RT w = w4[a];
+            if (kr < 0 || kr > p.nxr) w = RT(0);
+            else if (kr == 0) {
+                if (jb.mode == CM_SAL && p.sfixs == 1) { q.gS += w; w = -w; }
+            } else if (kr == p.nxr) {
+                if (jb.mode == CM_SAL && p.sfixn == 1) { q.gN += w; w = -w; }
+            }
+            kr = max(1, min(kr, p.nxmr));
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (kr - q.base == c) q.w[c] += w;
+        }
+        return q;
+    };
+    Taps tp[2] = {taps(t), taps(t + T)};
+    // 2 S of the walls: lane (a, b, l, wall) its point of the y / z stencil
+    const bool wall = jb.mode == CM_SAL && (2 * T < p.nxm || __any(tp[0].gS != RT(0) || tp[0].gN != RT(0) || tp[1].gS != RT(0) || tp[1].gN != RT(0)));
+    const int la = lane & 3, lb = (lane >> 2) & 3, ll = NL == 2 ? (lane >> 4) & 1 : 0;
+    const double *bp = lane < 32 ? p.salbp : p.saltp;
+    const int by = wrapf(y0 + 2 * ll + lb, p.nyr);
+    const RT bw = static_cast<const RT *>(jb.y_w)[4 * (J0 + ll) + lb];
+    RT bv = RT(0);
+    auto load_wall = [&](int zs) { bv = RT(2.0 * bp[(long long)wrapf(zs + la, p.nzr) * p.nyr + by]); };
+
+    int zr = sz[I0] - 1;
+    const int end = sz[I1 - 1] + 2;
+    int zw = wrapf(zr, p.nzr), zl = zr;                          // the plane to load next, on the periodic axis and off it
+    V R[PD][NU], W[4][NL];
+    auto load = [&](V (&r)[NU]) {
+        const RT *q = src + zw * p.planer;
+#pragma unroll
+        for (int c = 0; c < NU; ++c) r[c] = *reinterpret_cast<const V *>(q + ro[c]);
+        if (zl < end) { ++zl; if (++zw == p.nzr) zw = 0; }       // (past the end: the last plane again)
+    };
+#pragma unroll
+    for (int q = 0; q < PD; ++q) load(R[q]);
+    // the stencils of 64 coarse planes at a time, one per lane
+    int ic = I0, base = I0, tn = 0;
+    RT t0 = RT(0), t1 = RT(0), t2 = RT(0), t3 = RT(0);
+    auto fill = [&]() {
+        base = ic;
+        const int k = min(ic + lane, I1 - 1);
+        tn = jb.z_src[k] + 2;
+        const RT *w4 = static_cast<const RT *>(jb.z_w) + 4 * k;
+        t0 = w4[0]; t1 = w4[1]; t2 = w4[2]; t3 = w4[3];
+    };
+    fill();
+    int need = __builtin_amdgcn_readlane(tn, 0), e = 0;
+    if (wall) load_wall(need - 3);
+    auto store = [&](long long o, RT v) {
+        if (jb.mode == CM_SAL) static_cast<RT *>(jb.out)[o] = v;
+        else {
+            double *out = static_cast<double *>(jb.out);
+            const double val = jb.mode == CM_LAT ? jb.scale * double(v) : double(v);
+            out[o] = jb.accumulate ? out[o] + val : val;
+        }
+    };
+    auto emit = [&](int q) {
+        const int k = ic - base;
+        const RT w0 = lane_value(t0, k), w1 = lane_value(t1, k), w2 = lane_value(t2, k), w3 = lane_value(t3, k);
+        RT *b = sm + (e & 1) * NL * LD;
+        e ^= 1;
+#pragma unroll
+        for (int l = 0; l < NL; ++l) {
+            const V v = W[(q + 1) & 3][l] * w0 + W[(q + 2) & 3][l] * w1 + W[(q + 3) & 3][l] * w2 + W[q][l] * w3;
+            if (xw < p.nxmr) *reinterpret_cast<V *>(b + l * LD + NR + xw) = v;
+        }
+        __syncthreads();
+        RT g[2][NL] = {};
+        if (wall) {
+            RT s = bv * bw * (la == 0 ? w0 : la == 1 ? w1 : la == 2 ? w2 : w3);
+            s += dpp_move<0x128, 0xf, true>(s);                 // row_ror: the 16 points of a line and wall
+            s += dpp_move<0x124, 0xf, true>(s);
+            s += dpp_move<0x122, 0xf, true>(s);
+            s += dpp_move<0x121, 0xf, true>(s);
+#pragma unroll
+            for (int l = 0; l < NL; ++l) { g[0][l] = lane_value(s, 16 * l); g[1][l] = lane_value(s, 32 + 16 * l); }
+        }
+        auto point = [&](int kk, const Taps &q) {
+            if (kk >= p.nxm) return;
+#pragma unroll
+            for (int l = 0; l < NL; ++l) {
+                const RT *r = b + l * LD + NR - 1;
+                RT v = RT(0);
+#pragma unroll
+                for (int a = 0; a < 4; ++a) v += r[min(q.base + a, p.nxmr)] * q.w[a];
+                if (wall) v += q.gS * g[0][l] + q.gN * g[1][l];
+                store(bidx(p, kk, J0 + l, ic), v);
+            }
+        };
+        point(t, tp[0]);
+        point(t + T, tp[1]);
+        for (int kk = t + 2 * T; kk < p.nxm; kk += T) point(kk, taps(kk));
+        // salc(nx), phic(nx) stay zero (salinity.F90:463, phasefield.F90:476)
+        if (jb.mode != CM_LAT && t < NL) {
+            const long long o = bidx(p, p.nxm, J0 + t, ic);
+            if (jb.mode == CM_SAL) static_cast<RT *>(jb.out)[o] = RT(0);
+            else static_cast<double *>(jb.out)[o] = 0.0;
+        }
+        ++ic;
+    };
+    for (; zr <= end; zr += 4) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (zr + q > end) break;
+#pragma unroll
+            for (int l = 0; l < NL; ++l) W[q][l] = R[q % PD][2 * l] * wy[l][0] + R[q % PD][2 * l + 1] * wy[l][1] + R[q % PD][2 * l + 2] * wy[l][2] + R[q % PD][2 * l + 3] * wy[l][3];
+            load(R[q % PD]);
+            while (need == zr + q) {
+                emit(q);
+                if (ic >= I1) { need = end + 1; break; }
+                if (ic - base > 63) fill();
+                need = __builtin_amdgcn_readlane(tn, ic - base);
+                if (wall) load_wall(need - 3);
+            }
+        }
+    }
 }
 
 // index nxr of a refined field to zero

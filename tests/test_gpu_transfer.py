@@ -15,7 +15,7 @@ import pytest
 
 import pyafid
 import pyoracle
-from helpers import load_state, random_state, relerr
+from helpers import load_state, random_state, relerr, uniform
 from test_gpu_phase import PF, pf_state
 
 pytestmark = pytest.mark.gpu
@@ -68,3 +68,49 @@ def test_upload_between_graph_replays():
         g.close()
     for a, b in zip(got[:3], got[3:]):
         assert np.array_equal(a, b) and not np.any(b[..., 32])
+
+
+# refined -> coarse: wavefronts per row, rows that the coarse ones outnumber,
+# pairs of lines and single ones, ranges of z, grids that bracket and that do not
+DOWN = [((s, 4, 6), (2 * s, 8, 12), {}) for s in (2, 3, 4, 31, 32, 33, 63, 64, 65, 96, 127, 128, 129, 255, 256, 257, 384, 512)]
+DOWN += [((8, 2, 288), (16, 4, 576), {}), ((16, 9, 2), (32, 18, 4), {}), ((32, 64, 48), (64, 128, 96), {}), ((128, 192, 4), (256, 384, 8), {}),
+         ((20, 6, 9), (61, 13, 20), {}), ((24, 12, 6), (30, 18, 15), {}), ((24, 6, 6), (40, 12, 12), dict(istr3r=0)),
+         ((60, 3, 4), (120, 6, 8), dict(sfixs=0)), ((60, 3, 4), (120, 6, 8), dict(sfixn=0))]
+DOWN_FLAT = [((200, 4, 6), (256, 8, 12), {}), ((300, 4, 4), (330, 12, 12), dict(sfixs=0, sfixn=0))]      # mixed form only
+DOWN = [d + (p,) for d in DOWN for p in ("fp64", "mixed")] + [d + ("mixed",) for d in DOWN_FLAT]
+
+
+@pytest.mark.parametrize("base,fine,more,form", DOWN, ids=lambda s: s if isinstance(s, str) else "_".join(s) if isinstance(s, dict) else "x".join(map(str, s)))
+def test_to_coarse_matches_the_oracle(base, fine, more, form):
+    """Three stencils of 4 terms (absolute weights up to 1.3 each) of values
+    rounded once: 32 units of the result's max norm."""
+    tol = 32 * 2.0 ** (-53 if form == "fp64" else -24)
+    for kind, call, name in (("sal", "interp_sal_multigrid", "salc"), ("phi", "interp_phi_multigrid", "phic"), ("phi", "add_latent_heat", "hro")):
+        if form == "mixed" and call == "add_latent_heat":
+            continue                                            # per-routine physics is FP64
+        cfg = dict(nxm=base[0], nym=base[1], nzm=base[2], istr3=8, istr3r=8, rayt=1e6, prat=1.0, multires=1,
+                   nxmr=fine[0], nymr=fine[1], nzmr=fine[2])
+        cfg.update(dict(salinity=1, rays=-2e6, pras=4.0) if kind == "sal" else
+                   dict(phasefield=1, pf_a=PF["pf_a"], pf_s=PF["pf_s"], pf_tm=PF["pf_tm"], pf_eps=0.1))
+        cfg.update(more)
+        st = random_state(cfg, 9) if kind == "sal" else pf_state(cfg, 9)
+        if kind == "sal":
+            st["salbp"] = uniform(91, (fine[2], fine[1], 1))
+            st["saltp"] = uniform(92, (fine[2], fine[1], 1)) - 1.0
+        if call == "add_latent_heat":
+            st["rhsr"] = uniform(93, (fine[2], fine[1], fine[0] + 1)) - 0.5
+            st["hro"] = uniform(94, (base[2], base[1], base[0] + 1))
+            st["hro"][..., -1] = 0.0
+        else:
+            st[name] = np.ones((base[2], base[1], base[0] + 1))
+        o, g = pyoracle.Oracle(cfg), pyafid.Solver(dict(cfg, precision=pyafid.MIXED if form == "mixed" else pyafid.FP64))
+        load_state(o, st, upload=False)
+        load_state(g, st, upload=True)
+        for s in (o, g):
+            s.set_substep(1e-3, 1)
+            s.call(call)
+        n = base[0] if name == "hro" else base[0] + 1           # (hro(nx) is unused)
+        e = relerr(g.download(name)[..., :n], o.field(name)[..., :n])
+        assert e <= tol, (call, e, tol)
+        o.close()
+        g.close()
