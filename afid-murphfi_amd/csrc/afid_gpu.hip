@@ -55,6 +55,7 @@ struct CoarseTab {
     const double *x_w = nullptr, *y_w = nullptr, *z_w = nullptr;
     const float *x_wf = nullptr, *y_wf = nullptr, *z_wf = nullptr;
     int nseg = 1;                // ranges of z
+    bool two_x = false;          // k_to_coarse_x2: coarse x takes the refined 2 k - 1 .. 2 k + 2
     bool two = false;            // coarse y lines in pairs two refined lines apart (ratio 2)
     bool general = false;        // interpolate_xyz_to_coarse (refined grid does not bracket)
 };
@@ -471,12 +472,15 @@ static size_t coarse_lds(int nxmr) { return sizeof(RT) * 2 * NL * size_t((nxmr +
 // 4096 / 6144 wavefronts instead: 384 x 192^2 FP64 806 / 850 / 728 / 863,
 // 256^3 FP32 500 / 423 / 508 / 490; this rule takes the best of both.
 template <typename RT, int NR, int NL>
-static int coarse_ranges(afid_ctx *c) {
+static int coarse_ranges(afid_ctx *c, bool x2) {
     int per_cu = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_to_coarse<RT, NR, NL>, 64 * ((c->nxmr + 64 * NR - 1) / (64 * NR)),
-                                                     coarse_lds<RT, NR, NL>(c->nxmr)) != hipSuccess || per_cu < 1) per_cu = 1;
+    const int nch = (c->nxmr + 64 * NR - 1) / (64 * NR);
+    const hipError_t e = x2 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_to_coarse_x2<RT, NR, NL>, 256, 0)
+                            : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_to_coarse<RT, NR, NL>, 64 * nch, coarse_lds<RT, NR, NL>(c->nxmr));
+    if (e != hipSuccess || per_cu < 1) per_cu = 1;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || cus < 1) cus = 256;
-    const long long ngr = (c->ny + NL - 1) / NL, slots = (long long)per_cu * cus;
+    // items and slots: workgroups of whole rows, or (x2) single wavefronts
+    const long long ngr = (long long)((c->ny + NL - 1) / NL) * (x2 ? nch : 1), slots = (long long)per_cu * cus * (x2 ? 4 : 1);
     int best = 1;
     double least = 0;
     for (int n = 1; n <= c->nz; ++n) {
@@ -1001,8 +1005,10 @@ static int setup(afid_ctx *c) {
         if (es * size_t(2 * y8 * x64c) > 65536) return set_err(c, AFID_E_ARG, "refinement ratio too small for the refined -> coarse tiles");
         t.two = c->ny % 2 == 0;
         for (int j = 0; j + 1 < c->ny; j += 2) t.two = t.two && h.ys[size_t(j + 1)] == h.ys[size_t(j)] + 2;
-        t.nseg = c->mixed ? (t.two ? coarse_ranges<float, 4, 2>(c) : coarse_ranges<float, 4, 1>(c))
-                          : (t.two ? coarse_ranges<double, 2, 2>(c) : coarse_ranges<double, 2, 1>(c));
+        t.two_x = q == 1 && nxmr == 2 * nxm;
+        for (int k = 0; k < nxm; ++k) t.two_x = t.two_x && h.xs[size_t(k)] == 2 * k;
+        t.nseg = c->mixed ? (t.two ? coarse_ranges<float, 4, 2>(c, t.two_x) : coarse_ranges<float, 4, 1>(c, t.two_x))
+                          : (t.two ? coarse_ranges<double, 2, 2>(c, t.two_x) : coarse_ranges<double, 2, 1>(c, t.two_x));
     }
     if (most > 65536)
         return set_err(c, AFID_E_ARG, "refinement ratio too small for the transfer tiles (LDS plan above 64 KiB)");
@@ -1597,8 +1603,13 @@ static int xfer(afid_ctx *c, RT *out, const char *timer) {
 
 // refined -> coarse cell centres
 template <typename RT, int NR, int NL>
-static void launch_to_coarse(afid_ctx *c, const KP &p, CoarseJob &jb) {
+static void launch_to_coarse(afid_ctx *c, const KP &p, CoarseJob &jb, bool x2) {
     const int ngr = (c->ny + NL - 1) / NL;
+    if (x2) {
+        const long long items = (long long)ngr * jb.nseg * ((c->nxmr + 64 * NR - 1) / (64 * NR));
+        hipLaunchKernelGGL((k_to_coarse_x2<RT, NR, NL>), dim3(tile_grid((items + 3) / 4)), dim3(256), 0, c->stream, p, jb);
+        return;
+    }
     const size_t lds = coarse_lds<RT, NR, NL>(c->nxmr);
     const unsigned waves = unsigned((c->nxmr + 64 * NR - 1) / (64 * NR));
     hipLaunchKernelGGL((k_to_coarse<RT, NR, NL>), dim3(tile_grid((long long)ngr * jb.nseg)), dim3(64u * waves), lds, c->stream, p, jb);
@@ -1611,10 +1622,10 @@ static int to_coarse(afid_ctx *c, CoarseJob jb, const CoarseTab &t, const char *
     else { jb.x_w = t.x_w; jb.y_w = t.y_w; jb.z_w = t.z_w; }
     tstart(c, timer);
     jb.nseg = t.nseg;
-    if (c->mixed && t.two) launch_to_coarse<float, 4, 2>(c, p, jb);
-    else if (c->mixed) launch_to_coarse<float, 4, 1>(c, p, jb);
-    else if (t.two) launch_to_coarse<double, 2, 2>(c, p, jb);
-    else launch_to_coarse<double, 2, 1>(c, p, jb);
+    if (c->mixed && t.two) launch_to_coarse<float, 4, 2>(c, p, jb, t.two_x);
+    else if (c->mixed) launch_to_coarse<float, 4, 1>(c, p, jb, t.two_x);
+    else if (t.two) launch_to_coarse<double, 2, 2>(c, p, jb, t.two_x);
+    else launch_to_coarse<double, 2, 1>(c, p, jb, t.two_x);
     tstop(c);
     return check_launch(c, "k_to_coarse");
 }

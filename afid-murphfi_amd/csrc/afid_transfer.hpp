@@ -513,6 +513,131 @@ __global__ void __launch_bounds__(512) k_to_coarse(KP p, CoarseJob jb) {
     }
 }
 
+// The same for phi and d phi (mirrored ghosts) where every coarse x takes the
+// refined 2 k - 1 .. 2 k + 2: the x stencil comes first, on each row as it
+// arrives, from a lane's own NR points and one of either neighbour (at the ends
+// of a wavefront's run one load more), so that NR / 2 values a lane stay to be
+// contracted in y and z and nothing goes through LDS.  As fast as the form
+// above; it is here because the order x, y, z with these roundings (dot4) is
+// the more exact one for the FP32 fields: the kinetic energy of a 256 x 512^2
+// melting sphere after 100 steps is 9.6e-7 from the FP64 form's, 1.4e-6 with y,
+// z, x.  One wavefront per run of refined x, pair of lines and range of z.
+template <typename RT>
+__device__ __forceinline__ RT dot4(RT a0, RT w0, RT a1, RT w1, RT a2, RT w2, RT a3, RT w3) {
+    if constexpr (sizeof(RT) == 4) return __builtin_fmaf(a3, w3, __builtin_fmaf(a2, w2, __builtin_fmaf(a0, w0, a1 * w1)));
+    else return __builtin_fma(a3, w3, __builtin_fma(a2, w2, __builtin_fma(a0, w0, a1 * w1)));
+}
+template <typename RT, int NR, int NL>
+__global__ void __launch_bounds__(256) k_to_coarse_x2(KP p, CoarseJob jb) {
+    using V = typename XVec<RT, NR>::V;
+    constexpr int NU = 4 + 2 * (NL - 1), NC = NR / 2, PD = 4;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nch = (p.nxmr + 64 * NR - 1) / (64 * NR), ngr = (p.ny + NL - 1) / NL;
+    const int item = int(xcd_block(0)) * 4 + wave;
+    if (item >= nch * ngr * jb.nseg) return;
+    const int seg = item / (nch * ngr), rest = item - seg * nch * ngr, J0 = rest / nch * NL;
+    const int I0 = int((long long)p.nz * seg / jb.nseg), I1 = int((long long)p.nz * (seg + 1) / jb.nseg);
+    if (I0 >= I1) return;
+    const RT *src = static_cast<const RT *>(jb.src);
+    double *out = static_cast<double *>(jb.out);
+    const ConstTab<int> sy = const_tab(jb.y_src), sz = const_tab(jb.z_src);
+    const ConstTab<RT> ywc = const_tab(static_cast<const RT *>(jb.y_w));
+    const int y0 = sy[J0] - 1, xw = ((rest % nch) * 64 + lane) * NR, x = min(xw, (p.nxmr - 1) / NR * NR);
+    // the point beyond the run: the mirrored end at the walls
+    const int xh = lane == 0 ? max(xw - 1, 0) : lane == 63 ? min(xw + NR, p.nxmr - 1) : x;
+    RT wy[NL][4], wx[NC][4];
+    long long ro[NU];
+#pragma unroll
+    for (int l = 0; l < NL; ++l)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) wy[l][b] = ywc[4 * (J0 + l) + b];
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int a = 0; a < 4; ++a) wx[c][a] = static_cast<const RT *>(jb.x_w)[4 * min(xw / 2 + c, p.nxm - 1) + a];
+#pragma unroll
+    for (int c = 0; c < NU; ++c) ro[c] = (long long)wrapf(y0 + c, p.nyr) * p.ldxr;
+    int zr = sz[I0] - 1;
+    const int end = sz[I1 - 1] + 2;
+    int zw = wrapf(zr, p.nzr), zl = zr;                          // the plane to load next, on the periodic axis and off it
+    V R[PD][NU];
+    RT H[PD][NU], W[4][NL][NC];
+    auto load = [&](V (&r)[NU], RT (&h)[NU]) {
+        const RT *q = src + zw * p.planer;
+#pragma unroll
+        for (int c = 0; c < NU; ++c) { r[c] = *reinterpret_cast<const V *>(q + ro[c] + x); h[c] = q[ro[c] + xh]; }
+        if (zl < end) { ++zl; if (++zw == p.nzr) zw = 0; }       // (past the end: the last plane again)
+    };
+#pragma unroll
+    for (int q = 0; q < PD; ++q) load(R[q], H[q]);
+    // the stencils of 64 coarse planes at a time, one per lane
+    int ic = I0, base = I0, tn = 0;
+    RT t0 = RT(0), t1 = RT(0), t2 = RT(0), t3 = RT(0);
+    auto fill = [&]() {
+        base = ic;
+        const int k = min(ic + lane, I1 - 1);
+        tn = jb.z_src[k] + 2;
+        const RT *w4 = static_cast<const RT *>(jb.z_w) + 4 * k;
+        t0 = w4[0]; t1 = w4[1]; t2 = w4[2]; t3 = w4[3];
+    };
+    fill();
+    int need = __builtin_amdgcn_readlane(tn, 0);
+    auto contract = [&](int q) {
+        RT X[NU][NC];
+#pragma unroll
+        for (int c = 0; c < NU; ++c) {
+            const V v = R[q % PD][c];
+            RT a[NR + 2];
+            a[0] = pick(lane == 0, H[q % PD][c], lane_prev(RT(v[NR - 1])));
+            a[NR + 1] = pick(lane == 63, H[q % PD][c], lane_next(RT(v[0])));
+#pragma unroll
+            for (int j = 0; j < NR; ++j) a[j + 1] = v[j];
+#pragma unroll
+            for (int j = 3; j <= NR + 1; j += 2) a[j] = xw + j - 1 == p.nxmr ? a[j - 1] : a[j];      // the mirrored ghost
+#pragma unroll
+            for (int m = 0; m < NC; ++m) X[c][m] = dot4<RT>(a[2 * m], wx[m][0], a[2 * m + 1], wx[m][1], a[2 * m + 2], wx[m][2], a[2 * m + 3], wx[m][3]);
+        }
+#pragma unroll
+        for (int l = 0; l < NL; ++l)
+#pragma unroll
+            for (int m = 0; m < NC; ++m)
+                W[q][l][m] = dot4<RT>(X[2 * l][m], wy[l][0], X[2 * l + 1][m], wy[l][1], X[2 * l + 2][m], wy[l][2], X[2 * l + 3][m], wy[l][3]);
+    };
+    auto emit = [&](int q) {
+        const int k = ic - base;
+        const RT w0 = lane_value(t0, k), w1 = lane_value(t1, k), w2 = lane_value(t2, k), w3 = lane_value(t3, k);
+#pragma unroll
+        for (int l = 0; l < NL; ++l)
+#pragma unroll
+            for (int m = 0; m < NC; ++m) {
+                const RT v = dot4<RT>(W[(q + 1) & 3][l][m], w0, W[(q + 2) & 3][l][m], w1, W[(q + 3) & 3][l][m], w2, W[q][l][m], w3);
+                const int kk = xw / 2 + m;
+                const long long o = bidx(p, min(kk, p.nxm), J0 + l, ic);
+                const double val = jb.mode == CM_LAT ? jb.scale * double(v) : double(v);
+                if (kk < p.nxm) out[o] = jb.accumulate ? out[o] + val : val;
+            }
+        // phic(nx) stays zero (phasefield.F90:476)
+        if (jb.mode != CM_LAT && xw == 0)
+#pragma unroll
+            for (int l = 0; l < NL; ++l) out[bidx(p, p.nxm, J0 + l, ic)] = 0.0;
+        ++ic;
+    };
+    for (; zr <= end; zr += 4) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (zr + q > end) break;
+            contract(q);
+            load(R[q % PD], H[q % PD]);
+            while (need == zr + q) {
+                emit(q);
+                if (ic >= I1) { need = end + 1; break; }
+                if (ic - base > 63) fill();
+                need = __builtin_amdgcn_readlane(tn, ic - base);
+            }
+        }
+    }
+}
+
 // index nxr of a refined field to zero
 template <typename RT>
 __global__ void __launch_bounds__(256) k_zero_tail(RT *f, int n, int ld, long long rows) {
