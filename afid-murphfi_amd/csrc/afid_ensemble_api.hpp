@@ -396,14 +396,14 @@ int afid_ens_init(const afid_config *cfgs, const afid_run_control *ctl, int32_t 
         if (e->mixed) {
             R.pff = c->pff;
             R.specf = static_cast<cpx<float> *>(c->spec);
-            R.planf = c->plan_zf;
+            R.planf = c->ens_zf;
             R.div_tol = c->div_tol;
             R.max_sweeps = c->max_sweeps;
             e->max_sweeps = std::max(e->max_sweeps, c->max_sweeps);
         } else {
             R.pf = c->pois;
             R.spec = static_cast<cpx<double> *>(c->spec);
-            R.plan = c->plan_z;
+            R.plan = c->ens_z;
             R.max_sweeps = 1;
         }
         for (int s = 0; s < 3; ++s) { R.gam[s] = c->gam[s]; R.rom[s] = c->rom[s]; R.alm[s] = c->alm[s]; }

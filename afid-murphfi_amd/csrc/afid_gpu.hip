@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <functional>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -155,9 +156,9 @@ struct afid_ctx {
     // Poisson
     FftPlan<double> plan_y, plan_z;
     FftPlan<float> plan_yf, plan_zf;
-    int Ly = 1, Lz = 1, lds_y = 0, lds_z = 0;
-    int fftz_maxv = FFT_MAXV;           // values per thread and stage of k_fft_z
-    bool fft_z16 = true;                // FP32 z transform may take 16 values per thread (AFID_FFT_Z16=0: no)
+    FftPlan<double> ens_z;              // the z transform of an ensemble member (lds_fft)
+    FftPlan<float> ens_zf;
+    int lgy = 0, lgz = 0, ty = 64, tz = 64, lds_y = 0, lds_z = 0;   // log2 of the lines, threads, LDS of a transform workgroup
     PoissonFactors<double> pois{};
     PoissonFactors<float> pff{};
     int pchunk = 1;
@@ -430,16 +431,31 @@ static int run_tri(afid_ctx *c, int kind, double *rhs, double *q, int keep = 1) 
 // ---------------------------------------------------------------------------
 // set-up
 // ---------------------------------------------------------------------------
+// The radices of n = 2^a 3^b from those in `from`, largest first: as few as
+// there can be, of those plans one with the smallest largest radix, and of
+// those one with the largest smallest.
+static bool pick_radices(int n, const std::vector<int> &from, std::vector<int> &best) {
+    std::vector<int> now;
+    std::function<void(int, size_t)> go = [&](int m, size_t at) {
+        if (m == 1) {
+            if (best.empty() || now.size() < best.size() || (now.size() == best.size() && (now[0] < best[0] || (now[0] == best[0] && now.back() > best.back())))) best = now;
+            return;
+        }
+        if (!best.empty() && now.size() >= best.size()) return;      // (another factor at least)
+        for (size_t q = at; q < from.size(); ++q)
+            if (m % from[q] == 0) { now.push_back(from[q]); go(m / from[q], q); now.pop_back(); }
+    };
+    go(n, 0);
+    return n == 1 || !best.empty();
+}
 template <typename R>
-static int build_plan(afid_ctx *c, int n, FftPlan<R> &pl) {
+static int build_plan(afid_ctx *c, int n, FftPlan<R> &pl, FftPlan<R> *ens = nullptr) {
     pl = FftPlan<R>{};
     pl.n = n;
-    int m = n;
-    while (m % 8 == 0 && m > 1) { pl.rad[pl.nst++] = 8; m /= 8; }
-    while (m % 4 == 0 && m > 1) { pl.rad[pl.nst++] = 4; m /= 4; }
-    while (m % 2 == 0 && m > 1) { pl.rad[pl.nst++] = 2; m /= 2; }
-    while (m % 3 == 0 && m > 1) { pl.rad[pl.nst++] = 3; m /= 3; }
-    if (m != 1 || pl.nst > 12) return set_err(c, AFID_E_ARG, "periodic size " + std::to_string(n) + " must factor into 2 and 3");
+    std::vector<int> rad;
+    if (!pick_radices(n, {16, 12, 9, 8, 6, 4, 3, 2}, rad) || rad.size() > FFT_STAGES)
+        return set_err(c, AFID_E_ARG, "periodic size " + std::to_string(n) + " must factor into 2 and 3");
+    for (int r : rad) pl.rad[pl.nst++] = r;
     std::vector<cpx<R>> tw((size_t)(n));
     for (int t = 0; t < n; ++t) {
         tw[size_t(t)].x = R(std::cos(2.0 * kPi * t / n));
@@ -448,18 +464,60 @@ static int build_plan(afid_ctx *c, int n, FftPlan<R> &pl) {
     const cpx<R> *d = nullptr;
     int rc = upload_vec(c, tw, &d);
     pl.tw = d;
+    if (ens) {
+        *ens = pl;
+        ens->nst = 0;
+        int m = n;
+        for (int r : {8, 4, 2, 3})
+            while (m % r == 0 && m > 1) { ens->rad[ens->nst++] = r; m /= r; }
+    }
     return rc;
 }
 
-// lines per transform workgroup (a power of two): L lines of N complex
-// values within the LDS budget and the per-thread register budget
-// (L*N <= FFT_MAXV*FFT_THREADS), at most cap
+// log2 of the lines per transform workgroup: as many as 1 << cap (128-byte
+// rows) within LDS and threads
 template <typename R>
-static int pick_lines(int N, int maxlds, int cap, int maxv = FFT_MAXV) {
-    int L = 1;
-    while (2 * L * line_stride<R>(N) * int(sizeof(cpx<R>)) <= maxlds && 2 * L * N <= maxv * FFT_THREADS && 2 * L <= cap)
-        L *= 2;
-    return L;
+static int pick_lines(const FftPlan<R> &pl, int maxlds, int cap) {
+    int lg = 0;
+    while (lg < cap && (pl.n << (lg + 1)) * int(sizeof(cpx<R>)) <= maxlds && fft_threads(pl.n, pl.nst, pl.rad, 2 << lg) <= FFT_MAXT) ++lg;
+    return lg;
+}
+// f with the kernels' bound on the threads: 512 in FP64 where that is enough
+template <typename R, typename F>
+static void with_threads(int threads, F f) {
+    if constexpr (sizeof(R) == 8)
+        if (threads <= 512) return f(std::integral_constant<int, 512>{});
+    f(std::integral_constant<int, FFT_MAXT>{});
+}
+template <typename R>
+static int plan_lines(afid_ctx *c, const FftPlan<R> &py, const FftPlan<R> &pz, int maxlds) {
+    // y: 1 << lgy complex lines = twice as many x-adjacent real ones (16 FP64
+    // velocity values a row)
+    c->lgy = pick_lines(py, maxlds, 3);
+    c->lgz = pick_lines(pz, maxlds, sizeof(R) == 8 ? 3 : 4);
+    c->ty = fft_threads(py.n, py.nst, py.rad, 1 << c->lgy);
+    c->tz = fft_threads(pz.n, pz.nst, pz.rad, 1 << c->lgz);
+    // The y transforms read and write their rows in loops beside the
+    // butterflies: 256 threads at least, 512 where there are at most two
+    // workgroups to a CU (20 steps at 64^3 FP64: 3840 us with the butterflies'
+    // 64 threads, 3490 with 256, 3460 with 512; 192 x 256^2, divergence and
+    // forward transform: 101 us a launch with 128, 97 with 256, 102 with 512).
+    const int nbx = (c->nxm + (2 << c->lgy) - 1) >> (c->lgy + 1);
+    c->ty = std::max(c->ty, std::min((py.n << c->lgy) / 64 * 64, (long long)nbx * c->nz <= 512 ? 512 : 256));
+    c->lds_y = (py.n << c->lgy) * int(sizeof(cpx<R>));
+    c->lds_z = (pz.n << c->lgz) * int(sizeof(cpx<R>));
+    const auto more = [](const void *k, int lds) { if (lds > 65536) (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, lds); };
+    with_threads<R>(c->ty, [&](auto mt) {
+        more(reinterpret_cast<const void *>(k_div_fft_y<R, decltype(mt)::value>), c->lds_y);
+        more(reinterpret_cast<const void *>(k_ifft_y<R, decltype(mt)::value>), c->lds_y);
+    });
+    with_threads<R>(c->tz, [&](auto mt) {
+        more(reinterpret_cast<const void *>(k_fft_z<R, -1, decltype(mt)::value>), c->lds_z);
+        more(reinterpret_cast<const void *>(k_fft_z<R, 1, decltype(mt)::value>), c->lds_z);
+    });
+    if (c->lds_y > maxlds || c->lds_z > maxlds || c->ny > 8192 || c->nz > 8192 || c->ty > FFT_MAXT || c->tz > FFT_MAXT)
+        return set_err(c, AFID_E_ARG, "periodic size too large for one workgroup transform");
+    return AFID_OK;
 }
 
 // LDS of k_to_coarse: two refined rows of each line
@@ -675,10 +733,10 @@ static int setup(afid_ctx *c) {
     // Poisson transforms and factors
     if (c->mixed) {
         if ((rc = build_plan(c, c->ny, c->plan_yf))) return rc;
-        if ((rc = build_plan(c, c->nz, c->plan_zf))) return rc;
+        if ((rc = build_plan(c, c->nz, c->plan_zf, &c->ens_zf))) return rc;
     } else {
         if ((rc = build_plan(c, c->ny, c->plan_y))) return rc;
-        if ((rc = build_plan(c, c->nz, c->plan_z))) return rc;
+        if ((rc = build_plan(c, c->nz, c->plan_z, &c->ens_z))) return rc;
     }
     int maxlds = 65536;
     {
@@ -686,38 +744,7 @@ static int setup(afid_ctx *c) {
         if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device) == hipSuccess && v > 0)
             maxlds = std::min(v, 160 * 1024);
     }
-    // y: Ly complex lines = 2*Ly x-adjacent real lines (16 FP64 velocity
-    // values = 128 bytes per row); z: Lz x-adjacent lines (128-byte rows)
-    if (c->mixed) {
-        c->Ly = pick_lines<float>(c->ny, maxlds, 8);
-        // 16 values per thread and stage (k_fft_z<float, 16>) when 8 would
-        // leave rows shorter than 16 lines (128 bytes)
-        c->Lz = pick_lines<float>(c->nz, maxlds, 16);
-        if (c->Lz < 16 && c->fft_z16) {
-            c->Lz = pick_lines<float>(c->nz, maxlds, 16, 16);
-            c->fftz_maxv = 16;
-        }
-        c->lds_y = c->Ly * line_stride<float>(c->ny) * csize;
-        c->lds_z = c->Lz * line_stride<float>(c->nz) * csize;
-    } else {
-        c->Ly = pick_lines<double>(c->ny, maxlds, 8);
-        c->Lz = pick_lines<double>(c->nz, maxlds, 8);
-        c->lds_y = c->Ly * line_stride<double>(c->ny) * csize;
-        c->lds_z = c->Lz * line_stride<double>(c->nz) * csize;
-    }
-    if (c->lds_y > 65536) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(k_div_fft_y<double>), hipFuncAttributeMaxDynamicSharedMemorySize, c->lds_y);
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(k_div_fft_y<float>), hipFuncAttributeMaxDynamicSharedMemorySize, c->lds_y);
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(k_ifft_y<double>), hipFuncAttributeMaxDynamicSharedMemorySize, c->lds_y);
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(k_ifft_y<float>), hipFuncAttributeMaxDynamicSharedMemorySize, c->lds_y);
-    }
-    if (c->lds_z > 65536) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(k_fft_z<double>), hipFuncAttributeMaxDynamicSharedMemorySize, c->lds_z);
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(k_fft_z<float>), hipFuncAttributeMaxDynamicSharedMemorySize, c->lds_z);
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(k_fft_z<float, 16>), hipFuncAttributeMaxDynamicSharedMemorySize, c->lds_z);
-    }
-    if (c->lds_y > maxlds || c->lds_z > maxlds || c->ny > FFT_MAXV * FFT_THREADS || c->nz > FFT_MAXV * FFT_THREADS)
-        return set_err(c, AFID_E_ARG, "periodic size too large for one workgroup transform");
+    if ((rc = c->mixed ? plan_lines(c, c->plan_yf, c->plan_zf, maxlds) : plan_lines(c, c->plan_y, c->plan_z, maxlds))) return rc;
     {
         c->pchunk = (nxm + 63) / 64;
         if (c->pchunk > 16) return set_err(c, AFID_E_ARG, "nxm above 1024 is not supported");
@@ -1038,7 +1065,6 @@ static int ctx_create(const afid_config *cfg, hipStream_t shared, afid_ctx **out
     }
     c->device = dev;
     if (const char *e = std::getenv("AFID_COLUMN_FOUR_PASS")) c->col_four_pass = std::atoi(e) != 0;
-    if (const char *e = std::getenv("AFID_FFT_Z16")) c->fft_z16 = std::atoi(e) != 0;
     if (shared) {
         c->stream = shared;
         c->own_stream = false;
@@ -1381,31 +1407,38 @@ int afid_update_saturation(afid_ctx *c) {
 // the rest; slot_out receives max|div u| of a velocity source.
 // z transform of the spectrum (k_fft_z; the FP32 form may take 16 values per
 // thread and stage, see setup)
-template <typename R>
-static void launch_fft_z(afid_ctx *c, const KP &p, const FftPlan<R> &pz, cpx<R> *spec, int sign, Gate gate) {
-    const dim3 gr(unsigned((c->nxm + c->Lz - 1) / c->Lz), unsigned(c->nymh));
-    if constexpr (sizeof(R) == sizeof(float)) {
-        if (c->fftz_maxv == 16) {
-            hipLaunchKernelGGL((k_fft_z<R, 16>), gr, dim3(FFT_THREADS), c->lds_z, c->stream, p, pz, spec, c->Lz, sign, gate);
-            return;
-        }
-    }
-    hipLaunchKernelGGL((k_fft_z<R>), gr, dim3(FFT_THREADS), c->lds_z, c->stream, p, pz, spec, c->Lz, sign, gate);
+template <typename R, int SIGN>
+static void launch_fft_z(afid_ctx *c, const KP &p, const FftPlan<R> &pz, cpx<R> *spec, Gate gate) {
+    const dim3 gr(unsigned((c->nxm + (1 << c->lgz) - 1) >> c->lgz), unsigned(c->nymh));
+    with_threads<R>(c->tz, [&](auto mt) {
+        hipLaunchKernelGGL((k_fft_z<R, SIGN, decltype(mt)::value>), gr, dim3(unsigned(c->tz)), c->lds_z, c->stream, p, pz, spec, c->lgz, gate);
+    });
 }
+// us a launch: floor (the arrays once at 5.2 TB/s), the lines in LDS from load
+// to store with 1024 threads before, afid_fft.hpp now (k_div_fft_y / k_fft_z /
+// k_ifft_y):
+//   64^3 FP64                 4 / 2 / 2       8.3 / 9.4 / 5.8   8.3 / 5.7 / 5.5
+//   192 x 256^2 FP64         77 / 39 / 39     160 / 90 / 85     97 / 45 / 43
+//   384 x 192^2 FP64         88 / 44 / 44     191 / 118 / 110   110 / 47 / 48
+//   384 x 384^2 FP32, all sweeps of a substep     622 / 2 x 280 / 341   428 / 2 x 180 / 223
+// The divergence is read in a loop with few registers and little code, not by
+// the first stage's butterflies (64^3: 12.2 us a launch, 192 x 256^2 110).
 template <typename R>
 static int poisson_sweep(afid_ctx *c, const FftPlan<R> &py, const FftPlan<R> &pz, const PoissonFactors<R> &pf, int src,
                          Gate fwd_gate, Gate gate, unsigned long long *slot_out, unsigned long long *clear) {
     KP p = make_kp(c);
     cpx<R> *spec = static_cast<cpx<R> *>(c->spec);
-    const int TXy = 2 * c->Ly;
+    const int nbx = (c->nxm + (2 << c->lgy) - 1) >> (c->lgy + 1);
     tstart(c, "poisson_fwd_y");
-    hipLaunchKernelGGL(k_div_fft_y<R>, dim3(unsigned((c->nxm + TXy - 1) / TXy), unsigned(c->nz)), dim3(FFT_THREADS), c->lds_y,
-                       c->stream, p, py, spec, c->Ly, src, fwd_gate, slot_out, clear);
+    with_threads<R>(c->ty, [&](auto mt) {
+        hipLaunchKernelGGL((k_div_fft_y<R, decltype(mt)::value>), dim3(tile_grid((long long)nbx * c->nz)), dim3(unsigned(c->ty)), c->lds_y,
+                           c->stream, p, py, spec, c->lgy, nbx, src, fwd_gate, slot_out, clear);
+    });
     tstop(c);
     int rc = check_launch(c, "k_div_fft_y");
     if (rc) return rc;
     tstart(c, "poisson_fft_z");
-    launch_fft_z<R>(c, p, pz, spec, -1, gate);
+    launch_fft_z<R, -1>(c, p, pz, spec, gate);
     tstop(c);
     if ((rc = check_launch(c, "k_fft_z"))) return rc;
     tstart(c, "poisson_tridiag");
@@ -1419,12 +1452,13 @@ static int poisson_sweep(afid_ctx *c, const FftPlan<R> &py, const FftPlan<R> &pz
     tstop(c);
     if ((rc = check_launch(c, "k_poisson_tri"))) return rc;
     tstart(c, "poisson_fft_z");
-    launch_fft_z<R>(c, p, pz, spec, +1, gate);
+    launch_fft_z<R, 1>(c, p, pz, spec, gate);
     tstop(c);
     if ((rc = check_launch(c, "k_fft_z"))) return rc;
     tstart(c, "poisson_inv_y");
-    hipLaunchKernelGGL(k_ifft_y<R>, dim3(unsigned((c->nxm + TXy - 1) / TXy), unsigned(c->nz)), dim3(FFT_THREADS), c->lds_y,
-                       c->stream, p, py, spec, c->Ly, gate);
+    with_threads<R>(c->ty, [&](auto mt) {
+        hipLaunchKernelGGL((k_ifft_y<R, decltype(mt)::value>), dim3(unsigned(nbx), unsigned(c->nz)), dim3(unsigned(c->ty)), c->lds_y, c->stream, p, py, spec, c->lgy, gate);
+    });
     tstop(c);
     return check_launch(c, "k_ifft_y");
 }

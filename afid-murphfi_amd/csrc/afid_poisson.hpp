@@ -4,8 +4,7 @@
 //
 // Transforms run along the strided y and z directions with the contiguous x
 // direction mapped to lanes, so every global access is a run of x-adjacent
-// values; a workgroup holds L lines of length N in LDS and runs a
-// mixed-radix (8,4,3,2) Stockham transform on them.  The real y transform
+// values; a workgroup takes L lines (afid_fft.hpp).  The real y transform
 // packs two x-adjacent real lines into one complex line.
 //
 // Spectral layout: S[i][m][k] (complex, k = x fastest), m = 0..ny/2,
@@ -16,94 +15,13 @@
 #include "afid_params.hpp"
 #include "afid_stencils.hpp"
 #include "afid_kernels.hpp"
+#include "afid_fft.hpp"
 
 namespace afid {
 
-// complex value of real type R (double in the FP64 form, float in the mixed form)
-template <typename R>
-struct __align__(2 * sizeof(R)) cpx { R x, y; };
-template <typename R>
-__device__ __forceinline__ cpx<R> mk(R a, R b) { cpx<R> z; z.x = a; z.y = b; return z; }
-
-template <typename R>
-struct FftPlan {
-    int n = 1;
-    int nst = 0;
-    int rad[12] = {0};
-    const cpx<R> *tw = nullptr;   // exp(-2 pi i t/n), t = 0..n-1
-};
-
-template <typename R>
-__device__ __forceinline__ cpx<R> cmul(cpx<R> a, cpx<R> b) { return mk<R>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
-template <typename R>
-__device__ __forceinline__ cpx<R> cadd(cpx<R> a, cpx<R> b) { return mk<R>(a.x + b.x, a.y + b.y); }
-template <typename R>
-__device__ __forceinline__ cpx<R> csub(cpx<R> a, cpx<R> b) { return mk<R>(a.x - b.x, a.y - b.y); }
-// multiply by i*sign
-template <typename R>
-__device__ __forceinline__ cpx<R> cmulis(cpx<R> a, int sign) { return sign < 0 ? mk<R>(a.y, -a.x) : mk<R>(-a.y, a.x); }
-
-template <int N, typename R>
-struct DftSmall;
-template <typename R>
-struct DftSmall<2, R> {
-    static __device__ __forceinline__ void run(cpx<R> (&v)[2], int) {
-        cpx<R> a = v[0], b = v[1];
-        v[0] = cadd(a, b); v[1] = csub(a, b);
-    }
-};
-template <typename R>
-struct DftSmall<3, R> {
-    static __device__ __forceinline__ void run(cpx<R> (&v)[3], int sign) {
-        const R s3 = R(0.86602540378443864676);   // sin(2 pi/3)
-        cpx<R> t1 = cadd(v[1], v[2]), t2 = csub(v[1], v[2]);
-        cpx<R> m = mk<R>(v[0].x - R(0.5) * t1.x, v[0].y - R(0.5) * t1.y);
-        cpx<R> r = cmulis(mk<R>(s3 * t2.x, s3 * t2.y), sign);
-        v[0] = cadd(v[0], t1);
-        v[1] = cadd(m, r);
-        v[2] = csub(m, r);
-    }
-};
-template <typename R>
-struct DftSmall<4, R> {
-    static __device__ __forceinline__ void run(cpx<R> (&v)[4], int sign) {
-        cpx<R> a = cadd(v[0], v[2]), b = csub(v[0], v[2]), c = cadd(v[1], v[3]), d = cmulis(csub(v[1], v[3]), sign);
-        v[0] = cadd(a, c); v[2] = csub(a, c);
-        v[1] = cadd(b, d); v[3] = csub(b, d);
-    }
-};
-template <typename R>
-struct DftSmall<8, R> {
-    static __device__ __forceinline__ void run(cpx<R> (&v)[8], int sign) {
-        const R h = R(0.70710678118654752440);    // 1/sqrt(2)
-        cpx<R> e[4] = {v[0], v[2], v[4], v[6]}, o[4] = {v[1], v[3], v[5], v[7]};
-        DftSmall<4, R>::run(e, sign);
-        DftSmall<4, R>::run(o, sign);
-        // w8^k = exp(sign 2 pi i k/8)
-        cpx<R> w1 = mk<R>(h, R(sign) * h), w3 = mk<R>(-h, R(sign) * h);
-        cpx<R> t0 = o[0], t1 = cmul(o[1], w1), t2 = cmulis(o[2], sign), t3 = cmul(o[3], w3);
-        v[0] = cadd(e[0], t0); v[4] = csub(e[0], t0);
-        v[1] = cadd(e[1], t1); v[5] = csub(e[1], t1);
-        v[2] = cadd(e[2], t2); v[6] = csub(e[2], t2);
-        v[3] = cadd(e[3], t3); v[7] = csub(e[3], t3);
-    }
-};
-
-// Workgroup size of the transform kernels and the most complex values a
-// thread holds in a stage (L*N <= FFT_MAXV*FFT_THREADS): 16 wavefronts whose
-// butterflies of a stage stay in registers between its read and write phase.
-constexpr int FFT_THREADS = 1024, FFT_MAXV = 8;
-
-// Division by a workgroup-uniform d through one multiply: whenever x * d <=
-// 2^32, floor(x / d) = umulhi(x, ceil(2^32 / d)) (the error term, below
-// x / 2^32 <= 1/d, never reaches the next integer, since frac(x/d) <= 1 - 1/d).
-// d = 1 is passed through.
-struct FastDiv {
-    unsigned d, m;
-    __device__ __forceinline__ explicit FastDiv(unsigned d_) : d(d_), m(d_ > 1 ? 0xFFFFFFFFu / d_ + 1u : 0u) {}
-    __device__ __forceinline__ unsigned div(unsigned x) const { return d == 1 ? x : __umulhi(x, m); }
-};
-
+// Transform of an ensemble member's lines, held in LDS from the first stage to
+// the last.
+//
 // LDS layout of L lines of N complex values: element j of line l sits at
 // l*S + lpad(j), with one pad element per 32 banks of data (16 FP32 or 8
 // FP64 complex values) so the stride-R writes of a Stockham stage spread
@@ -115,7 +33,7 @@ template <typename R>
 __host__ __device__ __forceinline__ int line_stride(int n) { return lpad<R>(n) + 1; }
 
 // One Stockham stage of radix RD over L lines of length N held in LDS, by
-// the NT threads of the workgroup (L*N <= FFT_MAXV*NT).  Each thread keeps
+// the NT threads of the workgroup (L*N <= MAXV*NT).  Each thread keeps
 // at most MAXB butterflies of the stage in registers between the read and
 // the write phase, so the transform runs in place.
 template <int RD, int MAXB, typename R, int NT>
@@ -154,10 +72,10 @@ __device__ __forceinline__ void fft_stage(cpx<R> *buf, int L, int N, int S, int 
     __syncthreads();
 }
 
-// Full transform of L lines (L*N <= FFT_MAXV*NT), line stride S, by a
-// workgroup of NT threads.
-// MAXV: the most complex values a thread holds in a stage (L*N <= MAXV*NT).
-template <typename R, int NT = FFT_THREADS, int MAXV = FFT_MAXV>
+// Full transform of L lines (L*N <= MAXV*NT), line stride S, radices 8, 4, 2
+// and 3, by a workgroup of NT threads.
+// MAXV: the most complex values a thread holds in a stage.
+template <typename R, int NT, int MAXV>
 __device__ __forceinline__ void lds_fft(cpx<R> *buf, int L, int S, const FftPlan<R> &pl, int sign) {
     int Ns = 1;
     for (int s = 0; s < pl.nst; ++s) {
@@ -179,109 +97,105 @@ enum PoissonSrc { SRC_VELOCITY = 0, SRC_DPH = 1 };
 // forward y transform (pressure.F90:171-174) and the 1/(ny nz) scaling.
 // With slot_out, the maximum of |div u| (CheckDivergence units) is also
 // reduced into *slot_out; with slots_clear, workgroup 0 zeroes 4 slots.
-// Block: 2L x-adjacent real lines at one z.  grid (ceil(nxm/2L), nz).
-template <typename R>
-__global__ void __launch_bounds__(FFT_THREADS) k_div_fft_y(KP p, FftPlan<R> pl, cpx<R> *spec, int L, int src, Gate gate,
-                                                           unsigned long long *slot_out, unsigned long long *slots_clear) {
+// Workgroup: 2L x-adjacent real lines (L = 1 << lg complex ones) at one z;
+// those of one z, and neighbouring z, whose planes of vz are the same, on one
+// XCD.  nbx = ceil(nxm / 2L) workgroups per z.
+template <typename R, int MT>
+__global__ void __launch_bounds__(MT, fft_waves(MT)) k_div_fft_y(KP p, FftPlan<R> pl, cpx<R> *spec, int lg, int nbx, int src, Gate gate,
+                                                        unsigned long long *slot_out, unsigned long long *slots_clear) {
     if (gate_closed(gate)) return;
     extern __shared__ __align__(16) unsigned char smraw[];
     cpx<R> *lb = reinterpret_cast<cpx<R> *>(smraw);
-    const int N = p.ny, S = line_stride<R>(N), TX = 2 * L, i = blockIdx.y, k0 = blockIdx.x * TX;
+    if (slots_clear && blockIdx.x == 0 && threadIdx.x < 4) slots_clear[threadIdx.x] = 0ull;
+    const int item = int(xcd_block(0));
+    if (item >= nbx * p.nz) return;
+    const int N = p.ny, i = item / nbx, k0 = (item - i * nbx) << (lg + 1);
     const int ip = wrapp(i, p.nz);
     const double usdtal = 1.0 / (p.dt * p.al);
-    if (slots_clear && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 4) slots_clear[threadIdx.x] = 0ull;
     double dmax = 0.0;
-    const FastDiv dtx(TX);
-    for (int t = threadIdx.x; t < TX * N; t += FFT_THREADS) {
-        const int j = dtx.div(t), xo = t - j * TX, k = k0 + xo;
-        double d = 0.0;
-        if (k < p.nxm) {
-            if (src == SRC_DPH) d = p.dph[bidx(p, k, j, i)];
-            else {
-                const int jp = wrapp(j, N);
-                const double dv = (p.vz[bidx(p, k, j, ip)] - p.vz[bidx(p, k, j, i)]) * p.dz
-                                + (p.vy[bidx(p, k, jp, i)] - p.vy[bidx(p, k, j, i)]) * p.dy
-                                + (p.vx[bidx(p, k + 1, j, i)] - p.vx[bidx(p, k, j, i)]) * p.udx3m[k];
-                dmax = fmax(dmax, fabs(dv));
-                d = dv * usdtal;
-            }
-        }
-        R *slot = reinterpret_cast<R *>(&lb[(xo >> 1) * S + lpad<R>(j)]);
-        slot[xo & 1] = R(d);
-    }
+    using P2 = double __attribute__((ext_vector_type(2)));
+    const double *vz0 = p.vz + (long long)i * p.plane, *vz1 = p.vz + (long long)ip * p.plane;
+    const double *vy0 = p.vy + (long long)i * p.plane, *vx0 = p.vx + (long long)i * p.plane, *dp0 = p.dph + (long long)i * p.plane;
+    const auto ld = [&](int line, int j) {
+        const int k = k0 + 2 * line;
+        if (k >= p.nxm) return mk<R>(R(0), R(0));
+        const bool two = k + 1 < p.nxm;
+        const int o = j * p.ldx + k;
+        if (src == SRC_DPH) return mk<R>(R(dp0[o]), two ? R(dp0[o + 1]) : R(0));
+        const P2 z1 = *reinterpret_cast<const P2 *>(vz1 + o), z0 = *reinterpret_cast<const P2 *>(vz0 + o);
+        const P2 y1 = *reinterpret_cast<const P2 *>(vy0 + wrapp(j, N) * p.ldx + k), y0 = *reinterpret_cast<const P2 *>(vy0 + o);
+        const P2 x0 = *reinterpret_cast<const P2 *>(vx0 + o);
+        const double x2 = vx0[o + (two ? 2 : 1)];
+        const double da = (z1[0] - z0[0]) * p.dz + (y1[0] - y0[0]) * p.dy + (x0[1] - x0[0]) * p.udx3m[k];
+        const double db = two ? (z1[1] - z0[1]) * p.dz + (y1[1] - y0[1]) * p.dy + (x2 - x0[1]) * p.udx3m[k + 1] : 0.0;
+        dmax = fmax(dmax, fmax(fabs(da), fabs(db)));
+        return mk<R>(R(da * usdtal), R(db * usdtal));
+    };
+    for (int t = threadIdx.x; t < N << lg; t += blockDim.x) lb[t] = ld(t & ((1 << lg) - 1), t >> lg);
+    __syncthreads();
+    fft_lines<-1, true, true>(lb, lg, pl, [&](int line, int j) { return lb[(j << lg) + line]; },
+                              [&](int line, int j, cpx<R> v) { lb[(j << lg) + line] = v; });
     if (slot_out) {
         dmax = block_max(dmax);
         max_to_slot(slot_out, dmax);
     }
-    __syncthreads();
-    lds_fft<R>(lb, L, S, pl, -1);
     const R scale = R(1.0 / (double(p.ny) * double(p.nz)));
-    for (int t = threadIdx.x; t < TX * p.nymh; t += FFT_THREADS) {
-        const int m = dtx.div(t), xo = t - m * TX, k = k0 + xo;
+    for (int t = threadIdx.x; t < p.nymh << lg; t += blockDim.x) {
+        const int line = t & ((1 << lg) - 1), m = t >> lg, k = k0 + 2 * line;
         if (k >= p.nxm) continue;
-        const int line = xo >> 1;
-        const cpx<R> zm = lb[line * S + lpad<R>(m)], zn = lb[line * S + lpad<R>(m == 0 ? 0 : N - m)];
-        cpx<R> out;
-        if ((xo & 1) == 0) out = mk<R>(R(0.5) * (zm.x + zn.x), R(0.5) * (zm.y - zn.y));     // (Z_m + conj Z_{N-m})/2
-        else out = mk<R>(R(0.5) * (zm.y + zn.y), R(-0.5) * (zm.x - zn.x));                  // (Z_m - conj Z_{N-m})/(2i)
-        spec[((long long)i * p.nymh + m) * p.nxm + k] = mk<R>(out.x * scale, out.y * scale);
+        const cpx<R> zm = lb[(m << lg) + line], zn = lb[((m == 0 ? 0 : N - m) << lg) + line];
+        cpx<R> *o = spec + ((long long)i * p.nymh + m) * p.nxm + k;
+        // (Z_m + conj Z_{N-m})/2 and (Z_m - conj Z_{N-m})/(2i)
+        o[0] = mk<R>(R(0.5) * (zm.x + zn.x) * scale, R(0.5) * (zm.y - zn.y) * scale);
+        if (k + 1 < p.nxm) o[1] = mk<R>(R(0.5) * (zm.y + zn.y) * scale, R(-0.5) * (zm.x - zn.x) * scale);
     }
 }
 
 // Complex transform along z (pressure.F90:176 forward, :189 backward), in
-// place on the spectral array.  Block: L x-adjacent lines at one y-mode m.
-// MAXV: complex values per thread and stage (L*N <= MAXV*FFT_THREADS); 16
-// lets the FP32 form take 16 x-adjacent lines (128-byte rows) at N = 768.
-template <typename R, int MAXV = FFT_MAXV>
-__global__ void __launch_bounds__(FFT_THREADS) k_fft_z(KP p, FftPlan<R> pl, cpx<R> *spec, int L, int sign, Gate gate) {
+// place on the spectral array.  Workgroup: L = 1 << lg x-adjacent lines at one
+// y-mode m.
+template <typename R, int SIGN, int MT>
+__global__ void __launch_bounds__(MT, fft_waves(MT)) k_fft_z(KP p, FftPlan<R> pl, cpx<R> *spec, int lg, Gate gate) {
     if (gate_closed(gate)) return;
     extern __shared__ __align__(16) unsigned char smraw[];
     cpx<R> *lb = reinterpret_cast<cpx<R> *>(smraw);
-    const int N = p.nz, S = line_stride<R>(N), m = blockIdx.y, k0 = blockIdx.x * L;
+    const int m = blockIdx.y, k0 = blockIdx.x << lg;
     const long long sz = (long long)p.nymh * p.nxm;
-    cpx<R> *g = spec + (long long)m * p.nxm;
-    const FastDiv dl(L);
-    for (int t = threadIdx.x; t < L * N; t += FFT_THREADS) {
-        const int i = dl.div(t), xo = t - i * L, k = k0 + xo;
-        lb[xo * S + lpad<R>(i)] = k < p.nxm ? g[i * sz + k] : mk<R>(R(0), R(0));
-    }
-    __syncthreads();
-    lds_fft<R, FFT_THREADS, MAXV>(lb, L, S, pl, sign);
-    for (int t = threadIdx.x; t < L * N; t += FFT_THREADS) {
-        const int i = dl.div(t), xo = t - i * L, k = k0 + xo;
-        if (k < p.nxm) g[i * sz + k] = lb[xo * S + lpad<R>(i)];
-    }
+    cpx<R> *g = spec + (long long)m * p.nxm + k0;
+    const int left = p.nxm - k0;
+    fft_lines<SIGN, false, false>(lb, lg, pl,
+        [&](int line, int i) { return line < left ? g[i * sz + line] : mk<R>(R(0), R(0)); },
+        [&](int line, int i, cpx<R> v) { if (line < left) g[i * sz + line] = v; });
 }
 
 // Inverse real y transform (pressure.F90:193-195): two x-adjacent spectra
 // A, B (Hermitian, imaginary parts of the m=0 and m=N/2 terms ignored as a
 // c2r transform does) become Z = A + iB, whose inverse is a + ib, written
 // to dph.
-template <typename R>
-__global__ void __launch_bounds__(FFT_THREADS) k_ifft_y(KP p, FftPlan<R> pl, const cpx<R> *spec, int L, Gate gate) {
+template <typename R, int MT>
+__global__ void __launch_bounds__(MT, fft_waves(MT)) k_ifft_y(KP p, FftPlan<R> pl, const cpx<R> *spec, int lg, Gate gate) {
     if (gate_closed(gate)) return;
     extern __shared__ __align__(16) unsigned char smraw[];
     cpx<R> *lb = reinterpret_cast<cpx<R> *>(smraw);
-    const int N = p.ny, S = line_stride<R>(N), TX = 2 * L, i = blockIdx.y, k0 = blockIdx.x * TX;
-    const FastDiv dl(L), dtx(TX);
-    for (int t = threadIdx.x; t < L * p.nymh; t += FFT_THREADS) {
-        const int m = dl.div(t), line = t - m * L;
-        const int ka = k0 + 2 * line, kb = ka + 1;
-        const cpx<R> *row = spec + ((long long)i * p.nymh + m) * p.nxm;
-        cpx<R> A = ka < p.nxm ? row[ka] : mk<R>(R(0), R(0));
-        cpx<R> B = kb < p.nxm ? row[kb] : mk<R>(R(0), R(0));
+    const int N = p.ny, i = blockIdx.y, k0 = blockIdx.x << (lg + 1);
+    for (int t = threadIdx.x; t < p.nymh << lg; t += blockDim.x) {
+        const int line = t & ((1 << lg) - 1), m = t >> lg, k = k0 + 2 * line;
+        const cpx<R> *row = spec + ((long long)i * p.nymh + m) * p.nxm + k;
+        cpx<R> A = k < p.nxm ? row[0] : mk<R>(R(0), R(0));
+        cpx<R> B = k + 1 < p.nxm ? row[1] : mk<R>(R(0), R(0));
         if (m == 0 || 2 * m == N) { A.y = R(0); B.y = R(0); }
-        lb[line * S + lpad<R>(m)] = mk<R>(A.x - B.y, A.y + B.x);
-        if (m > 0 && N - m > m) lb[line * S + lpad<R>(N - m)] = mk<R>(A.x + B.y, B.x - A.y);
+        lb[(m << lg) + line] = mk<R>(A.x - B.y, A.y + B.x);
+        if (m > 0 && N - m > m) lb[((N - m) << lg) + line] = mk<R>(A.x + B.y, B.x - A.y);
     }
     __syncthreads();
-    lds_fft<R>(lb, L, S, pl, +1);
-    for (int t = threadIdx.x; t < TX * N; t += FFT_THREADS) {
-        const int j = dtx.div(t), xo = t - j * TX, k = k0 + xo;
-        if (k >= p.nxm) continue;
-        const cpx<R> z = lb[(xo >> 1) * S + lpad<R>(j)];
-        sel<R>(p.dph, p.dphf)[bidx(p, k, j, i)] = (xo & 1) ? z.y : z.x;      // dph in the sweep's arithmetic R
-    }
+    R *out = sel<R>(p.dph, p.dphf) + (long long)i * p.plane + k0;       // dph in the sweep's arithmetic R
+    fft_lines<1, true, false>(lb, lg, pl, [&](int line, int j) { return lb[(j << lg) + line]; },
+        [&](int line, int j, cpx<R> z) {
+            const int k = k0 + 2 * line;
+            R *o = out + (long long)j * p.ldx + 2 * line;
+            if (k + 1 < p.nxm) *reinterpret_cast<cpx<R> *>(o) = z;
+            else if (k < p.nxm) *o = z.x;
+        });
 }
 
 // Per-mode wall-normal tridiagonal (SolveTridiagonalPressure,
