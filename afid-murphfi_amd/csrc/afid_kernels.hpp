@@ -754,10 +754,13 @@ __global__ void __launch_bounds__(256) k_project(KP p, int do_vel, int do_pr, Ga
 // velocity and dph): the FP64 residual of the mixed form's iterative
 // refinement, max-reduced into *slot (CheckDivergence units).  Each thread
 // marches along z over PROJ_ZC planes and carries dph and vz of the planes
-// i-1, i, i+1 in registers, so no plane is read twice.
+// i-1, i, i+1 in registers, so no plane is read twice.  A workgroup's maximum
+// goes straight to the slot: 32 768 of them cost nothing at 256 x 512^2 (project
+// 3672 us a step; with partial maxima and a kernel over them 3690), and at 64^3
+// the second launch was 5 us of every substep.
 constexpr int PROJ_ZC = 8;
 __global__ void __launch_bounds__(256) k_project_res(KP p, double *vx_out, double *vy_out, double *vz_out,
-                                                     double *partial) {
+                                                     unsigned long long *slot) {
     const int k = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y;
     const int i0 = blockIdx.z * PROJ_ZC, i1 = min(i0 + PROJ_ZC, p.nz);
     double dvm = 0.0;
@@ -801,17 +804,7 @@ __global__ void __launch_bounds__(256) k_project_res(KP p, double *vx_out, doubl
             d_m = d_c; d_c = d_p; w_c = w_p;
         }
     }
-    dvm = block_max(dvm);
-    if (threadIdx.x == 0 && threadIdx.y == 0)
-        partial[((long long)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = dvm;
-}
-// max of n per-workgroup partial maxima into *slot (grid-stride, one atomic
-// per workgroup of a small grid)
-__global__ void __launch_bounds__(256) k_max_partials(const double *partial, long long n, unsigned long long *slot) {
-    double v = 0.0;
-    for (long long q = (long long)blockIdx.x * 256 + threadIdx.x; q < n; q += (long long)gridDim.x * 256) v = fmax(v, partial[q]);
-    v = block_max(v);
-    if (threadIdx.x == 0) atomicMax(slot, (unsigned long long)__double_as_longlong(v));
+    max_to_slot(slot, block_max(dvm));
 }
 
 // ---------------------------------------------------------------------------
