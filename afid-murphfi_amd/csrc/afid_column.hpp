@@ -198,6 +198,8 @@ __global__ void __launch_bounds__(64 * NW) k_column_base_reg(KP p, BaseConst<HT>
     constexpr int CPB = col_per_block<LPC, NW>(), SB = COL_STRIP / CPB;
     const unsigned nxm = p.nxm, rmax = p.ldx - 2;
     const bool use_bref = sizeof(HT) == 4 && p.bref;
+    // (without salinity bycs, formed from parameters nobody set, may be infinite or NaN)
+    const HT bycs = p.active_s == 1 ? HT(p.bycs) : HT(0);
     const bool lo_lane = l == 0, hi_lane = l == LPC - 1;
     // rows r, r+1 of a table (the global metrics end at row ldx, the factors hold whole groups)
     auto tp = [&](int q, unsigned r) {
@@ -289,7 +291,7 @@ __global__ void __launch_bounds__(64 * NW) k_column_base_reg(KP p, BaseConst<HT>
                     // FP32 terms: buoyancy as its deviation from the row's FP64 reference
                     if (use_bref) h += HT(p.byct * (p.active_t * 0.5 * (AFID_E(t) + AFID_E(tk))) - AFID_E(bref));
                     else h += HT(p.byct) * (HT(p.active_t) * HT(0.5) * (HT(AFID_E(t)) + HT(AFID_E(tk))));
-                    h -= HT(p.bycs) * AFID_E(sal);
+                    h -= bycs * AFID_E(sal);
                 }
                 const double br = AFID_E(bref), px = (AFID_E(q) - AFID_E(qk)) * (p.al * AFID_E(u3c));
                 const double dxx = AFID_E(xn) * AFID_E(apc) + AFID_E(x) * (-AFID_E(apc) - AFID_E(amc)) + AFID_E(xk) * AFID_E(amc);
@@ -326,7 +328,7 @@ __global__ void __launch_bounds__(64 * NW) k_column_base_reg(KP p, BaseConst<HT>
                 HT h = -(hyx + hyy + hyz) + (vjp_ - HT(2.0) * vc + vjm_) * k.dyqr + (vip_ - HT(2.0) * vc + vim_) * k.dzqr + HT(p.Gy);
                 if (p.gaxis == 2) {
                     h += HT(p.byct) * (HT(p.active_t) * HT(0.5) * (HT(AFID_E(t)) + HT(AFID_E(gt))));
-                    h -= HT(p.bycs) * AFID_E(sal);
+                    h -= bycs * AFID_E(sal);
                 }
                 const double ap = AFID_E(aps), ac = AFID_E(acs), am = AFID_E(ams);
                 const double dxv = (kh[e] ? -(ac + am) * p.xplusu * p.inslwn : dn * ap) + AFID_E(v) * ac + (kl[e] ? -(ac + ap) * p.xminusu * p.inslws : dk * am);
@@ -359,7 +361,7 @@ __global__ void __launch_bounds__(64 * NW) k_column_base_reg(KP p, BaseConst<HT>
                 HT h = -(hzx + hzy + hzz) + (wip_ - HT(2.0) * wc_ + wim_) * k.dzqr + (wjp_ - HT(2.0) * wc_ + wjm_) * k.dyqr;
                 if (p.gaxis == 3) {
                     h += HT(p.byct) * (HT(p.active_t) * HT(0.5) * (HT(AFID_E(t)) + HT(AFID_E(gt))));
-                    h -= HT(p.bycs) * AFID_E(sal);
+                    h -= bycs * AFID_E(sal);
                 }
                 const double dxw = dn * AFID_E(aps) + AFID_E(w) * AFID_E(acs) + dk * AFID_E(ams);
                 d[2][e] = wc[e] ? (p.ga * double(h) + p.ro * double(AFID_E(oz)) + k.alren * dxw - (AFID_E(q) - AFID_E(qim)) * p.dz * p.al) * p.dt : 0.0;
