@@ -1576,7 +1576,7 @@ static void launch_xfer_yz(afid_ctx *c, XferJob &jb) {
     const long long nch = (jb.nx + 64 * NR - 1) / (64 * NR), ngr = (jb.nO + NL - 1) / NL, waves = nch * ngr;
     jb.nseg = 1;
     while (jb.nseg < 8 && waves * jb.nseg < (SUM ? 1024 : 2048)) jb.nseg *= 2;
-    const size_t lds = SUM && jb.nseg > 1 ? sizeof(RT) * NR * 64 * NL * size_t(jb.nseg) : 0;
+    const size_t lds = SUM && jb.nseg > 1 ? sizeof(double) * NR * 64 * NL * size_t(jb.nseg) : 0;
     if (jb.nseg > 1)
         hipLaunchKernelGGL((k_xfer_yz<RT, NR, NL, SUM, true>), dim3(tile_grid(waves)), dim3(64u * unsigned(jb.nseg)), lds, c->stream, jb);
     else

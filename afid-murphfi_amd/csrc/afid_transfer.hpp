@@ -167,13 +167,18 @@ __device__ __forceinline__ double lane_value(double v, int k) {
 // NL adjacent refined lines per wavefront (their sources span NL + 3 coarse
 // lines), NR refined x per lane.  SUM: the walk carries the sum (vyr, vzr).
 // With nseg > 1 a workgroup's wavefronts share one walk: each takes a range
-// of refined steps; for a sum they first add up their ranges.
+// of refined steps; for a sum they first add up their ranges.  The sum runs in
+// FP64 also for FP32 fields: an FP32 one rounds the whole value at every step
+// (a mean flow of 350 drifts by 2e-4 over 288 steps instead of one rounding of
+// 1.5e-5) and left vyr, vzr of a flow without a mean 6% further from FP64.  It
+// takes no longer (384 x 384^2 -> 768^3: 3.01 ms a step both).
 template <typename RT, int NR, int NL, bool SUM, bool SEG>
 __global__ void __launch_bounds__(SEG ? 512 : 256) k_xfer_yz(XferJob jb) {
     using V = typename XVec<RT, NR>::V;
+    using VS = typename XVec<std::conditional_t<SUM, double, RT>, NR>::V;     // value of a refined step
     constexpr int NU = NL + 3, PD = 4;                           // coarse lines; coarse steps loaded ahead
-    extern __shared__ __align__(16) unsigned char smraw[];
-    V *tot = reinterpret_cast<V *>(smraw);                       // [seg][line][lane]
+    extern __shared__ __align__(32) unsigned char smraw[];
+    VS *tot = reinterpret_cast<VS *>(smraw);                     // [seg][line][lane]
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nch = (jb.nx + 64 * NR - 1) / (64 * NR), ngr = (jb.nO + NL - 1) / NL;
     // x chunks fastest: neighbouring wavefronts write one row
@@ -201,14 +206,14 @@ __global__ void __launch_bounds__(SEG ? 512 : 256) k_xfer_yz(XferJob jb) {
     RT *out[NL];
 #pragma unroll
     for (int l = 0; l < NL; ++l) out[l] = static_cast<RT *>(jb.out) + min(l0 + l, jb.nO - 1) * jb.ro + x;
-    const RT dl = RT(jb.dl);
-    auto put = [&](int s, const V (&v)[NL]) {
+    const double dl = jb.dl;
+    auto put = [&](int s, const VS (&v)[NL]) {
 #pragma unroll
-        for (int l = 0; l < NL; ++l) __builtin_nontemporal_store(v[l], reinterpret_cast<V *>(out[l] + s * jb.rs));
+        for (int l = 0; l < NL; ++l) __builtin_nontemporal_store(__builtin_convertvector(v[l], V), reinterpret_cast<V *>(out[l] + s * jb.rs));
     };
     const int nt = SUM ? jb.nS - 1 : jb.nS;
     const int sa = SEG ? int((long long)nt * seg / jb.nseg) : 0, sb = SEG ? int((long long)nt * (seg + 1) / jb.nseg) : nt;
-    V v[NL];
+    VS v[NL];
     // walk of the refined steps sa .. sb - 1
     auto walk = [&](auto store) {
         if (sa >= sb) return;
@@ -252,7 +257,8 @@ __global__ void __launch_bounds__(SEG ? 512 : 256) k_xfer_yz(XferJob jb) {
 #pragma unroll
             for (int l = 0; l < NL; ++l) {
                 const V tv = W[(q + 1) & 3][l] * w0 + W[(q + 2) & 3][l] * w1 + W[(q + 3) & 3][l] * w2 + W[q][l] * w3;
-                v[l] = SUM ? v[l] + tv * dl : tv;
+                if constexpr (SUM) v[l] += __builtin_convertvector(tv, VS) * dl;
+                else v[l] = tv;
             }
             if (store) put(SUM ? s : s - 1, v);
         };
@@ -290,7 +296,7 @@ __global__ void __launch_bounds__(SEG ? 512 : 256) k_xfer_yz(XferJob jb) {
     if (SUM) {
         if (SEG) {
 #pragma unroll
-            for (int l = 0; l < NL; ++l) v[l] = V(RT(0));
+            for (int l = 0; l < NL; ++l) v[l] = VS(0);
             walk(std::false_type{});
 #pragma unroll
             for (int l = 0; l < NL; ++l) tot[(seg * NL + l) * 64 + lane] = v[l];
@@ -298,13 +304,13 @@ __global__ void __launch_bounds__(SEG ? 512 : 256) k_xfer_yz(XferJob jb) {
         }
         const RT *F = static_cast<const RT *>(jb.F);
 #pragma unroll
-        for (int l = 0; l < NL; ++l) v[l] = V(RT(0));
+        for (int l = 0; l < NL; ++l) v[l] = VS(0);
         if (F)
 #pragma unroll
             for (int c = 0; c < NU; ++c) {
                 const V f = *reinterpret_cast<const V *>(F + (long long)wrapf(o0 + c, jb.cO) * jb.ld + x);
 #pragma unroll
-                for (int l = 0; l < NL; ++l) v[l] += f * w[l][c];
+                for (int l = 0; l < NL; ++l) v[l] += __builtin_convertvector(f, VS) * double(w[l][c]);
             }
         if (seg == 0) put(0, v);
         for (int q = 0; SEG && q < seg; ++q)
