@@ -521,8 +521,8 @@ static int plan_lines(afid_ctx *c, const FftPlan<R> &py, const FftPlan<R> &pz, i
 }
 
 // LDS of k_to_coarse: two refined rows of each line
-template <typename RT, int NR, int NL>
-static size_t coarse_lds(int nxmr) { return sizeof(RT) * 2 * NL * size_t((nxmr + 3 * NR - 1) / NR * NR); }
+template <int NR, int NL>
+static size_t coarse_lds(int nxmr) { return sizeof(double) * 2 * NL * size_t((nxmr + 3 * NR - 1) / NR * NR); }
 // Ranges of z of k_to_coarse: each reads 2 to 4 refined planes of its
 // neighbour's, and a last round of workgroups that is nearly empty costs as
 // much as a full one, so the number is the one with the least rounds x planes
@@ -534,7 +534,7 @@ static int coarse_ranges(afid_ctx *c, bool x2) {
     int per_cu = 0, cus = 0;
     const int nch = (c->nxmr + 64 * NR - 1) / (64 * NR);
     const hipError_t e = x2 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_to_coarse_x2<RT, NR, NL>, 256, 0)
-                            : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_to_coarse<RT, NR, NL>, 64 * nch, coarse_lds<RT, NR, NL>(c->nxmr));
+                            : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_to_coarse<RT, NR, NL>, 64 * nch, coarse_lds<NR, NL>(c->nxmr));
     if (e != hipSuccess || per_cu < 1) per_cu = 1;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || cus < 1) cus = 256;
     // items and slots: workgroups of whole rows, or (x2) single wavefronts
@@ -1642,15 +1642,15 @@ static void launch_to_coarse(afid_ctx *c, const KP &p, CoarseJob &jb, bool x2) {
         hipLaunchKernelGGL((k_to_coarse_x2<RT, NR, NL>), dim3(tile_grid((items + 3) / 4)), dim3(256), 0, c->stream, p, jb);
         return;
     }
-    const size_t lds = coarse_lds<RT, NR, NL>(c->nxmr);
+    const size_t lds = coarse_lds<NR, NL>(c->nxmr);
     const unsigned waves = unsigned((c->nxmr + 64 * NR - 1) / (64 * NR));
     hipLaunchKernelGGL((k_to_coarse<RT, NR, NL>), dim3(tile_grid((long long)ngr * jb.nseg)), dim3(64u * waves), lds, c->stream, p, jb);
 }
-// (FP32 weights of the table for the mixed form's FP32 refined fields)
+// (FP32 weights of the table for k_to_coarse_x2 of the mixed form)
 static int to_coarse(afid_ctx *c, CoarseJob jb, const CoarseTab &t, const char *timer) {
     KP p = make_kp(c);
     jb.x_src = t.x_src; jb.y_src = t.y_src; jb.z_src = t.z_src;
-    if (c->mixed) { jb.x_w = t.x_wf; jb.y_w = t.y_wf; jb.z_w = t.z_wf; }
+    if (c->mixed && t.two_x) { jb.x_w = t.x_wf; jb.y_w = t.y_wf; jb.z_w = t.z_wf; }
     else { jb.x_w = t.x_w; jb.y_w = t.y_w; jb.z_w = t.z_w; }
     tstart(c, timer);
     jb.nseg = t.nseg;

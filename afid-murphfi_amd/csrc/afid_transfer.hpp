@@ -332,7 +332,8 @@ enum CoarseMode {
 };
 // Per axis and coarse index: the first of the 4 refined sources (1-based
 // reference index: x may name the wall ghosts 0 and nxr or the zero entries
-// beyond them, y/z may name periodic images) and its 4 weights (RT).  The
+// beyond them, y/z may name periodic images) and its 4 weights (FP64 for
+// k_to_coarse, RT for k_to_coarse_x2).  The
 // bracketing (fast) path of interpolate_xyz_to_coarse_fast and the general
 // path of interpolate_xyz_to_coarse differ only in these tables.
 struct CoarseJob {
@@ -354,22 +355,27 @@ struct CoarseJob {
 // Ghosts at the walls are folded into the x weights: the mirrored value into
 // the tap it mirrors, the wall's 2 S into gS / gN, whose y / z contraction 16
 // lanes form.
+// Weights and sums are FP64 also for FP32 fields, so that only what is stored
+// is rounded: in FP32 the order y, z, x was up to 5% less accurate (rms) than
+// x, y, z at x ratios such as 7/4.  It costs 5 us of 56 a step at 64 x 96^2
+// from 128 x 192^2, 80 of 1580 at 384 x 384^2 from 768^3.
 // What bounds it: the read of the refined field once (us a launch, at 5.2 TB/s,
 // now, and as 64 x 8 x 16 tiles staged in LDS with a barrier per refined plane
 // before, which left 72 workgroups at 64^3):
 //   64^3 from 128^3 FP64                 4     13     190
 //   384 x 192^2 from 768 x 384^2 FP64  196    242     495
-//   384 x 384^2 from 768^3 FP32        370    497    1189
-//   256 x 256^2 from 512^3 FP32 (phi)  129    148     482
+//   384 x 384^2 from 768^3 FP32        370    526    1189
+//   256^3 from 448 x 512^2 FP32 (phi)  116    145
 // Single lines instead of pairs: 1147 against 850 us a step at 384 x 192^2 (8
 // rows instead of 6 for two lines), 44 against 50 at 64^3 before the choice of
 // ranges (35 now).
 template <typename RT, int NR, int NL>
 __global__ void __launch_bounds__(512) k_to_coarse(KP p, CoarseJob jb) {
     using V = typename XVec<RT, NR>::V;
+    using VD = typename XVec<double, NR>::V;
     constexpr int NU = 4 + 2 * (NL - 1), PD = 2;                // rows; planes loaded ahead (4: the same)
-    extern __shared__ __align__(16) unsigned char smraw[];
-    RT *sm = reinterpret_cast<RT *>(smraw);                     // [2][line][reference refined x + NR - 1]
+    extern __shared__ __align__(32) unsigned char smraw[];
+    double *sm = reinterpret_cast<double *>(smraw);             // [2][line][reference refined x + NR - 1]
     const int LD = (p.nxmr + 3 * NR - 1) / NR * NR;
     const int t = threadIdx.x, T = blockDim.x, lane = t & 63;
     const int ngr = (p.ny + NL - 1) / NL, item = int(xcd_block(0));
@@ -379,9 +385,9 @@ __global__ void __launch_bounds__(512) k_to_coarse(KP p, CoarseJob jb) {
     if (I0 >= I1) return;
     const RT *src = static_cast<const RT *>(jb.src);
     const ConstTab<int> sy = const_tab(jb.y_src), sz = const_tab(jb.z_src);
-    const ConstTab<RT> ywc = const_tab(static_cast<const RT *>(jb.y_w));
+    const ConstTab<double> ywc = const_tab(static_cast<const double *>(jb.y_w));
     const int y0 = sy[J0] - 1, xw = t * NR, x = min(xw, (p.nxmr - 1) / NR * NR);
-    RT wy[NL][4];
+    double wy[NL][4];
     long long ro[NU];
 #pragma unroll
     for (int l = 0; l < NL; ++l)
@@ -390,18 +396,18 @@ __global__ void __launch_bounds__(512) k_to_coarse(KP p, CoarseJob jb) {
 #pragma unroll
     for (int c = 0; c < NU; ++c) ro[c] = (long long)wrapf(y0 + c, p.nyr) * p.ldxr + x;
     // taps of coarse k: weights of reference x base .. base + 3, all interior
-    struct Taps { int base; RT w[4], gS, gN; };
+    struct Taps { int base; double w[4], gS, gN; };
     auto taps = [&](int k) {
-        Taps q{1, {RT(0), RT(0), RT(0), RT(0)}, RT(0), RT(0)};
+        Taps q{1, {0.0, 0.0, 0.0, 0.0}, 0.0, 0.0};
         if (k >= p.nxm) return q;
-        const RT *w4 = static_cast<const RT *>(jb.x_w) + 4 * k;
+        const double *w4 = static_cast<const double *>(jb.x_w) + 4 * k;
         const int s = jb.x_src[k];
         q.base = max(1, min(s, p.nxmr - 3));
 #pragma unroll
         for (int a = 0; a < 4; ++a) {
             int kr = s + a;
-            RT w = w4[a];
-            if (kr < 0 || kr > p.nxr) w = RT(0);
+            double w = w4[a];
+            if (kr < 0 || kr > p.nxr) w = 0.0;
             else if (kr == 0) {
                 if (jb.mode == CM_SAL && p.sfixs == 1) { q.gS += w; w = -w; }
             } else if (kr == p.nxr) {
@@ -416,18 +422,19 @@ __global__ void __launch_bounds__(512) k_to_coarse(KP p, CoarseJob jb) {
     };
     Taps tp[2] = {taps(t), taps(t + T)};
     // 2 S of the walls: lane (a, b, l, wall) its point of the y / z stencil
-    const bool wall = jb.mode == CM_SAL && (2 * T < p.nxm || __any(tp[0].gS != RT(0) || tp[0].gN != RT(0) || tp[1].gS != RT(0) || tp[1].gN != RT(0)));
+    const bool wall = jb.mode == CM_SAL && (2 * T < p.nxm || __any(tp[0].gS != 0.0 || tp[0].gN != 0.0 || tp[1].gS != 0.0 || tp[1].gN != 0.0));
     const int la = lane & 3, lb = (lane >> 2) & 3, ll = NL == 2 ? (lane >> 4) & 1 : 0;
     const double *bp = lane < 32 ? p.salbp : p.saltp;
     const int by = wrapf(y0 + 2 * ll + lb, p.nyr);
-    const RT bw = static_cast<const RT *>(jb.y_w)[4 * (J0 + ll) + lb];
-    RT bv = RT(0);
-    auto load_wall = [&](int zs) { bv = RT(2.0 * bp[(long long)wrapf(zs + la, p.nzr) * p.nyr + by]); };
+    const double bw = static_cast<const double *>(jb.y_w)[4 * (J0 + ll) + lb];
+    double bv = 0.0;
+    auto load_wall = [&](int zs) { bv = 2.0 * bp[(long long)wrapf(zs + la, p.nzr) * p.nyr + by]; };
 
     int zr = sz[I0] - 1;
     const int end = sz[I1 - 1] + 2;
     int zw = wrapf(zr, p.nzr), zl = zr;                          // the plane to load next, on the periodic axis and off it
-    V R[PD][NU], W[4][NL];
+    V R[PD][NU];
+    VD W[4][NL];
     auto load = [&](V (&r)[NU]) {
         const RT *q = src + zw * p.planer;
 #pragma unroll
@@ -438,39 +445,39 @@ __global__ void __launch_bounds__(512) k_to_coarse(KP p, CoarseJob jb) {
     for (int q = 0; q < PD; ++q) load(R[q]);
     // the stencils of 64 coarse planes at a time, one per lane
     int ic = I0, base = I0, tn = 0;
-    RT t0 = RT(0), t1 = RT(0), t2 = RT(0), t3 = RT(0);
+    double t0 = 0.0, t1 = 0.0, t2 = 0.0, t3 = 0.0;
     auto fill = [&]() {
         base = ic;
         const int k = min(ic + lane, I1 - 1);
         tn = jb.z_src[k] + 2;
-        const RT *w4 = static_cast<const RT *>(jb.z_w) + 4 * k;
+        const double *w4 = static_cast<const double *>(jb.z_w) + 4 * k;
         t0 = w4[0]; t1 = w4[1]; t2 = w4[2]; t3 = w4[3];
     };
     fill();
     int need = __builtin_amdgcn_readlane(tn, 0), e = 0;
     if (wall) load_wall(need - 3);
-    auto store = [&](long long o, RT v) {
-        if (jb.mode == CM_SAL) static_cast<RT *>(jb.out)[o] = v;
+    auto store = [&](long long o, double v) {
+        if (jb.mode == CM_SAL) static_cast<RT *>(jb.out)[o] = RT(v);
         else {
             double *out = static_cast<double *>(jb.out);
-            const double val = jb.mode == CM_LAT ? jb.scale * double(v) : double(v);
+            const double val = jb.mode == CM_LAT ? jb.scale * v : v;
             out[o] = jb.accumulate ? out[o] + val : val;
         }
     };
     auto emit = [&](int q) {
         const int k = ic - base;
-        const RT w0 = lane_value(t0, k), w1 = lane_value(t1, k), w2 = lane_value(t2, k), w3 = lane_value(t3, k);
-        RT *b = sm + (e & 1) * NL * LD;
+        const double w0 = lane_value(t0, k), w1 = lane_value(t1, k), w2 = lane_value(t2, k), w3 = lane_value(t3, k);
+        double *b = sm + (e & 1) * NL * LD;
         e ^= 1;
 #pragma unroll
         for (int l = 0; l < NL; ++l) {
-            const V v = W[(q + 1) & 3][l] * w0 + W[(q + 2) & 3][l] * w1 + W[(q + 3) & 3][l] * w2 + W[q][l] * w3;
-            if (xw < p.nxmr) *reinterpret_cast<V *>(b + l * LD + NR + xw) = v;
+            const VD v = W[(q + 1) & 3][l] * w0 + W[(q + 2) & 3][l] * w1 + W[(q + 3) & 3][l] * w2 + W[q][l] * w3;
+            if (xw < p.nxmr) *reinterpret_cast<VD *>(b + l * LD + NR + xw) = v;
         }
         __syncthreads();
-        RT g[2][NL] = {};
+        double g[2][NL] = {};
         if (wall) {
-            RT s = bv * bw * (la == 0 ? w0 : la == 1 ? w1 : la == 2 ? w2 : w3);
+            double s = bv * bw * (la == 0 ? w0 : la == 1 ? w1 : la == 2 ? w2 : w3);
             s += dpp_move<0x128, 0xf, true>(s);                 // row_ror: the 16 points of a line and wall
             s += dpp_move<0x124, 0xf, true>(s);
             s += dpp_move<0x122, 0xf, true>(s);
@@ -482,8 +489,8 @@ __global__ void __launch_bounds__(512) k_to_coarse(KP p, CoarseJob jb) {
             if (kk >= p.nxm) return;
 #pragma unroll
             for (int l = 0; l < NL; ++l) {
-                const RT *r = b + l * LD + NR - 1;
-                RT v = RT(0);
+                const double *r = b + l * LD + NR - 1;
+                double v = 0.0;
 #pragma unroll
                 for (int a = 0; a < 4; ++a) v += r[min(q.base + a, p.nxmr)] * q.w[a];
                 if (wall) v += q.gS * g[0][l] + q.gN * g[1][l];
@@ -506,7 +513,10 @@ __global__ void __launch_bounds__(512) k_to_coarse(KP p, CoarseJob jb) {
         for (int q = 0; q < 4; ++q) {
             if (zr + q > end) break;
 #pragma unroll
-            for (int l = 0; l < NL; ++l) W[q][l] = R[q % PD][2 * l] * wy[l][0] + R[q % PD][2 * l + 1] * wy[l][1] + R[q % PD][2 * l + 2] * wy[l][2] + R[q % PD][2 * l + 3] * wy[l][3];
+            for (int l = 0; l < NL; ++l) {
+                const auto row = [&](int b) { return __builtin_convertvector(R[q % PD][2 * l + b], VD); };
+                W[q][l] = row(0) * wy[l][0] + row(1) * wy[l][1] + row(2) * wy[l][2] + row(3) * wy[l][3];
+            }
             load(R[q % PD]);
             while (need == zr + q) {
                 emit(q);
@@ -524,10 +534,13 @@ __global__ void __launch_bounds__(512) k_to_coarse(KP p, CoarseJob jb) {
 // arrives, from a lane's own NR points and one of either neighbour (at the ends
 // of a wavefront's run one load more), so that NR / 2 values a lane stay to be
 // contracted in y and z and nothing goes through LDS.  As fast as the form
-// above; it is here because the order x, y, z with these roundings (dot4) is
-// the more exact one for the FP32 fields: the kinetic energy of a 256 x 512^2
-// melting sphere after 100 steps is 9.6e-7 from the FP64 form's, 1.4e-6 with y,
-// z, x.  One wavefront per run of refined x, pair of lines and range of z.
+// above (434 / 460 against 429 / 446 us a step, d phi / phi of 512^3 FP32).  It
+// is here for its roundings: in FP32 the order x, y, z with dot4 gives phic to
+// the bit as the kernel before both did, and the mixed form's melting sphere is
+// compared with the FP64 form's after 100 steps, where the kinetic energy of
+// the weak flow amplifies round-off (9.6e-7 apart; 1.3e-6 with the exact
+// contraction above, which is no worse a solution).  One wavefront per run of
+// refined x, pair of lines and range of z.
 template <typename RT>
 __device__ __forceinline__ RT dot4(RT a0, RT w0, RT a1, RT w1, RT a2, RT w2, RT a3, RT w3) {
     if constexpr (sizeof(RT) == 4) return __builtin_fmaf(a3, w3, __builtin_fmaf(a2, w2, __builtin_fmaf(a0, w0, a1 * w1)));
