@@ -179,7 +179,11 @@ enum ColTab { CT_RK, CT_U3C, CT_U3M, CT_APC, CT_AMC, CT_APS, CT_ACS, CT_AMS, CT_
 // keeps the instruction scheduler from moving every load of a group to its
 // top: without it the kernel needs 223 to 256 registers and spills
 #define AFID_FENCE __builtin_amdgcn_sched_barrier(0);
-template <int LPC, int MG, int NW, int KEEP, bool LT, typename HT>
+// WIDE: fields of 4 GiB and more, whose planes take 64-bit bases; the others
+// reach a whole field through 32-bit offsets from its start.  With bases for all
+// the kernel is 1 to 3% slower (192 x 256^2 FP64 451 -> 459 us a launch, 256 x
+// 512^2 mixed 2050 -> 2100): the scalar registers run out.
+template <int LPC, int MG, int NW, int KEEP, bool LT, bool WIDE, typename HT>
 __global__ void __launch_bounds__(64 * NW) k_column_base_reg(KP p, BaseConst<HT> k, TriFactors fx, TriFactors fyz, TriFactors ft, BaseOut o) {
     using H2 = typename Pair<HT>::T;
     constexpr unsigned ROWS = 2u * LPC * MG;
@@ -219,13 +223,17 @@ __global__ void __launch_bounds__(64 * NW) k_column_base_reg(KP p, BaseConst<HT>
     const bool live = LPC == 64 || jw + int(lane / LPC) < p.ny;
     const int j = live ? jw + int(lane / LPC) : jw;
     const int im = wrapm(i, p.nz), ip = wrapp(i, p.nz);
-    // byte offsets into whole FP64 fields (below 4 GiB: the host checks)
-    const unsigned pl = unsigned(p.plane) * 8u, row = unsigned(p.ldx) * 8u;
+    // byte offsets into whole FP64 fields (below 4 GiB: the host checks), or
+    // into the planes at i - 1, i, i + 1
+    const unsigned pl = WIDE ? 0u : unsigned(p.plane) * 8u, row = unsigned(p.ldx) * 8u;
     const unsigned jo = unsigned(j) * row, jmo = unsigned(wrapm(j, p.ny)) * row, jpo = unsigned(wrapp(j, p.ny)) * row;
     const unsigned io = unsigned(i) * pl, imo = unsigned(im) * pl, ipo = unsigned(ip) * pl;
     const unsigned o_c = io + jo, o_jm = io + jmo, o_jp = io + jpo, o_im = imo + jo, o_ip = ipo + jo, o_jpim = imo + jpo, o_jmip = ipo + jmo;
-    const double *X = p.vx, *Y = p.vy, *Z = p.vz, *T = p.temp, *P = p.pr;
-    HT *RX = sel<HT>(p.rux, p.ruxf), *RY = sel<HT>(p.ruy, p.ruyf), *RZ = sel<HT>(p.ruz, p.ruzf), *RT = sel<HT>(p.rut, p.rutf);
+    const long long pc = WIDE ? (long long)i * p.plane : 0, pm = WIDE ? (long long)im * p.plane : 0, pp = WIDE ? (long long)ip * p.plane : 0;
+    const double *X = p.vx + pc, *Y = p.vy + pc, *Z = p.vz + pc, *T = p.temp + pc, *P = p.pr + pc;
+    const double *Xm = p.vx + pm, *Xp = p.vx + pp, *Ym = p.vy + pm, *Yp = p.vy + pp, *Zm = p.vz + pm, *Zp = p.vz + pp;
+    const double *Tm = p.temp + pm, *Tp = p.temp + pp, *Pm = p.pr + pm;
+    HT *RX = sel<HT>(p.rux, p.ruxf) + pc, *RY = sel<HT>(p.ruy, p.ruyf) + pc, *RZ = sel<HT>(p.ruz, p.ruzf) + pc, *RT = sel<HT>(p.rut, p.rutf) + pc;
     // (opaque, so that the row tables are read where they are used and not kept in registers from block to block)
     unsigned l2 = 2u * l;
     asm volatile("" : "+v"(l2));
@@ -236,11 +244,10 @@ __global__ void __launch_bounds__(64 * NW) k_column_base_reg(KP p, BaseConst<HT>
 #pragma unroll
     for (int g = 0; g < MG; ++g) {
         const unsigned r0 = 2u * unsigned(g) * LPC + l2, rb = min(r0, rmax) * 8u, c = o_c + rb;
-        
         // loads of the vx term
         const double2 x = ldp(X, c), v = ldp(Y, c), w = ldp(Z, c), t = ldp(T, c), q = ldp(P, c);
-        const double2 xjm = ldp(X, o_jm + rb), xjp = ldp(X, o_jp + rb), xim = ldp(X, o_im + rb), xip = ldp(X, o_ip + rb);
-        const double2 vjp = ldp(Y, o_jp + rb), wip = ldp(Z, o_ip + rb);
+        const double2 xjm = ldp(X, o_jm + rb), xjp = ldp(X, o_jp + rb), xim = ldp(Xm, o_im + rb), xip = ldp(Xp, o_ip + rb);
+        const double2 vjp = ldp(Y, o_jp + rb), wip = ldp(Zp, o_ip + rb);
         const unsigned ch = c / 8u * unsigned(sizeof(HT));
         const H2 ox = ldp_nt(RX, ch);
         // the rows just outside the group, by its end lanes
@@ -248,18 +255,18 @@ __global__ void __launch_bounds__(64 * NW) k_column_base_reg(KP p, BaseConst<HT>
         if ((lo_lane && g > 0) || hi_lane) {
             const unsigned eb = hi_lane ? min(r0 + 2u, rmax + 1u) * 8u : rb - 8u;
             ex = ld1(X, o_c + eb); ev = ld1(Y, o_c + eb); ew = ld1(Z, o_c + eb); et = ld1(T, o_c + eb);
-            if (hi_lane) { exjm = ld1(X, o_jm + eb); exim = ld1(X, o_im + eb); }
-            else { eq = ld1(P, o_c + eb); evjp = ld1(Y, o_jp + eb); ewip = ld1(Z, o_ip + eb); }
+            if (hi_lane) { exjm = ld1(X, o_jm + eb); exim = ld1(Xm, o_im + eb); }
+            else { eq = ld1(P, o_c + eb); evjp = ld1(Y, o_jp + eb); ewip = ld1(Zp, o_ip + eb); }
         }
         H2 sal;
         sal.x = HT(0); sal.y = HT(0);
-        if (p.active_s == 1) sal = ldp(sel<HT>(p.salc, p.salcf), ch);
+        if (p.active_s == 1) sal = ldp(sel<HT>(p.salc, p.salcf) + pc, ch);
         double2 bref = make_double2(0.0, 0.0);
         if (use_bref) bref = ldp(p.bref, rb);
         AFID_FENCE
         // loads of the vy term, in flight over the vx term; vz and T follow alike
-        const double2 vjm = ldp(Y, o_jm + rb), vim = ldp(Y, o_im + rb), vip = ldp(Y, o_ip + rb);
-        const double2 wjm = ldp(Z, o_jm + rb), wjmip = ldp(Z, o_jmip + rb), qjm = ldp(P, o_jm + rb);
+        const double2 vjm = ldp(Y, o_jm + rb), vim = ldp(Ym, o_im + rb), vip = ldp(Yp, o_ip + rb);
+        const double2 wjm = ldp(Z, o_jm + rb), wjmip = ldp(Zp, o_jmip + rb), qjm = ldp(P, o_jm + rb);
         const H2 oy = ldp_nt(RY, ch);
         AFID_FENCE
         // the two rows' values: V of the pair, of the row below, above
@@ -304,7 +311,7 @@ __global__ void __launch_bounds__(64 * NW) k_column_base_reg(KP p, BaseConst<HT>
         keep[wave][g][1][lane] = v;
         if (KEEP == 4) { keep[wave][g][KEEP - 2][lane] = w; keep[wave][g][KEEP - 1][lane] = t; }
         AFID_FENCE
-        const double2 wim = ldp(Z, o_im + rb), wjp = ldp(Z, o_jp + rb), vjpim = ldp(Y, o_jpim + rb), qim = ldp(P, o_im + rb);
+        const double2 wim = ldp(Zm, o_im + rb), wjp = ldp(Z, o_jp + rb), vjpim = ldp(Ym, o_jpim + rb), qim = ldp(Pm, o_im + rb);
         const H2 oz = ldp_nt(RZ, ch);
         AFID_FENCE
         const double2 u3m = tp(CT_U3M, r0), aps = tp(CT_APS, r0), acs = tp(CT_ACS, r0), ams = tp(CT_AMS, r0);
@@ -338,7 +345,7 @@ __global__ void __launch_bounds__(64 * NW) k_column_base_reg(KP p, BaseConst<HT>
             if (live && r0 < nxm) stp_nt(RY, ch, hy);
         }
         AFID_FENCE
-        const double2 tjm = ldp(T, o_jm + rb), tjp = ldp(T, o_jp + rb), tim = ldp(T, o_im + rb), tip = ldp(T, o_ip + rb);
+        const double2 tjm = ldp(T, o_jm + rb), tjp = ldp(T, o_jp + rb), tim = ldp(Tm, o_im + rb), tip = ldp(Tp, o_ip + rb);
         const H2 ot = ldp_nt(RT, ch);
         AFID_FENCE
         {
@@ -347,7 +354,7 @@ __global__ void __launch_bounds__(64 * NW) k_column_base_reg(KP p, BaseConst<HT>
             const double2 xn = hi2(x, pick(hi_lane, ex, lane_next(x.x)));
             const HT xima = pick(hi_lane, HT(exim), lane_next(HT(xim.x)));
             double2 gt = t;
-            if (p.gaxis == 3) gt = ldp(T, o_im + rb);
+            if (p.gaxis == 3) gt = ldp(Tm, o_im + rb);
             H2 hz;
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
@@ -385,7 +392,7 @@ __global__ void __launch_bounds__(64 * NW) k_column_base_reg(KP p, BaseConst<HT>
                 const HT htz = (HT(AFID_E(wip)) * (tip_ + tc) - HT(AFID_E(w)) * (tc + tim_)) * k.dz2;
                 const HT hty = (HT(AFID_E(vjp)) * (tjp_ + tc) - HT(AFID_E(v)) * (tc + tjm_)) * k.dy2;
                 HT h = -(htx + hty + htz) + (tip_ - HT(2.0) * tc + tim_) * k.dzqp + (tjp_ - HT(2.0) * tc + tjm_) * k.dyqp;
-                if (p.moist && wc[e]) h = HT(double(h) + condensation_heat(p, (long long)(o_c / 8u), r0 + e));
+                if (p.moist && wc[e]) h = HT(double(h) + condensation_heat(p, pc + (long long)(o_c / 8u), r0 + e));
                 const double ap = AFID_E(apt), ac = AFID_E(act), am = AFID_E(amt);
                 const double dxt = (kh[e] ? -(am + ac) * ttp * p.tfixn : AFID_E(tn) * ap) + AFID_E(t) * ac + (kl[e] ? -(ap + ac) * tbp * p.tfixs : AFID_E(tk) * am);
                 d[3][e] = wc[e] ? (p.ga * double(h) + p.ro * double(AFID_E(ot)) + k.alpect * dxt) * p.dt : 0.0;
@@ -452,16 +459,16 @@ __global__ void __launch_bounds__(64 * NW) k_column_base_reg(KP p, BaseConst<HT>
         if (live && r0 < nxm) {
             const bool in1 = r0 + 1 < nxm;
             // walls of vx: ImplicitAndUpdateVX.F90:86-87; the unused index nx of the others is carried over
-            stp_nt(o.vx, c, make_double2(r0 >= 1 ? u0.x + s[0][0] : 0.0, in1 ? u0.y + s[0][1] : 0.0));
-            stp_nt(o.vy, c, make_double2(u1.x + s[1][0], in1 ? u1.y + s[1][1] : u1.y));
-            stp_nt(o.vz, c, make_double2(u2.x + s[2][0], in1 ? u2.y + s[2][1] : u2.y));
-            stp_nt(o.temp, c, make_double2(u3.x + s[3][0], in1 ? u3.y + s[3][1] : u3.y));
+            stp_nt(o.vx + pc, c, make_double2(r0 >= 1 ? u0.x + s[0][0] : 0.0, in1 ? u0.y + s[0][1] : 0.0));
+            stp_nt(o.vy + pc, c, make_double2(u1.x + s[1][0], in1 ? u1.y + s[1][1] : u1.y));
+            stp_nt(o.vz + pc, c, make_double2(u2.x + s[2][0], in1 ? u2.y + s[2][1] : u2.y));
+            stp_nt(o.temp + pc, c, make_double2(u3.x + s[3][0], in1 ? u3.y + s[3][1] : u3.y));
         }
     }
     if (live && lo_lane && !(nxm & 1u)) {      // the face nx, alone in its pair when nxm is even
         const unsigned b = o_c + nxm * 8u;
         const double a1 = ld1(Y, b), a2 = ld1(Z, b), a3 = ld1(T, b);
-        const unsigned q = b / 8u;
+        const long long q = pc + (long long)(b / 8u);
         o.vx[q] = 0.0; o.vy[q] = a1; o.vz[q] = a2; o.temp[q] = a3;
     }
     }

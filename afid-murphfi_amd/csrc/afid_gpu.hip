@@ -120,6 +120,7 @@ struct afid_ctx {
     double *d_phi_part = nullptr, *d_phi_out = nullptr;
     int mean_groups = 0, sal_groups = 0, phi_groups = 0;
     bool col_four_pass = false;         // base columns through the four-pass kernel (AFID_COLUMN_FOUR_PASS=1)
+    bool col_wide = false;              // register form for fields of 4 GiB and more on any field (AFID_COLUMN_WIDE=1)
     // mixed form, gAxis = 1: the FP32 vx explicit term and its history hold
     // the buoyancy minus a per-row FP64 reference bref (that of the
     // conductive profile between the mean wall temperatures), which the FP64
@@ -1065,6 +1066,7 @@ static int ctx_create(const afid_config *cfg, hipStream_t shared, afid_ctx **out
     }
     c->device = dev;
     if (const char *e = std::getenv("AFID_COLUMN_FOUR_PASS")) c->col_four_pass = std::atoi(e) != 0;
+    if (const char *e = std::getenv("AFID_COLUMN_WIDE")) c->col_wide = std::atoi(e) != 0;
     if (shared) {
         c->stream = shared;
         c->own_stream = false;
@@ -1749,20 +1751,18 @@ static void launch_column_base(afid_ctx *c, const KP &p) {
     else if (c->pf) launch_column_base_form<CH, double, true>(c, p);
     else launch_column_base_form<CH, double, false>(c, p);
 }
-// single-pass kernel through LDS; CH here is the chunk of the nxm-row systems
-template <int CH, typename HT, bool PF>
+// single-pass kernel through LDS (phase field); CH here is the chunk of the nxm-row systems
+template <int CH, typename HT>
 static void launch_column_base1_form(afid_ctx *c, const KP &p) {
     BaseOut o{c->alt[0], c->alt[1], c->alt[2], c->alt[3]};
     const dim3 gr(unsigned((strip_blocks(c->ny, c->nz) + 7) / 8 * 8));
-    hipLaunchKernelGGL((k_column_base1<CH, HT, PF>), gr, dim3(256), 0, c->stream, p, factors(c, MAT_X), factors(c, MAT_YZ),
+    hipLaunchKernelGGL((k_column_base1<CH, HT>), gr, dim3(256), 0, c->stream, p, factors(c, MAT_X), factors(c, MAT_YZ),
                        factors(c, MAT_T), o);
 }
 template <int CH>
 static void launch_column_base1(afid_ctx *c, const KP &p) {
-    if (c->mixed && c->pf) launch_column_base1_form<CH, float, true>(c, p);
-    else if (c->mixed) launch_column_base1_form<CH, float, false>(c, p);
-    else if (c->pf) launch_column_base1_form<CH, double, true>(c, p);
-    else launch_column_base1_form<CH, double, false>(c, p);
+    if (c->mixed) launch_column_base1_form<CH, float>(c, p);
+    else launch_column_base1_form<CH, double>(c, p);
 }
 // ExplicitHumidity + ImplicitHumidity + SolveImpEqnUpdate_Humidity of every
 // column into humid_alt; the caller swaps the buffers once the base column
@@ -1787,15 +1787,15 @@ static int column_humid(afid_ctx *c) {
 }
 // the register kernel (k_column_base_reg): LPC lanes per column, MG groups,
 // NW wavefronts per workgroup, KEEP old fields in LDS, row tables in LDS (LT)
-template <int LPC, int MG, int NW, int KEEP, bool LT>
+template <int LPC, int MG, int NW, int KEEP, bool LT, bool WIDE>
 static void launch_column_reg(afid_ctx *c, const KP &p, long long nblk, long long nwg) {
     const BaseOut o{c->alt[0], c->alt[1], c->alt[2], c->alt[3]};
     const dim3 gr(unsigned(std::min((nblk + 7) / 8 * 8, nwg)));
     if (c->mixed)
-        hipLaunchKernelGGL((k_column_base_reg<LPC, MG, NW, KEEP, LT, float>), gr, dim3(64 * NW), 0, c->stream, p, base_const<float>(p),
+        hipLaunchKernelGGL((k_column_base_reg<LPC, MG, NW, KEEP, LT, WIDE, float>), gr, dim3(64 * NW), 0, c->stream, p, base_const<float>(p),
                            factors(c, MAT_X), factors(c, MAT_YZ), factors(c, MAT_T), o);
     else
-        hipLaunchKernelGGL((k_column_base_reg<LPC, MG, NW, KEEP, LT, double>), gr, dim3(64 * NW), 0, c->stream, p, base_const<double>(p),
+        hipLaunchKernelGGL((k_column_base_reg<LPC, MG, NW, KEEP, LT, WIDE, double>), gr, dim3(64 * NW), 0, c->stream, p, base_const<double>(p),
                            factors(c, MAT_X), factors(c, MAT_YZ), factors(c, MAT_T), o);
 }
 // The grid is what the card holds at once (two wavefronts per SIMD by
@@ -1807,30 +1807,32 @@ static void launch_column_reg(afid_ctx *c, const KP &p, long long nblk, long lon
 // only where every workgroup has a single block of at most 64 rows: 18.6
 // against 21.1 us for a 64 x 64^2 launch; elsewhere they win (128 x 256^2:
 // 313 against 387 us, 48 x 96^2: 32.6 against 34.0).
+template <bool WIDE>
 static int column_base_reg(afid_ctx *c, const KP &p) {
     const long long b32 = col_blocks<32, 4>(c->ny, c->nz), b64 = col_blocks<64, 4>(c->ny, c->nz), b8 = col_blocks<64, 8>(c->ny, c->nz);
     switch (c->chunk[MAT_YZ]) {
     case 1:
-        if (b32 <= 512) launch_column_reg<32, 1, 4, 4, false>(c, p, b32, 512);
-        else launch_column_reg<32, 1, 4, 4, true>(c, p, b32, 512);
+        if (!WIDE && b32 <= 512) launch_column_reg<32, 1, 4, 4, false, false>(c, p, b32, 512);
+        else launch_column_reg<32, 1, 4, 4, true, WIDE>(c, p, b32, 512);
         break;
-    case 2: launch_column_reg<64, 1, 4, 4, true>(c, p, b64, 512); break;
-    case 3: launch_column_reg<32, 3, 4, 4, true>(c, p, b32, 512); break;
-    case 4: launch_column_reg<64, 2, 4, 4, true>(c, p, b64, 512); break;
-    case 5: case 6: launch_column_reg<64, 3, 8, 4, true>(c, p, b8, 256); break;
-    default: launch_column_reg<64, 4, 8, 2, true>(c, p, b8, 256); break;
+    case 2: launch_column_reg<64, 1, 4, 4, true, WIDE>(c, p, b64, 512); break;
+    case 3: launch_column_reg<32, 3, 4, 4, true, WIDE>(c, p, b32, 512); break;
+    case 4: launch_column_reg<64, 2, 4, 4, true, WIDE>(c, p, b64, 512); break;
+    case 5: case 6: launch_column_reg<64, 3, 8, 4, true, WIDE>(c, p, b8, 256); break;
+    default: launch_column_reg<64, 4, 8, 2, true, WIDE>(c, p, b8, 256); break;
     }
     return check_launch(c, "k_column_base_reg");
 }
 static int column_base(afid_ctx *c) {
     KP p = make_kp(c);
     int rc;
-    // up to 512 wall-normal cells: the register kernel for fields it can
-    // address with 32-bit byte offsets, else (and with the phase field, whose
-    // solves are masked) the single pass through LDS; four passes above
-    const bool reg = !c->pf && (unsigned long long)p.plane * c->nz * sizeof(double) < (1ull << 32);
-    if (!c->col_four_pass && c->chunk[MAT_YZ] <= 8 && reg) {
-        if ((rc = column_base_reg(c, p))) return rc;
+    // up to 512 wall-normal cells: the register kernel, with 32-bit byte
+    // offsets into whole fields where these are below 4 GiB; with the phase
+    // field, whose solves are masked, the single pass through LDS; four passes
+    // above
+    const bool wide = c->col_wide || (unsigned long long)p.plane * c->nz * sizeof(double) >= (1ull << 32);
+    if (!c->col_four_pass && c->chunk[MAT_YZ] <= 8 && !c->pf) {
+        if ((rc = wide ? column_base_reg<true>(c, p) : column_base_reg<false>(c, p))) return rc;
     } else if (!c->col_four_pass && c->chunk[MAT_YZ] <= 8) {
         switch (c->chunk[MAT_YZ]) {
 #define AFID_CB1_CASE(CH) case CH: launch_column_base1<CH>(c, p); break;

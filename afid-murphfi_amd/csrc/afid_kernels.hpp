@@ -514,12 +514,12 @@ __global__ void __launch_bounds__(256) k_column_base(KP p, TriFactors fx, TriFac
 }
 
 // Right-hand sides of vx, vy, vz and T at row r < nx of one column (the
-// stencil phase of column_base_rows for the four fields at once, no phase
+// stencil phase of column_base_rows for the four fields at once, with the phase
 // field): every neighbour value is loaded once for the four explicit terms,
 // and the explicit terms are stored to their history arrays after all
 // loads.  Rows without an equation (vx rows 0 and nxm, the unused index
 // nxm of the others) give 0.
-template <typename HT, bool PF = false>
+template <typename HT>
 __device__ __forceinline__ void base_rhs4(const KP &p, const Nb &n, long long c0, unsigned r, double (&rhs)[4],
                                           unsigned &solid) {
     const unsigned nxm = p.nxm;
@@ -531,7 +531,7 @@ __device__ __forceinline__ void base_rhs4(const KP &p, const Nb &n, long long c0
     double bref = 0.0, r0 = 0.0, r1 = 0.0, r2 = 0.0, r3 = 0.0;
     // phase field: solid rows of vx, vy, vz (bits 0..2); vx rows 0 and nxm
     // are identity rows (SolveImpEqnUpdate_X_pf)
-    bool sx = PF && !wx, sy = false, sz = false;
+    bool sx = !wx, sy = false, sz = false;
     if (wx) {
         if (sizeof(HT) == sizeof(float) && p.bref) {
             // FP32 terms: buoyancy as its deviation from the row's FP64
@@ -542,12 +542,10 @@ __device__ __forceinline__ void base_rhs4(const KP &p, const Nb &n, long long c0
             h0 = ex_vx<HT>(p, n, r);
         }
         if (p.gaxis == 1) h0 -= sb;
-        if (PF) {
-            // AddVolumePenalty (phasefield.F90:525-566); the row is solid where
-            // the averaged phic exceeds pf_direct_force = 0.9 (:29, :821-930)
-            h0 -= HT((n.pc[r] + n.pc[r - 1]) * n.vx[r] * p.heta);
-            sx = 0.5 * (n.pc[r] + n.pc[r + 1]) > 0.9;
-        }
+        // AddVolumePenalty (phasefield.F90:525-566); the row is solid where
+        // the averaged phic exceeds pf_direct_force = 0.9 (:29, :821-930)
+        h0 -= HT((n.pc[r] + n.pc[r - 1]) * n.vx[r] * p.heta);
+        sx = 0.5 * (n.pc[r] + n.pc[r + 1]) > 0.9;
         r0 = double(rux[r]);
     }
     if (wc) {
@@ -556,14 +554,12 @@ __device__ __forceinline__ void base_rhs4(const KP &p, const Nb &n, long long c0
         h2 = ex_vz<HT>(p, n, r);
         if (p.gaxis == 3) h2 -= sb;
         h3 = ex_temp<HT>(p, n, r);
-        if (PF) {
-            const double py = n.pc[r] + n.pc_jm[r], pz = n.pc[r] + n.pc_im[r];
-            h1 -= HT(py * n.vy[r] * p.heta);
-            h2 -= HT(pz * n.vz[r] * p.heta);
-            sy = 0.5 * py > 0.9;
-            sz = 0.5 * pz > 0.9;
-            h3 += HT(p.qlat[c0 + r]);            // AddLatentHeat (:651-725)
-        }
+        const double py = n.pc[r] + n.pc_jm[r], pz = n.pc[r] + n.pc_im[r];
+        h1 -= HT(py * n.vy[r] * p.heta);
+        h2 -= HT(pz * n.vz[r] * p.heta);
+        sy = 0.5 * py > 0.9;
+        sz = 0.5 * pz > 0.9;
+        h3 += HT(p.qlat[c0 + r]);                // AddLatentHeat (:651-725)
         if (p.moist) h3 = HT(double(h3) + condensation_heat(p, c0, r));
         r1 = double(ruy[r]); r2 = double(ruz[r]); r3 = double(rut[r]);
     }
@@ -571,12 +567,10 @@ __device__ __forceinline__ void base_rhs4(const KP &p, const Nb &n, long long c0
     rhs[1] = wc ? rhs_vy(p, n, double(h1), r1, r) : 0.0;
     rhs[2] = wc ? rhs_vz(p, n, double(h2), r2, r) : 0.0;
     rhs[3] = wc ? rhs_temp(p, n, double(h3), r3, r) : 0.0;
-    if (PF) {
-        // a solid row is the identity with right-hand side -u
-        if (sx) rhs[0] = -n.vx[r];
-        if (sy) rhs[1] = -n.vy[r];
-        if (sz) rhs[2] = -n.vz[r];
-    }
+    // a solid row is the identity with right-hand side -u
+    if (sx) rhs[0] = -n.vx[r];
+    if (sy) rhs[1] = -n.vy[r];
+    if (sz) rhs[2] = -n.vz[r];
     solid = unsigned(sx) | unsigned(sy) << 1 | unsigned(sz) << 2;
     if (wx) rux[r] = h0;
     if (wc) { ruy[r] = h1; ruz[r] = h2; rut[r] = h3; }
@@ -603,7 +597,7 @@ __device__ __forceinline__ void column_solve_masked_bytes(double *buf, const uns
     for (int m = 0; m < CH; ++m) buf[lane * CHP + m] = v[m];
 }
 
-// Single-pass form of k_column_base.  One sweep over the rows forms the
+// Single-pass form of k_column_base with the phase field.  One sweep over the rows forms the
 // four right-hand sides, loading every neighbour value once for all four
 // explicit terms.  Those of vx and vy go to two LDS columns of the
 // wavefront, those of vz and T stay in registers.  The vx and vy solves and
@@ -611,18 +605,18 @@ __device__ __forceinline__ void column_solve_masked_bytes(double *buf, const uns
 // LDS columns for their solves and updates.  Two LDS columns per wavefront
 // instead of four keep 4 wavefronts per SIMD; the updates read the old value
 // of the own column again (from cache).
-// With PF the velocity terms carry the volume penalty, T the latent heat,
+// The velocity terms carry the volume penalty, T the latent heat,
 // and solid velocity rows are identity rows: their flags go to LDS as bytes
 // (vx, vy; vz's flags wait in a register bit mask) for the masked solves.
 // CH = ceil(nxm / 64) is the size of the largest system (nxm rows); when
 // nx = 64 CH + 1 the last face has no equation (the wall of vx, the unused
 // index of the others) and only the update touches it.
-template <int CH, typename HT, bool PF>
+template <int CH, typename HT>
 __global__ void __launch_bounds__(256) k_column_base1(KP p, TriFactors fx, TriFactors fyz, TriFactors ft, BaseOut o) {
     constexpr int CHP = lds_chunk_tight<CH>();
     constexpr unsigned NROW = 64u * CH;
     __shared__ double lds[4][2][lds_col_size<CH, CHP>()];
-    __shared__ unsigned char mskb[PF ? 4 : 1][2][PF ? NROW : 1];
+    __shared__ unsigned char mskb[4][2][NROW];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const unsigned lane = threadIdx.x & 63;
     int j, i;
@@ -631,7 +625,7 @@ __global__ void __launch_bounds__(256) k_column_base1(KP p, TriFactors fx, TriFa
     const long long c0 = (long long)i * p.plane + (long long)j * p.ldx;
     const unsigned nx = p.nx, nxm = p.nxm;
     double *b0 = lds[wave][0], *b1 = lds[wave][1];
-    unsigned char *m0 = mskb[PF ? wave : 0][0], *m1 = mskb[PF ? wave : 0][1];
+    unsigned char *m0 = mskb[wave][0], *m1 = mskb[wave][1];
     double keep[2][CH];                          // right-hand sides of vz and T
     unsigned zsolid = 0;                         // vz's solid flags, bit m for row lane + 64 m
 #pragma unroll
@@ -639,17 +633,15 @@ __global__ void __launch_bounds__(256) k_column_base1(KP p, TriFactors fx, TriFa
         const unsigned r = lane + 64u * m;
         double rhs[4] = {0.0, 0.0, 0.0, 0.0};
         unsigned solid = 0;
-        if (live && r < nxm) base_rhs4<HT, PF>(p, n, c0, r, rhs, solid);
+        if (live && r < nxm) base_rhs4<HT>(p, n, c0, r, rhs, solid);
         const unsigned q = lds_row<CH, CHP>(r);
         b0[q] = rhs[0];
         b1[q] = rhs[1];
         keep[0][m] = rhs[2];
         keep[1][m] = rhs[3];
-        if (PF) {
-            m0[r] = (unsigned char)(solid & 1u);
-            m1[r] = (unsigned char)((solid >> 1) & 1u);
-            zsolid |= ((solid >> 2) & 1u) << m;
-        }
+        m0[r] = (unsigned char)(solid & 1u);
+        m1[r] = (unsigned char)((solid >> 1) & 1u);
+        zsolid |= ((solid >> 2) & 1u) << m;
     }
     __syncthreads();
 #pragma unroll
@@ -660,18 +652,13 @@ __global__ void __launch_bounds__(256) k_column_base1(KP p, TriFactors fx, TriFa
                 const unsigned q = lds_row<CH, CHP>(lane + 64u * m);
                 b0[q] = keep[0][m];
                 b1[q] = keep[1][m];
-                if (PF) m0[lane + 64u * m] = (unsigned char)((zsolid >> m) & 1u);
+                m0[lane + 64u * m] = (unsigned char)((zsolid >> m) & 1u);
             }
             __syncthreads();
         }
-        if (PF) {
-            column_solve_masked_bytes<CH, CHP>(b0, m0, g == 0 ? fx : fyz);
-            if (g == 0) column_solve_masked_bytes<CH, CHP>(b1, m1, fyz);
-            else column_solve_lds<CH, CHP>(b1, ft);
-        } else {
-            column_solve_lds<CH, CHP>(b0, g == 0 ? fx : fyz);
-            column_solve_lds<CH, CHP>(b1, g == 0 ? fyz : ft);
-        }
+        column_solve_masked_bytes<CH, CHP>(b0, m0, g == 0 ? fx : fyz);
+        if (g == 0) column_solve_masked_bytes<CH, CHP>(b1, m1, fyz);
+        else column_solve_lds<CH, CHP>(b1, ft);
         __syncthreads();
         if (live) {
 #pragma unroll
