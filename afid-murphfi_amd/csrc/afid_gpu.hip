@@ -453,8 +453,12 @@ template <typename R>
 static int build_plan(afid_ctx *c, int n, FftPlan<R> &pl, FftPlan<R> *ens = nullptr) {
     pl = FftPlan<R>{};
     pl.n = n;
-    std::vector<int> rad;
-    if (!pick_radices(n, {16, 12, 9, 8, 6, 4, 3, 2}, rad) || rad.size() > FFT_STAGES)
+    // (rad8: radices of an ensemble member's transform, one stage each)
+    std::vector<int> rad, rad8;
+    int m = n;
+    for (int r : {8, 4, 2, 3})
+        while (m % r == 0 && m > 1) { rad8.push_back(r); m /= r; }
+    if (!pick_radices(n, {16, 12, 9, 8, 6, 4, 3, 2}, rad) || rad.size() > FFT_STAGES || rad8.size() > FFT_STAGES)
         return set_err(c, AFID_E_ARG, "periodic size " + std::to_string(n) + " must factor into 2 and 3");
     for (int r : rad) pl.rad[pl.nst++] = r;
     std::vector<cpx<R>> tw((size_t)(n));
@@ -468,9 +472,7 @@ static int build_plan(afid_ctx *c, int n, FftPlan<R> &pl, FftPlan<R> *ens = null
     if (ens) {
         *ens = pl;
         ens->nst = 0;
-        int m = n;
-        for (int r : {8, 4, 2, 3})
-            while (m % r == 0 && m > 1) { ens->rad[ens->nst++] = r; m /= r; }
+        for (int r : rad8) ens->rad[ens->nst++] = r;
     }
     return rc;
 }
