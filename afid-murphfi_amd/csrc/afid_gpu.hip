@@ -205,6 +205,7 @@ static int dalloc(afid_ctx *ctx, void **p, size_t bytes) {
     hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess) {
         ctx->err = "hipMalloc(" + std::to_string(bytes) + ") failed: " + hipGetErrorString(e);
+        (void)hipGetLastError();            // reported here; not to the next launch's check
         return AFID_E_MEM;
     }
     ctx->bufs.push_back({*p, bytes});
@@ -509,6 +510,8 @@ static int plan_lines(afid_ctx *c, const FftPlan<R> &py, const FftPlan<R> &pz, i
     c->ty = std::max(c->ty, std::min((py.n << c->lgy) / 64 * 64, (long long)nbx * c->nz <= 512 ? 512 : 256));
     c->lds_y = (py.n << c->lgy) * int(sizeof(cpx<R>));
     c->lds_z = (pz.n << c->lgz) * int(sizeof(cpx<R>));
+    if (c->lds_y > maxlds || c->lds_z > maxlds || c->ny > 8192 || c->nz > 8192 || c->ty > FFT_MAXT || c->tz > FFT_MAXT)
+        return set_err(c, AFID_E_ARG, "periodic size too large for one workgroup transform");
     const auto more = [](const void *k, int lds) { if (lds > 65536) (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, lds); };
     with_threads<R>(c->ty, [&](auto mt) {
         more(reinterpret_cast<const void *>(k_div_fft_y<R, decltype(mt)::value>), c->lds_y);
@@ -518,8 +521,6 @@ static int plan_lines(afid_ctx *c, const FftPlan<R> &py, const FftPlan<R> &pz, i
         more(reinterpret_cast<const void *>(k_fft_z<R, -1, decltype(mt)::value>), c->lds_z);
         more(reinterpret_cast<const void *>(k_fft_z<R, 1, decltype(mt)::value>), c->lds_z);
     });
-    if (c->lds_y > maxlds || c->lds_z > maxlds || c->ny > 8192 || c->nz > 8192 || c->ty > FFT_MAXT || c->tz > FFT_MAXT)
-        return set_err(c, AFID_E_ARG, "periodic size too large for one workgroup transform");
     return AFID_OK;
 }
 
