@@ -164,9 +164,9 @@ struct afid_ctx {
     PoissonFactors<float> pff{};
     int pchunk = 1;
     // coarse -> refined transfers: rows of refined x per coarse column, and
-    // those of the velocity of the first plane (k_xfer_x); whether pairs
-    // of refined z lines read at most 5 coarse ones (k_xfer_yz)
-    void *xfer = nullptr, *xfer0 = nullptr;
+    // those of the velocity of the first plane (xfer_rows)
+    void *xfer = nullptr;               // their own scratch, where the second buffer of S / phi is too small
+    // whether pairs of refined z lines read at most 5 coarse ones (k_xfer_yz)
     bool pair_z = false;
     // refined steps of y / z two by two (ratio 2, see XferJob::two)
     bool two_y = false, two_z = false;
@@ -1009,9 +1009,9 @@ static int setup(afid_ctx *c) {
     c->two_z = twos(sz.src, nzr);
     c->pair_z = pairs(sz.src, nzr);
     {
-        const size_t e = c->mixed ? sizeof(float) : sizeof(double);
-        if ((rc = dalloc(c, &c->xfer, e * size_t(c->nz) * c->ny * c->ldxr))) return rc;
-        if ((rc = dalloc(c, &c->xfer0, e * size_t(std::max(c->ny, c->nz)) * c->ldxr))) return rc;
+        // rows of k_xfer_x: one per coarse column, and those of the first plane
+        const size_t rows = size_t(c->nz) * c->ny + size_t(std::max(c->ny, c->nz)), e = c->mixed ? sizeof(float) : sizeof(double);
+        if (rows > size_t(nzr) * nyr && (rc = dalloc(c, &c->xfer, e * rows * c->ldxr))) return rc;
     }
     // Refinement ratios that set-up admits: the coarse spans of 64 x, 16 y and
     // 4 z refined points of the transfers, as a block of 64 KiB holds them.
@@ -1540,13 +1540,21 @@ static int clean_tails(afid_ctx *c) {
     }
     return AFID_OK;
 }
+// Rows of refined x of the transfers: the second buffer of S or phi, which
+// holds nothing between one column step and the next (it writes every row).
+template <typename RT>
+static RT *xfer_rows(const afid_ctx *c) {
+    if (c->xfer) return static_cast<RT *>(c->xfer);
+    if constexpr (sizeof(RT) == 8) return c->sal ? c->sal_alt : c->phi_alt;
+    else return c->sal ? c->sal_alt_f : c->phi_alt_f;
+}
 // one coarse -> refined transfer: the x part of every coarse column, then the
 // y / z part of every refined line
 template <typename RT, int FLD>
 static int xfer_x(afid_ctx *c, const KP &p) {
     const long long ncol = (long long)c->ny * c->nz;
     const int ch = (std::max(c->nxm, c->nxmr) + 63) / 64;
-    RT *D = static_cast<RT *>(c->xfer), *F = static_cast<RT *>(c->xfer0);
+    RT *D = xfer_rows<RT>(c), *F = D + ncol * c->ldxr;
     // 512 workgroups: two on each CU, each loading the weights once; fewer
     // wavefronts where the rows of 8 do not fit beside the weights in 64 KiB
     auto launch = [&](auto k, int chr) {
@@ -1617,9 +1625,10 @@ static int xfer(afid_ctx *c, RT *out, const char *timer) {
     const RT *yw = sizeof(RT) == 8 ? reinterpret_cast<const RT *>(c->d_ys_w) : reinterpret_cast<const RT *>(c->f_ys_w);
     const RT *zw = sizeof(RT) == 8 ? reinterpret_cast<const RT *>(c->d_zs_w) : reinterpret_cast<const RT *>(c->f_zs_w);
     XferJob jb{};
-    jb.D = c->xfer; jb.out = out; jb.nx = c->nxmr; jb.ld = c->ldxr;
+    RT *D = xfer_rows<RT>(c);
+    jb.D = D; jb.out = out; jb.nx = c->nxmr; jb.ld = c->ldxr;
     // vzr starts from zero on a single plane (InterpVelMgrd.F90:184)
-    jb.F = FLD == XF_VY || (FLD == XF_VZ && c->nz > 1) ? c->xfer0 : nullptr;
+    jb.F = FLD == XF_VY || (FLD == XF_VZ && c->nz > 1) ? D + (long long)c->ny * c->nz * c->ldxr : nullptr;
     if (FLD == XF_VZ) {
         jb.s_src = c->d_zs_src; jb.o_src = c->d_ys_src; jb.s_w = zw; jb.o_w = yw;
         jb.nS = c->nzr; jb.nO = c->nyr; jb.cS = c->nz; jb.cO = c->ny;

@@ -1,0 +1,52 @@
+"""Device memory of a two-grid context: the refined fields and the second buffer
+of S or phi, and no scratch of the transfers beside them (at ratio 2 that would
+be a quarter of a refined field; a sixteenth is left for tables)."""
+import numpy as np
+import pytest
+
+import pyafid
+from helpers import load_state, random_state
+
+pytestmark = pytest.mark.gpu
+
+
+# refined arrays: S, its explicit terms, three velocities (FP64: two more for the per-routine calls) and the second buffer of S;
+# phi, its explicit terms, T, d phi (FP64: one more) and the second buffer of phi.  base: FP64 and FP32 arrays of the base grid
+# that the single-grid context does not have (phic, the latent heat; salc)
+@pytest.mark.parametrize("kind,form,refined,base", [("sal", "fp64", 8, (0, 0)), ("sal", "mixed", 6, (0, 1)), ("phi", "fp64", 6, (1, 0)), ("phi", "mixed", 5, (2, 0))])
+def test_two_grid_context(kind, form, refined, base):
+    one = dict(nxm=96, nym=96, nzm=128, istr3=8, rayt=1e6, prat=1.0, precision=pyafid.MIXED if form == "mixed" else pyafid.FP64)
+    two = dict(one, multires=1, nxmr=192, nymr=192, nzmr=256, istr3r=8)
+    two.update(dict(salinity=1, rays=-2e6, pras=4.0) if kind == "sal" else dict(phasefield=1, pf_eps=0.1))
+    size = []
+    for cfg in (one, two):
+        g = pyafid.Solver(cfg)
+        size.append(g.device_bytes())
+        g.close()
+    field = (4 if form == "mixed" else 8) * 256 * 192 * (-(-193 // 16) * 16)
+    nb = 128 * 96 * (-(-97 // 16) * 16)
+    assert size[1] - size[0] <= refined * field + (8 * base[0] + 4 * base[1]) * nb + field // 16
+
+
+@pytest.mark.parametrize("form", ["fp64", "mixed"])
+def test_transfers_leave_the_scalar_alone(form):
+    """A transfer between two steps (as a host that looks at vxr makes) changes nothing in the steps."""
+    cfg = dict(nxm=20, nym=12, nzm=16, istr3=8, istr3r=8, rayt=1e6, prat=1.0, multires=1, nxmr=40, nymr=24, nzmr=32, salinity=1,
+               rays=-2e6, pras=4.0, active_s=1, precision=pyafid.MIXED if form == "mixed" else pyafid.FP64)
+    st, got = random_state(cfg, 41), []
+    for more in (False, True):
+        g = pyafid.Solver(cfg)
+        load_state(g, st, upload=True)
+        for _ in range(3):
+            if more:
+                g.call("interp_vel_mgrd")
+                g.call("interp_sal_multigrid")
+                g.call("interp_vel_mgrd")
+            else:
+                g.call("interp_vel_mgrd")
+                g.call("interp_sal_multigrid")
+            g.time_marcher(1e-3)
+        got.append({f: g.download(f) for f in ("vx", "vy", "vz", "temp", "sal", "rusal", "vxr", "salc")})
+        g.close()
+    for f in got[0]:
+        assert np.array_equal(got[0][f], got[1][f]), f
