@@ -1991,6 +1991,9 @@ int afid_time_marcher(afid_ctx *c, double dt) {
 int afid_time_marcher_graph(afid_ctx *c, double dt, int nsteps) {
     if (!c || nsteps < 0) return AFID_E_ARG;
     int rc;
+    // the captured steps leave index nxr of vyr, vzr and tempr alone: cleared
+    // here after an upload, ahead of a capture or of a replay
+    if (nsteps > 0 && (rc = clean_tails(c))) return rc;
     bool same = c->graph && c->graph_dt == dt;
     for (int f = 0; same && f < AFID_NFIELDS; ++f) same = c->graph_ptrs[f] == c->f[f];
     if (!same && nsteps >= 2) {
@@ -2017,8 +2020,6 @@ int afid_time_marcher_graph(afid_ctx *c, double dt, int nsteps) {
         for (int f = 0; f < AFID_NFIELDS; ++f) c->graph_ptrs[f] = c->f[f];
     }
     int done = 0;
-    // (an upload between replays: the captured steps leave index nxr alone)
-    if (nsteps > 0 && (rc = clean_tails(c))) return rc;
     if (c->graph)
         for (; done + 2 <= nsteps; done += 2) HIPCHK(c, hipGraphLaunch(c->graph, c->stream));
     for (; done < nsteps; ++done)
