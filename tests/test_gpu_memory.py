@@ -50,3 +50,17 @@ def test_transfers_leave_the_scalar_alone(form):
         g.close()
     for f in got[0]:
         assert np.array_equal(got[0][f], got[1][f]), f
+
+
+@pytest.mark.parametrize("form,fields", [("fp64", 16), ("mixed", 10)])
+def test_ensemble_rows(form, fields):
+    """The rows of an ensemble member are whole 64 bytes, no more: 71 values take 72, 80 take 80, so that
+    eight values a row and field lie between the two runs (16 or more fields in FP64, the 10 of the state
+    and its second buffers at least in the mixed form)."""
+    size = []
+    for nxm in (70, 79):
+        cfg = dict(nxm=nxm, nym=1, nzm=256, istr3=8, rayt=1e6, prat=1.0, precision=pyafid.MIXED if form == "mixed" else pyafid.FP64)
+        e = pyafid.Ensemble([cfg], [dict(dt=1e-3)])
+        size.append(e.device_bytes())
+        e.close()
+    assert size[1] - size[0] >= fields * 8 * 256 * 8
