@@ -50,7 +50,7 @@ struct TimerRec {
 
 // Refined -> coarse tables of one transfer (k_to_coarse), per axis
 // and coarse index: the first refined source and 4 weights (FP64, and FP32
-// for the mixed form), with the tile's LDS plan.
+// for k_to_coarse_x2 of the mixed form), with what chooses the kernel.
 struct CoarseTab {
     const int *x_src = nullptr, *y_src = nullptr, *z_src = nullptr;
     const double *x_w = nullptr, *y_w = nullptr, *z_w = nullptr;
@@ -927,7 +927,7 @@ static int setup(afid_ctx *c) {
         if ((rc = upload_vec(c, h.xw, &w))) return; t.x_w = w;
         if ((rc = upload_vec(c, h.yw, &w))) return; t.y_w = w;
         if ((rc = upload_vec(c, h.zw, &w))) return; t.z_w = w;
-        if (c->mixed) {
+        if (c->mixed && c->pf) {
             const float *f;
             std::vector<float> a(h.xw.begin(), h.xw.end()), b(h.yw.begin(), h.yw.end()), d(h.zw.begin(), h.zw.end());
             if ((rc = upload_vec(c, a, &f))) return; t.x_wf = f;
@@ -988,7 +988,7 @@ static int setup(afid_ctx *c) {
         for (int f : {AFID_SALBP, AFID_SALTP})
             if ((rc = dalloc(c, reinterpret_cast<void **>(&c->f[f]), sizeof(double) * size_t(nyr) * nzr))) return rc;
     if (nxmr > 1024) return set_err(c, AFID_E_ARG, "refined wall-normal size above 1024 is not supported");
-    // LDS plan of the tiled transfer kernels: largest coarse block of any tile
+    // largest coarse span of any run of `tile` refined points
     auto span = [](const std::vector<int> &src, int n, int tile) {
         int m = 0;
         for (int a = 0; a < n; a += tile) {
@@ -1015,8 +1015,10 @@ static int setup(afid_ctx *c) {
         const size_t rows = size_t(c->nz) * c->ny + size_t(std::max(c->ny, c->nz)), e = c->mixed ? sizeof(float) : sizeof(double);
         if (rows > size_t(nzr) * nyr && (rc = dalloc(c, &c->xfer, e * rows * c->ldxr))) return rc;
     }
-    // Refinement ratios that set-up admits: the coarse spans of 64 x, 16 y and
-    // 4 z refined points of the transfers, as a block of 64 KiB holds them.
+    // Refinement ratios that set-up admits.  The kernels take others too; the
+    // line is that of an earlier form, which held the coarse spans of 64 x, 16 y
+    // and 4 z refined points in 64 KiB of LDS, and stays so that what is
+    // accepted and what is refused does not change.
     const size_t es = c->mixed ? sizeof(float) : sizeof(double);
     const int x64 = span(sx.src, nxmr, 64);
     if (x64 > 128) return set_err(c, AFID_E_ARG, "refined x coarser than the base x is not supported");
@@ -1028,7 +1030,7 @@ static int setup(afid_ctx *c) {
         return set_err(c, AFID_E_ARG, "refinement ratio too small for the vyr/vzr tiles");
     const auto block_yz = [&](int cs, int co) { return es * size_t(std::max(x64 * cs * co, cs * 4 * 64) + x64 * cs * 4); };
     const size_t most = std::max(es * size_t(x64 * y16 * z4 + x64 * y16 * 4 + x64 * 16 * 4), std::max(block_yz(ys, yo), block_yz(zs, zo)));
-    // refined -> coarse: the span of 64 x and 8 y coarse points, two planes in 64 KiB
+    // refined -> coarse alike: the span of 64 x and 8 y coarse points, two planes in 64 KiB
     for (int q = 0; q < 2; ++q) {
         const HostTab &h = q == 0 ? hs : hp;
         CoarseTab &t = q == 0 ? c->tab_sal : c->tab_phi;
@@ -1409,11 +1411,7 @@ int afid_update_saturation(afid_ctx *c) {
 
 }  // extern "C"
 
-// One Poisson sweep: forward transforms of the source, per-mode tridiagonals,
-// inverse transforms into dph.  fwd_gate gates the forward y transform, gate
-// the rest; slot_out receives max|div u| of a velocity source.
-// z transform of the spectrum (k_fft_z; the FP32 form may take 16 values per
-// thread and stage, see setup)
+// z transform of the spectrum
 template <typename R, int SIGN>
 static void launch_fft_z(afid_ctx *c, const KP &p, const FftPlan<R> &pz, cpx<R> *spec, Gate gate) {
     const dim3 gr(unsigned((c->nxm + (1 << c->lgz) - 1) >> c->lgz), unsigned(c->nymh));
@@ -1421,6 +1419,9 @@ static void launch_fft_z(afid_ctx *c, const KP &p, const FftPlan<R> &pz, cpx<R> 
         hipLaunchKernelGGL((k_fft_z<R, SIGN, decltype(mt)::value>), gr, dim3(unsigned(c->tz)), c->lds_z, c->stream, p, pz, spec, c->lgz, gate);
     });
 }
+// One Poisson sweep: forward transforms of the source, per-mode tridiagonals,
+// inverse transforms into dph.  fwd_gate gates the forward y transform, gate
+// the rest; slot_out receives max|div u| of a velocity source.
 // us a launch: floor (the arrays once at 5.2 TB/s), the lines in LDS from load
 // to store with 1024 threads before, afid_fft.hpp now (k_div_fft_y / k_fft_z /
 // k_ifft_y):
@@ -1527,8 +1528,9 @@ static int poisson_mixed(afid_ctx *c) {
 }
 
 static constexpr int kTailFields[3] = {AFID_VYR, AFID_VZR, AFID_TEMPR};
-// the reference clears vyr, vzr, tempr before it fills them: index nxr, which
-// no kernel writes, after an upload that may have set it
+// The reference clears vyr, vzr, tempr before it fills them.  Index nxr, which
+// k_xfer_yz leaves alone (or writes 0 to, where a row's last vector holds it),
+// is cleared here after an upload that may have set it.
 static int clean_tails(afid_ctx *c) {
     for (int q = 0; q < 3; ++q) {
         if (!c->tail_dirty[q]) continue;
@@ -1640,8 +1642,7 @@ static int xfer(afid_ctx *c, RT *out, const char *timer) {
         jb.nS = c->nyr; jb.nO = c->nzr; jb.cS = c->ny; jb.cO = c->nz;
         jb.ds = c->ldxr; jb.dq = plane; jb.rs = c->ldxr; jb.ro = p.planer; jb.dl = 1.0 / c->dyr;
     }
-    // vxr has a face more; the other fields leave the unused index nxr alone
-    // (zero: clean_tails)
+    // vxr has a face more; the unused index nxr of the others is zero (clean_tails)
     if (FLD == XF_VX) jb.nx = c->nxr;
     jb.two = (FLD == XF_VZ ? c->two_z : c->two_y) ? 1 : 0;
     rc = xfer_yz<RT, SUM>(c, jb, c->pair_z);

@@ -1,8 +1,9 @@
 // afid_phase.hpp -- phase-field kernels (src/phasefield.F90): the explicit
-// and implicit phi terms on the refined grid, the fused phi column, the
-// masked velocity solves, the coarse -> refined temperature transfer and the
-// seeded sphere.  The refined -> coarse transfers (phic, latent heat) share
-// k_to_coarse with InterpSalMultigrid.
+// and implicit phi terms, the volume penalty and the masked velocity solves of
+// the per-routine calls, and the seeded sphere.  In the fused step the phi
+// column is k_column_refined and the masked solves are part of k_column_base1
+// (four passes: k_column_base); the transfers (tempr, phic, latent heat) are in
+// afid_transfer.hpp.
 #pragma once
 #include <hip/hip_runtime.h>
 #include "afid_params.hpp"
