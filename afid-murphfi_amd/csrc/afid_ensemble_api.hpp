@@ -368,7 +368,7 @@ int afid_ens_init(const afid_config *cfgs, const afid_run_control *ctl, int32_t 
         if (!(ctl[r].dt > 0.0) || !(ctl[r].limit_cfl > 0.0)) return ens_err(e, AFID_E_ARG, who + "DT and CFLMAX must be positive");
         if (g.nxm + 1 > 256) return ens_err(e, AFID_E_ARG, who + "nxm above 255 is not supported by the ensemble");
         afid_ctx *c = nullptr;
-        int rc = ctx_create(&g, e->stream, &c);
+        int rc = ctx_create(&g, e->stream, ROW_TIGHT, &c);
         if (rc) {
             std::string m = who + (c ? c->err : std::string("set-up failed"));
             if (c) afid_gpu_finalize(c);

@@ -61,6 +61,12 @@ struct CoarseTab {
     bool general = false;        // interpolate_xyz_to_coarse (refined grid does not bracket)
 };
 
+// Rows of a field are padded to whole 128 bytes of FP64 values: base columns of
+// 192 x 256^2 476 -> 455 us a launch against 64.  64 where memory does not
+// suffice otherwise, and in ensemble members, which run other kernels: there
+// 128 lengthen the rows of 65 to 129 values by 6 to 11% and a step by 1 to 4%.
+constexpr int ROW_WIDE = 16, ROW_TIGHT = 8;
+
 struct afid_ctx {
     afid_config c{};
     std::string err;
@@ -69,6 +75,7 @@ struct afid_ctx {
     int device = 0;
     // sizes
     int nxm, nx, ny, nz, ldx, ldt, nymh;
+    int row = ROW_WIDE;
     int nxmr = 0, nxr = 0, nyr = 0, nzr = 0, ldxr = 0;
     bool sal = false;
     // physics
@@ -569,14 +576,12 @@ static int setup(afid_ctx *c) {
     if (c->pf && c->sal) return set_err(c, AFID_E_ARG, "phase field together with salinity is not supported");
     if (c->pf && !(g.pf_a != 0.0 && g.pf_s != 0.0)) return set_err(c, AFID_E_ARG, "phase field needs pf_A and pf_S nonzero");
     c->nxm = g.nxm; c->nx = g.nxm + 1; c->ny = g.nym; c->nz = g.nzm;
-    // rows of 128 bytes; of 64 in an ensemble member, whose rows of 65 to 129
-    // values the padding would lengthen by 6 to 11%
-    c->ldx = c->own_stream ? (c->nx + 15) / 16 * 16 : (c->nx + 7) / 8 * 8;
+    c->ldx = (c->nx + c->row - 1) / c->row * c->row;
     c->ldt = (c->nx + 3 + 7) / 8 * 8;
     c->nymh = c->ny / 2 + 1;
     if (c->sal || c->pf) {
         c->nxmr = g.nxmr; c->nxr = g.nxmr + 1; c->nyr = g.nymr; c->nzr = g.nzmr;
-        c->ldxr = (c->nxr + 15) / 16 * 16;
+        c->ldxr = (c->nxr + c->row - 1) / c->row * c->row;
         if (c->nxmr < 2 || c->nyr < 2 || c->nzr < 2) return set_err(c, AFID_E_ARG, "refined grid too small");
     }
     // ReadInputFile.F90:101-122
@@ -1059,8 +1064,9 @@ extern "C" {
 
 static int scratch_ptr_for_device(afid_ctx *c, int dev);
 
-// A context on the caller's stream (shared) or on a stream of its own.
-static int ctx_create(const afid_config *cfg, hipStream_t shared, afid_ctx **out) {
+// A context on the caller's stream (shared) or on a stream of its own, its rows
+// padded to row values.
+static int ctx_create(const afid_config *cfg, hipStream_t shared, int row, afid_ctx **out) {
     if (!cfg || !out) return AFID_E_ARG;
     *out = nullptr;
     afid_ctx *c = new afid_ctx();
@@ -1072,6 +1078,7 @@ static int ctx_create(const afid_config *cfg, hipStream_t shared, afid_ctx **out
         return AFID_E_HIP;
     }
     c->device = dev;
+    c->row = row;
     if (const char *e = std::getenv("AFID_COLUMN_FOUR_PASS")) c->col_four_pass = std::atoi(e) != 0;
     if (const char *e = std::getenv("AFID_COLUMN_WIDE")) c->col_wide = std::atoi(e) != 0;
     if (shared) {
@@ -1100,7 +1107,16 @@ static int ctx_create(const afid_config *cfg, hipStream_t shared, afid_ctx **out
 
 extern "C" {
 
-int afid_gpu_init(const afid_config *cfg, afid_ctx **out) { return ctx_create(cfg, nullptr, out); }
+int afid_gpu_init(const afid_config *cfg, afid_ctx **out) {
+    const char *e = std::getenv("AFID_TIGHT_ROWS");
+    const int row = e && std::atoi(e) != 0 ? ROW_TIGHT : ROW_WIDE;
+    int rc = ctx_create(cfg, nullptr, row, out);
+    if (rc == AFID_E_MEM && row == ROW_WIDE) {                 // again with the rows that take less
+        (void)afid_gpu_finalize(*out);
+        rc = ctx_create(cfg, nullptr, ROW_TIGHT, out);
+    }
+    return rc;
+}
 
 int afid_gpu_finalize(afid_ctx *c) {
     if (!c) return AFID_OK;
