@@ -189,16 +189,21 @@ __global__ void __launch_bounds__(SEG ? 512 : 256) k_xfer_yz(XferJob jb) {
     const ConstTab<RT> wO = const_tab(static_cast<const RT *>(jb.o_w));
     const int l0 = grp * NL;
     const int o0 = sO[l0] - 1;
-    RT w[NL][NU];
+    static_assert(!SUM || NL == 1, "a sum walks single lines");
+    RT w[NL][4];
     long long ro[NU];
 #pragma unroll
     for (int c = 0; c < NU; ++c) ro[c] = (long long)wrapf(o0 + c, jb.cO) * jb.dq;
 #pragma unroll
     for (int l = 0; l < NL; ++l) {
-        const int ll = min(l0 + l, jb.nO - 1), d = sO[ll] - 1 - o0;
+        const int ll = min(l0 + l, jb.nO - 1);
 #pragma unroll
-        for (int c = 0; c < NU; ++c) w[l][c] = c >= d && c < d + 4 ? wO[4 * ll + (c >= d && c < d + 4 ? c - d : 0)] : RT(0);
+        for (int c = 0; c < 4; ++c) w[l][c] = wO[4 * ll + c];
     }
+    // whether the second line of a pair starts one coarse line after the first:
+    // a walk each, so that a line takes its own 4 rows and no fifth with weight
+    // 0, which would carry an infinity to where no stencil reads it
+    const bool shift = NL == 2 && sO[min(l0 + NL - 1, jb.nO - 1)] - 1 > o0;
     // lanes past the row repeat its last vector (the same values to the same place)
     const int x = min((chunk * 64 + lane) * NR, (jb.nx - 1) / NR * NR);
     const RT *D = static_cast<const RT *>(jb.D);
@@ -215,7 +220,7 @@ __global__ void __launch_bounds__(SEG ? 512 : 256) k_xfer_yz(XferJob jb) {
     const int sa = SEG ? int((long long)nt * seg / jb.nseg) : 0, sb = SEG ? int((long long)nt * (seg + 1) / jb.nseg) : nt;
     VS v[NL];
     // walk of the refined steps sa .. sb - 1
-    auto walk = [&](auto store) {
+    auto walk = [&](auto store, auto sh) {
         if (sa >= sb) return;
         int cs = sS[sa] - 1;
         const int end = sS[sb - 1] + 2;
@@ -244,9 +249,12 @@ __global__ void __launch_bounds__(SEG ? 512 : 256) k_xfer_yz(XferJob jb) {
         auto contract = [&](int q) {
 #pragma unroll
             for (int l = 0; l < NL; ++l) {
-                V P = R[q % PD][0] * w[l][0];
-#pragma unroll
-                for (int c = 1; c < NU; ++c) P += R[q % PD][c] * w[l][c];
+                // (fixed roundings, those of a chain over all NU rows)
+                const int d = l ? int(sh) : 0;
+                V P = R[q % PD][1] * w[l][1 - d];
+                P = __builtin_elementwise_fma(R[q % PD][2 * d], V(w[l][d]), P);
+                P = __builtin_elementwise_fma(R[q % PD][d + 2], V(w[l][2]), P);
+                P = __builtin_elementwise_fma(R[q % PD][d + 3], V(w[l][3]), P);
                 W[q][l] = P;
             }
         };
@@ -297,7 +305,7 @@ __global__ void __launch_bounds__(SEG ? 512 : 256) k_xfer_yz(XferJob jb) {
         if (SEG) {
 #pragma unroll
             for (int l = 0; l < NL; ++l) v[l] = VS(0);
-            walk(std::false_type{});
+            walk(std::false_type{}, std::integral_constant<int, 0>{});
 #pragma unroll
             for (int l = 0; l < NL; ++l) tot[(seg * NL + l) * 64 + lane] = v[l];
             __syncthreads();
@@ -317,7 +325,13 @@ __global__ void __launch_bounds__(SEG ? 512 : 256) k_xfer_yz(XferJob jb) {
 #pragma unroll
             for (int l = 0; l < NL; ++l) v[l] += tot[(q * NL + l) * 64 + lane];
     }
-    walk(std::true_type{});
+    if constexpr (NL == 2) {
+        if (shift) {
+            walk(std::true_type{}, std::integral_constant<int, 1>{});
+            return;
+        }
+    }
+    walk(std::true_type{}, std::integral_constant<int, 0>{});
 }
 
 // Refined -> coarse cell centres through the fast coarse-grid loop of
@@ -395,20 +409,22 @@ __global__ void __launch_bounds__(512) k_to_coarse(KP p, CoarseJob jb) {
         for (int b = 0; b < 4; ++b) wy[l][b] = ywc[4 * (J0 + l) + b];
 #pragma unroll
     for (int c = 0; c < NU; ++c) ro[c] = (long long)wrapf(y0 + c, p.nyr) * p.ldxr + x;
-    // taps of coarse k: weights of reference x base .. base + 3, all interior
+    // taps of coarse k: weights of reference x base .. base + 3, 0 on those
+    // outside, where the rows in LDS hold 0 (a clamped base would read points
+    // that the stencil does not, and carry an infinity to k)
     struct Taps { int base; double w[4], gS, gN; };
     auto taps = [&](int k) {
         Taps q{1, {0.0, 0.0, 0.0, 0.0}, 0.0, 0.0};
         if (k >= p.nxm) return q;
         const double *w4 = static_cast<const double *>(jb.x_w) + 4 * k;
         const int s = jb.x_src[k];
-        q.base = max(1, min(s, p.nxmr - 3));
+        q.base = max(-1, min(s, p.nxmr - 1));
 #pragma unroll
         for (int a = 0; a < 4; ++a) {
             int kr = s + a;
             double w = w4[a];
-            if (kr < 0 || kr > p.nxr) w = 0.0;
-            else if (kr == 0) {
+            if (kr < 0 || kr > p.nxr) continue;
+            if (kr == 0) {
                 if (jb.mode == CM_SAL && p.sfixs == 1) { q.gS += w; w = -w; }
             } else if (kr == p.nxr) {
                 if (jb.mode == CM_SAL && p.sfixn == 1) { q.gN += w; w = -w; }
@@ -429,6 +445,12 @@ __global__ void __launch_bounds__(512) k_to_coarse(KP p, CoarseJob jb) {
     const double bw = static_cast<const double *>(jb.y_w)[4 * (J0 + ll) + lb];
     double bv = 0.0;
     auto load_wall = [&](int zs) { bv = 2.0 * bp[(long long)wrapf(zs + la, p.nzr) * p.nyr + by]; };
+
+    // (seen by the others after the first barrier of a coarse plane)
+    for (int q = t; q < 2 * NL * 4; q += T) {
+        const int g = q & 3;                                    // reference x -1, 0, nxmr + 1, nxmr + 2
+        sm[(q >> 2) * LD + NR - 1 + (g < 2 ? g - 1 : p.nxmr + g - 1)] = 0.0;
+    }
 
     int zr = sz[I0] - 1;
     const int end = sz[I1 - 1] + 2;
@@ -472,7 +494,12 @@ __global__ void __launch_bounds__(512) k_to_coarse(KP p, CoarseJob jb) {
 #pragma unroll
         for (int l = 0; l < NL; ++l) {
             const VD v = W[(q + 1) & 3][l] * w0 + W[(q + 2) & 3][l] * w1 + W[(q + 3) & 3][l] * w2 + W[q][l] * w3;
-            if (xw < p.nxmr) *reinterpret_cast<VD *>(b + l * LD + NR + xw) = v;
+            double *at = b + l * LD + NR + xw;
+            if (xw + NR <= p.nxmr) *reinterpret_cast<VD *>(at) = v;
+            else
+#pragma unroll
+                for (int c = 0; c < NR; ++c)
+                    if (xw + c < p.nxmr) at[c] = v[c];
         }
         __syncthreads();
         double g[2][NL] = {};
@@ -492,7 +519,7 @@ __global__ void __launch_bounds__(512) k_to_coarse(KP p, CoarseJob jb) {
                 const double *r = b + l * LD + NR - 1;
                 double v = 0.0;
 #pragma unroll
-                for (int a = 0; a < 4; ++a) v += r[min(q.base + a, p.nxmr)] * q.w[a];
+                for (int a = 0; a < 4; ++a) v += r[q.base + a] * q.w[a];
                 if (wall) v += q.gS * g[0][l] + q.gN * g[1][l];
                 store(bidx(p, kk, J0 + l, ic), v);
             }
