@@ -57,6 +57,7 @@ struct CoarseTab {
     const float *x_wf = nullptr, *y_wf = nullptr, *z_wf = nullptr;
     int nseg = 1;                // ranges of z
     bool two_x = false;          // k_to_coarse_x2: coarse x takes the refined 2 k - 1 .. 2 k + 2
+    bool narrow = false;         // FP32 rows of up to 128 points: 8 bytes a lane
     bool two = false;            // coarse y lines in pairs two refined lines apart (ratio 2)
     bool general = false;        // interpolate_xyz_to_coarse (refined grid does not bracket)
 };
@@ -1047,7 +1048,12 @@ static int setup(afid_ctx *c) {
         for (int j = 0; j + 1 < c->ny; j += 2) t.two = t.two && h.ys[size_t(j + 1)] == h.ys[size_t(j)] + 2;
         t.two_x = q == 1 && nxmr == 2 * nxm;
         for (int k = 0; k < nxm; ++k) t.two_x = t.two_x && h.xs[size_t(k)] == 2 * k;
-        t.nseg = c->mixed ? (t.two ? coarse_ranges<float, 4, 2>(c, t.two_x) : coarse_ranges<float, 4, 1>(c, t.two_x))
+        // 8 bytes a lane where 16 would leave half the lanes of a wavefront idle:
+        // 128 x 192^2 -> 64 x 96^2 in FP32 57 -> 51.5 us a step, 128 x 288^2 88 ->
+        // 79; at 160 points 62 -> 65 and 100 -> 115, at 768 1580 -> 2100
+        t.narrow = c->mixed && !t.two_x && nxmr <= 128;
+        t.nseg = t.narrow ? (t.two ? coarse_ranges<float, 2, 2>(c, false) : coarse_ranges<float, 2, 1>(c, false))
+               : c->mixed ? (t.two ? coarse_ranges<float, 4, 2>(c, t.two_x) : coarse_ranges<float, 4, 1>(c, t.two_x))
                           : (t.two ? coarse_ranges<double, 2, 2>(c, t.two_x) : coarse_ranges<double, 2, 1>(c, t.two_x));
     }
     if (most > 65536)
@@ -1687,7 +1693,9 @@ static int to_coarse(afid_ctx *c, CoarseJob jb, const CoarseTab &t, const char *
     else { jb.x_w = t.x_w; jb.y_w = t.y_w; jb.z_w = t.z_w; }
     tstart(c, timer);
     jb.nseg = t.nseg;
-    if (c->mixed && t.two) launch_to_coarse<float, 4, 2>(c, p, jb, t.two_x);
+    if (t.narrow && t.two) launch_to_coarse<float, 2, 2>(c, p, jb, false);
+    else if (t.narrow) launch_to_coarse<float, 2, 1>(c, p, jb, false);
+    else if (c->mixed && t.two) launch_to_coarse<float, 4, 2>(c, p, jb, t.two_x);
     else if (c->mixed) launch_to_coarse<float, 4, 1>(c, p, jb, t.two_x);
     else if (t.two) launch_to_coarse<double, 2, 2>(c, p, jb, t.two_x);
     else launch_to_coarse<double, 2, 1>(c, p, jb, t.two_x);

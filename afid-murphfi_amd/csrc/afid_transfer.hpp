@@ -371,8 +371,8 @@ struct CoarseJob {
 // lanes form.
 // Weights and sums are FP64 also for FP32 fields, so that only what is stored
 // is rounded: in FP32 the order y, z, x was up to 5% less accurate (rms) than
-// x, y, z at x ratios such as 7/4.  It costs 5 us of 56 a step at 64 x 96^2
-// from 128 x 192^2, 80 of 1580 at 384 x 384^2 from 768^3.
+// x, y, z at x ratios such as 7/4.  It costs 80 us of 1580 a step at 384 x 384^2
+// from 768^3, 1 of 51 at 64 x 96^2 from 128 x 192^2.
 // What bounds it: the read of the refined field once (us a launch, at 5.2 TB/s,
 // now, and as 64 x 8 x 16 tiles staged in LDS with a barrier per refined plane
 // before, which left 72 workgroups at 64^3):
